@@ -628,11 +628,8 @@ __global__ __launch_bounds__(64) void k_fm2d_solve(mct_fm2d_args A)
 
 // Lanes per problem in the grouped heap-loop kernel (64 / GRP_LANES problems per
 // wave) and the waves per SIMD it is compiled for.  LDS bounds the problems in
-// flight (a 512-entry heap is 6.4 KB with 32-bit entries, 5.3 KB with 16-bit
-// ones: 24 or 30 per CU), so registers are not the limit.  Measured on a 64-chain order-1 batch at 201x201 (40,960 problems):
-// 16 lanes 1.84 s, 8 lanes 1.90 s, 4 lanes 2.69 s, one problem per wave 2.31 s;
-// heaps of 384, 640 and 768 entries 2.55, 2.13 and 2.53 s (a smaller heap
-// sends more problems to the lane solver, a larger one runs fewer at once).
+// flight (a 512-entry heap is 6.2 KB with 32-bit entries, 5.1 KB with 16-bit
+// ones: 26 or 31 per CU), so registers are not the limit.
 #ifndef WAVE_EU
 #define WAVE_EU 2
 #endif
@@ -644,53 +641,104 @@ namespace {
 // ---- the heap loop, several problems per wave ----------------------------------------
 // The reference's heap loop (travel, fm2d_ttime.f90:41-238) for the mixed-order
 // problems, with each problem's heap and keys in LDS.  A wave runs 64/GL
-// problems, one group of GL lanes each: every lane of a group holds its
-// problem's state and runs the heap operations (so one vector instruction
-// advances every problem of the wave), the group's first lane alone writes
-// global memory, and lanes 0-3 of a group load and solve the popped node's four
-// neighbours.  The state array keeps each heap node's position, as the
-// reference's does.  A neighbour already in the heap needs that position for
-// updtree: it arrives with the stencil, the downtree's moves are logged in LDS
-// while the loads are in flight and replayed on it, and the neighbours'
-// addtree / updtree moves are applied as they happen, so it is loaded once.  A
-// band that outgrows the LDS heap leaves the problem to the lane solver.
+// problems, one group of GL lanes each.  The loop is a chain of dependent
+// steps, so its time is what one pop takes; the lanes of a group shorten it:
+//   * downtree reads the subtree under the hole (5 levels on 64 lanes, 3 on
+//     16) at once.  Each lane says whether its entry is the smaller sibling and
+//     smaller than the moving one; a lane is on the path exactly when that holds
+//     for itself and all its ancestors in the block, which is one test of the
+//     ballot against its ancestors' bits.  The path's entries then move up
+//     together.  addtree and updtree read all ancestors of a position at once
+//     and move those above the new key down together.  Same comparisons, same
+//     ties and same final arrangement as the reference's level-by-level loops.
+//   * the popped node's four neighbours are solved on 16 lanes, one quadrant of
+//     fouds1 / fouds2 each, and the four quadrants' times reduced to their
+//     minimum.  Their stencils are loaded before the heap moves.
+// The state array keeps each heap node's position, as the reference's does; a
+// neighbour already in the heap needs it for updtree.  It arrives with the
+// stencil and follows the moves of the pop in closed form (a path node moves to
+// half its position, a moved ancestor to twice it or one more).  A band that
+// outgrows the LDS heap leaves the problem to a later pass.
+// What bounds it: a lone wave issues about an instruction every four cycles, and
+// a pop is ~450 of them (280 VALU) plus ~1,200 cycles of waiting on LDS and
+// the stencils.  A pop of a problem alone on its wave takes 1.45 us instead of
+// 2.84 with level-by-level heap moves in one lane (41 x 41 grid, 160 problems:
+// 8.9 ms instead of 16.8); 10,240 problems at 201 x 201, four to a wave, 312 ms
+// instead of 514.
 struct wave_grid {
     int nnx, nnz, ld;
+    unsigned mag;           // ceil(2^32 / ld): a 16-bit offset over ld is its high product
     double gox, goz, dnx, dnz;
     double *t;              // times (global)
     int32_t *s;             // state: -1 far, 0 alive, >0 heap position (global)
-    const double *v;
+    const double *v;        // velocity and slowness, leading dimension vld
+    const double *sl;
     int vld;
     void *hb;               // the group's LDS heap, 1-based (entries of type ET below)
     double *hk;             // its keys, hk[p] = time of hb[p]
-    int2 *mv;               // its log of a downtree's moves (at most 16)
     int cap, ntr, full;
     int vnl, vnr, vnt, vnb;
     int base;               // the group's first lane
     bool lead;              // this lane is it
 };
 
-// heap positions of up to four neighbours, followed through the moves of a pop
-struct w_track {
-    int p[4];
-    __device__ __forceinline__ void move(int from, int to)
-    {
-#pragma unroll
-        for (int k = 0; k < 4; k++) p[k] = p[k] == from ? to : p[k];
-    }
-};
-
-__device__ __forceinline__ double w_shfl_d(double v, int src)
-{
-    return __shfl(v, src, 64);
-}
-
-// Lanes of one wave read what a group's first lane wrote: keep the accesses in order.
+// Lanes of one wave read what others of it wrote: keep the accesses in order.
 __device__ __forceinline__ void w_sync()
 {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// the group's bits of a ballot
+template <int GL>
+__device__ __forceinline__ unsigned long long w_ballot(const wave_grid &G, bool p)
+{
+    const unsigned long long m = __ballot(p);
+    return GL == 64 ? m : ((m >> G.base) & 0xffffull);
+}
+// a value that every lane of the group holds (one wave: a scalar)
+template <int GL>
+__device__ __forceinline__ int w_uni(int v) { return GL == 64 ? __builtin_amdgcn_readfirstlane(v) : v; }
+template <int GL>
+__device__ __forceinline__ double w_uni_d(double v)
+{
+    if (GL != 64) return v;
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_readfirstlane((int)b), hi = __builtin_amdgcn_readfirstlane((int)(b >> 32));
+    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+template <int GL, class T>
+__device__ __forceinline__ T *w_uni_p(T *p)
+{
+    if (GL != 64) return p;
+    const unsigned long long b = (unsigned long long)p;
+    const unsigned lo = (unsigned)__builtin_amdgcn_readfirstlane((int)b);
+    const unsigned hi = (unsigned)__builtin_amdgcn_readfirstlane((int)(b >> 32));
+    return (T *)(((unsigned long long)hi << 32) | lo);
+}
+// lane SRC of the group to all of it (16 lanes: row_newbcast; 64: a lane read)
+template <int GL, int SRC>
+__device__ __forceinline__ int w_bcast(int v)
+{
+    return GL == 64 ? __builtin_amdgcn_readlane(v, SRC)
+                    : __builtin_amdgcn_update_dpp(v, v, 0x150 | SRC, 0xf, 0xf, false);
+}
+template <int GL, int SRC>
+__device__ __forceinline__ double w_bcast_d(double v)
+{
+    const long long b = __double_as_longlong(v);
+    const int lo = w_bcast<GL, SRC>((int)b), hi = w_bcast<GL, SRC>((int)(b >> 32));
+    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+// the value of the lane whose index differs in bit 0 (0xb1) or bit 1 (0x4e)
+template <int CTRL>
+__device__ __forceinline__ double w_quad_d(double v)
+{
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp((int)b, (int)b, CTRL, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp((int)(b >> 32), (int)(b >> 32), CTRL, 0xf, 0xf, false);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
 
 // A heap entry names its node as (ix << 16) | iz (ET = int32_t), or, where the
@@ -708,116 +756,185 @@ __device__ __forceinline__ int w_enc(const wave_grid &G, int iz, int ix)
 template <class ET>
 __device__ __forceinline__ void w_dec(const wave_grid &G, int e, int &iz, int &ix)
 {
-    if (sizeof(ET) == 2) { ix = e / G.ld + 1; iz = e % G.ld + 1; }
-    else { ix = BPX(e); iz = BPZ(e); }
+    if (sizeof(ET) == 2) {
+        const int q = (int)__umulhi((unsigned)e, G.mag);
+        ix = q + 1;
+        iz = e - q * G.ld + 1;
+    } else {
+        ix = BPX(e); iz = BPZ(e);
+    }
 }
 template <class ET>
 __device__ __forceinline__ void w_setpos(const wave_grid &G, int e, int pos)
 {
-    if (!G.lead) return;
     if (sizeof(ET) == 2) G.s[e] = pos;
     else LS(G, BPZ(e), BPX(e)) = pos;
 }
+__device__ __forceinline__ int w_level(int p) { return 31 - __clz(p); }
 
-// addtree (fm2d_ttime.f90:527-564)
-template <class ET>
-__device__ static void w_addtree(wave_grid &G, int iz, int ix, double tv, w_track &trk)
-{
-    if (G.ntr + 1 > G.cap) { G.full = 1; return; }
-    G.ntr = G.ntr + 1;
-    int tpc = G.ntr, tpp = tpc / 2;
-    while (tpp > 0) {
-        const int ep = w_get<ET>(G, tpp);
-        const double kp = G.hk[tpp];
-        if (tv < kp) {
-            w_setpos<ET>(G, ep, tpc);
-            w_put<ET>(G, tpc, ep);
-            G.hk[tpc] = kp;
-            trk.move(tpp, tpc);
-            tpc = tpp;
-            tpp = tpc / 2;
-        } else {
-            tpp = 0;
-        }
+// A lane's place in a downtree block: the node `off` of level `lv` under the
+// hole (its index in the block is 2^lv - 2 + off, so siblings are lanes i, i^1),
+// and the bits of itself and its ancestors in the block.
+template <int GL>
+struct w_block {
+    static constexpr int LV = GL == 64 ? 5 : 3, N = (2 << LV) - 2;
+    static constexpr int MAX = GL == 64 ? 3 : 4;   // blocks on a path: heaps hold at most 4,096 entries, 12 levels
+    int lv, off;
+    unsigned long long anc;
+    __device__ __forceinline__ w_block(int gl)
+    {
+        lv = w_level(gl + 2);
+        off = gl + 2 - (1 << lv);
+        anc = 0;
+        for (int j = gl + 2; j >= 2; j >>= 1) anc |= 1ull << (j - 2);
     }
-    const int e = w_enc<ET>(G, iz, ix);
-    w_setpos<ET>(G, e, tpc);
-    w_put<ET>(G, tpc, e);
-    G.hk[tpc] = tv;
+};
+
+// A value read ahead of the branch that uses it (the compiler would move the LDS
+// read into the branch, behind the tests it could overlap).
+__device__ __forceinline__ void w_pin(int &v) { asm volatile("" : "+v"(v)); }
+
+// The sift-up of addtree (fm2d_ttime.f90:527-564) and updtree (:653-680): entry e
+// with key tv starts at position p.  pos is a heap position to follow (0: none).
+template <class ET, int GL>
+__device__ __forceinline__ void w_siftup(wave_grid &G, int gl, int p, int e, double tv, int &pos)
+{
+    const int m = w_level(p);
+    const bool act = gl < m;                      // lane j - 1 holds the ancestor p >> j
+    const int q = act ? p >> (gl + 1) : 1;
+    const double k = G.hk[q];
+    int ee = w_get<ET>(G, q);
+    w_pin(ee);
+    const unsigned long long stop = w_ballot<GL>(G, act && !(tv < k));
+    const int n = stop ? __builtin_ctzll(stop) : m;
+    // ancestors one level down; the lane after them places the entry itself
+    const int own = gl == n ? 1 : 0;
+    if (gl <= n) {
+        const int to = p >> gl;
+        const int ew = own ? e : ee;
+        w_put<ET>(G, to, ew);
+        G.hk[to] = own ? tv : k;
+        w_setpos<ET>(G, ew, to);
+    }
+    const int sh = w_level(p) - w_level(pos | 1);
+    if (pos > 0 && sh >= 1 && sh <= n && (p >> sh) == pos) pos = p >> (sh - 1);
+    w_sync();
 }
 
-// downtree (fm2d_ttime.f90:575-644); its moves (from, to) go to the group's
-// log, their count to nmv
-template <class ET>
-__device__ static void w_downtree(wave_grid &G, int &nmv)
+// downtree (fm2d_ttime.f90:575-644): the last entry el with key kl moves down
+// from the root (the heap is left with `last` entries).  k, e: the lane's entry of
+// the block under the root.  The moves are made in LDS at once and noted in
+// mv (the lane's entry of block i and the position it moved to, 0 if none);
+// the state array hears of them after the neighbours' loads have landed,
+// because a wait for a load also waits for the stores issued since.  Returns the
+// position the moving entry ends at.
+template <class ET, int GL>
+__device__ __forceinline__ int w_downtree(wave_grid &G, int gl, const w_block<GL> &B, int last, int el, double kl,
+                                          double k, int e, int (&me)[w_block<GL>::MAX], int (&mp)[w_block<GL>::MAX])
 {
-    nmv = 0;
-    if (G.ntr == 1) { G.ntr = G.ntr - 1; return; }
-    const int old = G.ntr;
-    const int el = w_get<ET>(G, old);
-    const double kl = G.hk[old];
-    G.ntr = G.ntr - 1;
-    int tpp = 1, tpc = 2 * tpp;
-    while (tpc < G.ntr) {
-        const int e1 = w_get<ET>(G, tpc), e2 = w_get<ET>(G, tpc + 1);
-        const double k1 = G.hk[tpc], k2 = G.hk[tpc + 1];
-        int ec = e1;
-        double kc = k1;
-        if (k1 > k2) { tpc = tpc + 1; ec = e2; kc = k2; }
-        if (kc < kl) {
-            w_setpos<ET>(G, ec, tpp);
-            w_put<ET>(G, tpp, ec);
-            G.hk[tpp] = kc;
-            G.mv[nmv] = make_int2(tpc, tpp);
-            nmv++;
-            tpp = tpc;
-            tpc = 2 * tpp;
-        } else {
-            tpc = G.ntr + 1;
+    int hole = 1;
+    bool more = last > 0;
+#pragma unroll
+    for (int i = 0; i < w_block<GL>::MAX; i++) {
+        mp[i] = 0;
+        me[i] = 0;
+        if (!more) continue;
+        const int c = (hole << B.lv) + B.off;
+        const bool ok = gl < B.N && c <= last;
+        if (i > 0) {
+            const int q = ok ? c : 1;
+            k = G.hk[q];
+            e = w_get<ET>(G, q);
+            w_pin(e);
+        }
+        if (!ok) k = __builtin_huge_val();
+        const double ks = w_quad_d<0xb1>(k);
+        // the right child when the left one's key is larger, else the left one
+        const bool sel = (gl & 1) ? ks > k : !(k > ks);
+        const unsigned long long P = w_ballot<GL>(G, ok && sel && k < kl);
+        const bool on = gl < B.N && (P & B.anc) == B.anc;
+        const unsigned long long path = w_ballot<GL>(G, on);
+        if (on) {
+            w_put<ET>(G, c >> 1, e);
+            G.hk[c >> 1] = k;
+            me[i] = e;
+            mp[i] = c >> 1;
+        }
+        more = false;
+        if (path) {
+            const int j = 63 - __builtin_clzll(path) + 2;   // the deepest, as 2^level + offset
+            const int l = w_level(j);
+            hole = (hole << l) + j - (1 << l);
+            more = l == B.LV && 2 * hole <= last;
         }
     }
-    if (tpc == G.ntr) {
-        const int ec = w_get<ET>(G, tpc);
-        const double kc = G.hk[tpc];
-        if (kc < kl) {
-            w_setpos<ET>(G, ec, tpp);
-            w_put<ET>(G, tpp, ec);
-            G.hk[tpp] = kc;
-            G.mv[nmv] = make_int2(tpc, tpp);
-            nmv++;
-            tpp = tpc;
-        }
+    if (G.lead && last > 0) {
+        w_put<ET>(G, hole, el);
+        G.hk[hole] = kl;
     }
-    w_setpos<ET>(G, el, tpp);
-    w_put<ET>(G, tpp, el);
-    G.hk[tpp] = kl;
-    G.mv[nmv] = make_int2(old, tpp);
-    nmv++;
+    w_sync();
+    return hole;
 }
 
-// updtree (fm2d_ttime.f90:653-680) from heap position tpc
-template <class ET>
-__device__ static void w_updtree(wave_grid &G, int tpc, int iz, int ix, double tv, w_track &trk)
+// One quadrant of fouds1 (fm2d_ttime.f90:248-332) or fouds2 (:342-518): tj, tk the
+// x and z neighbours' times, tj2, tk2 the ones behind them, a* whether alive.
+// Returns W_NONE when neither neighbour is alive.
+#define W_NONE 1e300
+template <int FOM>
+__device__ __forceinline__ double w_quadrant(bool aj, bool aj2, bool ak, bool ak2, double tj, double tj2, double tk,
+                                             double tk2, double slown, double dnx, double dnz)
 {
-    int tpp = tpc / 2;
-    while (tpp > 0) {
-        const int ep = w_get<ET>(G, tpp);
-        const double kp = G.hk[tpp];
-        if (tv < kp) {
-            w_setpos<ET>(G, ep, tpc);
-            w_put<ET>(G, tpc, ep);
-            G.hk[tpc] = kp;
-            trk.move(tpp, tpc);
-            tpc = tpp;
-            tpp = tpc / 2;
+    const bool J = FOM != 0 && aj && aj2 && tj > tj2, K = FOM != 0 && ak && ak2 && tk > tk2;
+    const double ss = slown * slown, xx = dnx * dnx, zz = dnz * dnz;
+    double a = 1.0, b = 0.0, c, tref, tdiv = 1.0;
+    if (aj && ak) {
+        double uu, vv, em;
+        if (J && K) {
+            uu = 4.0 * xx; vv = 4.0 * zz;
+            tref = 4.0 * tj - tj2;
+            em = tref - 4.0 * tk;
+            em = em + tk2;
+            a = vv + uu;
+            b = 2.0 * em * uu;
+            tdiv = 3.0;
+        } else if (J) {
+            uu = zz; vv = 4.0 * xx;
+            em = 3.0 * tk - 4.0 * tj + tj2;
+            a = vv + 9.0 * uu;
+            b = 6.0 * em * uu;
+            tref = tk;
+        } else if (K) {
+            uu = xx; vv = 4.0 * zz;
+            em = 3.0 * tj - 4.0 * tk + tk2;
+            a = vv + 9.0 * uu;
+            b = 6.0 * em * uu;
+            tref = tj;
         } else {
-            tpp = 0;
+            uu = xx; vv = zz;
+            em = tk - tj;
+            a = uu + vv;
+            b = -(2.0 * uu * em);
+            tref = tj;
         }
+        c = uu * (em * em - vv * ss);
+    } else if (aj) {
+        c = -((J ? 4.0 * xx : xx) * ss);
+        tref = J ? 4.0 * tj - tj2 : tj;
+        tdiv = J ? 3.0 : 1.0;
+    } else if (ak) {
+        // fouds1 squares slown * dnz as one product, fouds2 the squares of each
+        const double sz = slown * dnz;
+        c = FOM == 0 ? -(sz * sz) : -((K ? 4.0 * zz : zz) * ss);
+        tref = K ? 4.0 * tk - tk2 : tk;
+        tdiv = K ? 3.0 : 1.0;
+    } else {
+        return W_NONE;
     }
-    const int e = w_enc<ET>(G, iz, ix);
-    w_setpos<ET>(G, e, tpc);
-    w_put<ET>(G, tpc, e);
-    G.hk[tpc] = tv;
+    double rd1 = b * b - 4.0 * a * c;
+    if (rd1 < 0.0) rd1 = 0.0;
+    const double tdsh = (-b + sqrt(rd1)) / (2.0 * a);
+    const double trav = tref + tdsh;
+    return FOM == 0 ? trav : trav / tdiv;
 }
 
 // travel (fm2d_ttime.f90:41-238) on a group; -1 source outside, -2 heap full.
@@ -826,6 +943,7 @@ template <int FOM, int GL, class ET>
 __device__ static int w_travel(wave_grid &G, double scx, double scz, int urg)
 {
     const int gl = threadIdx.x - G.base;
+    const w_block<GL> B(gl);
     int isx = (int)((scx - G.gox) / G.dnx) + 1;
     int isz = (int)((scz - G.goz) / G.dnz) + 1;
     if (isx < 1 || isx > G.nnx || isz < 1 || isz > G.nnz) return -1;
@@ -833,38 +951,27 @@ __device__ static int w_travel(wave_grid &G, double scx, double scz, int urg)
     if (isz == G.nnz) isz = isz - 1;
     G.ntr = 0;
     G.full = 0;
-    w_track none;
-    none.p[0] = none.p[1] = none.p[2] = none.p[3] = 0;
+    int none = 0;
     if (urg == 2) {
-        // the band in the reference's scan order (x outer, z inner), GL nodes at a time
-        const long n = (long)G.nnx * G.nnz;
-        const unsigned long long gmask = GL == 64 ? ~0ull : ((1ull << GL) - 1ull);
-        for (long q0 = 0; q0 < n; q0 += GL) {
-            const long q = q0 + gl;
-            int i = 1, j = 1;
-            bool band = false;
-            double tq = 0.0;
-            if (q < n) {
-                i = (int)(q / G.nnz) + 1;
-                j = (int)(q % G.nnz) + 1;
-                band = LS(G, j, i) > 0;
-                if (band) tq = LT(G, j, i);
+        // the band in the reference's scan order (x outer, z inner), GL nodes at a
+        // time; it lies in the refined grid's window
+        for (int i = G.vnl; i <= G.vnr; i++)
+            for (int j0 = G.vnt; j0 <= G.vnb; j0 += GL) {
+                const int j = j0 + gl;
+                const bool band = j <= G.vnb && LS(G, j, i) > 0;
+                const double tq = band ? LT(G, j, i) : 0.0;
+                unsigned long long m = w_ballot<GL>(G, band);
+                while (m) {
+                    const int b = __builtin_ctzll(m);
+                    m &= m - 1;
+                    if (G.ntr + 1 > G.cap) return -2;
+                    G.ntr = G.ntr + 1;
+                    w_siftup<ET, GL>(G, gl, G.ntr, w_enc<ET>(G, j0 + b, i), __shfl(tq, G.base + b, 64), none);
+                }
             }
-            unsigned long long m = (__ballot(band) >> G.base) & gmask;
-            while (m) {
-                const int b = __builtin_ctzll(m);
-                m &= m - 1;
-                const int bi = __shfl(i, G.base + b, 64), bj = __shfl(j, G.base + b, 64);
-                w_addtree<ET>(G, bj, bi, w_shfl_d(tq, G.base + b), none);
-                if (G.full) return -2;
-            }
-            w_sync();
-        }
     } else {
-        for (long q = gl; q < (long)G.nnx * G.nnz; q += GL) {
-            const int i = (int)(q / G.nnz) + 1, j = (int)(q % G.nnz) + 1;
-            LS(G, j, i) = -1;
-        }
+        for (int i = 1; i <= G.nnx; i++)
+            for (int j = gl + 1; j <= G.nnz; j += GL) LS(G, j, i) = -1;
         w_sync();
         double vss[2][2];
         for (int i = 1; i <= 2; i++)
@@ -878,16 +985,27 @@ __device__ static int w_travel(wave_grid &G, double scx, double scz, int urg)
                 double ds = sqrt(ex * ex + ez * ez);
                 const double tc = 2.0 * ds / (vss[i - 1][j - 1] + vsrc);
                 if (G.lead) LT(G, isz - 1 + j, isx - 1 + i) = tc;
-                w_addtree<ET>(G, isz - 1 + j, isx - 1 + i, tc, none);
+                G.ntr = G.ntr + 1;
+                w_siftup<ET, GL>(G, gl, G.ntr, w_enc<ET>(G, isz - 1 + j, isx - 1 + i), tc, none);
             }
-        w_sync();
     }
-    // lane k < 4 of the group takes neighbour k (x-1, x+1, z-1, z+1: the reference's order)
-    const int kn = gl & 3;
+    // lanes 4k + 2 sj + sk of the group's first 16 take quadrant (sj, sk) of
+    // neighbour k (x-1, x+1, z-1, z+1: the reference's order)
+    const int kn = (gl >> 2) & 3;
     const int dx = kn == 0 ? -1 : (kn == 1 ? 1 : 0), dz = kn == 2 ? -1 : (kn == 3 ? 1 : 0);
+    const int ddx = (gl & 2) ? 1 : -1, ddz = (gl & 1) ? 1 : -1;
     while (G.ntr > 0) {
+        // one round trip to LDS: the root, the last entry and the block under the root
+        const int old = G.ntr, last = old - 1;
+        const int c0 = (1 << B.lv) + B.off;
+        const int q0 = gl < B.N && c0 <= last ? c0 : 1;
+        const int er = w_get<ET>(G, 1);
+        int el = w_get<ET>(G, old), eb = w_get<ET>(G, q0);
+        const double kl0 = G.hk[old], kb = G.hk[q0];
+        w_pin(el);
+        w_pin(eb);
         int ix, iz;
-        w_dec<ET>(G, w_get<ET>(G, 1), iz, ix);
+        w_dec<ET>(G, w_uni<GL>(er), iz, ix);
         if (urg == 1) {   // stop when the band reaches an inner edge of the refined grid
             int swrg = 0;
             if (ix == 1 && G.vnl != 1) swrg = 1;
@@ -900,53 +1018,71 @@ __device__ static int w_travel(wave_grid &G, double scx, double scz, int urg)
                 break;
             }
         }
-        if (G.lead) LS(G, iz, ix) = 0;
-        w_sync();
-        // the neighbours' states (heap positions) and stencils, read before the heap moves
+        // the neighbours' states (heap positions) and stencils, read before the heap
+        // moves; entries off the grid read the neighbour itself
         const int nx = ix + dx, nz = iz + dz;
-        const bool in = gl < 4 && nx >= 1 && nx <= G.nnx && nz >= 1 && nz <= G.nnz;
+        const bool in = gl < 16 && nx >= 1 && nx <= G.nnx && nz >= 1 && nz <= G.nnz;
         const int cx = in ? nx : ix, cz = in ? nz : iz;
-        const int st = in ? LS(G, cz, cx) : 0;
-        lane_grid L;
-        L.nnx = G.nnx; L.nnz = G.nnz; L.ld = G.ld; L.t = G.t; L.s = G.s; L.v = G.v; L.vld = G.vld; L.fom = FOM;
-        l_sten S;
-        l_load_sten(L, cz, cx, S);
-        // the heap moves while the loads are in flight; the neighbours'
-        // positions then follow the logged moves, each lane its own
-        int nmv = 0;
-        w_downtree<ET>(G, nmv);
-        w_sync();
-        int mypos = st > 0 ? st : 0;
-        for (int q = 0; q < nmv; q++) {
-            const int2 m = G.mv[q];
-            mypos = mypos == m.x ? m.y : mypos;
+        const int x1 = cx + ddx, x2 = cx + 2 * ddx, z1 = cz + ddz, z2 = cz + 2 * ddz;
+        const bool ix1 = x1 >= 1 && x1 <= G.nnx, iz1 = z1 >= 1 && z1 <= G.nnz;
+        const bool ix2 = FOM != 0 && x2 >= 1 && x2 <= G.nnx, iz2 = FOM != 0 && z2 >= 1 && z2 <= G.nnz;
+        const int oP = (ix - 1) * G.ld + (iz - 1);
+        const int o = (cx - 1) * G.ld + (cz - 1);
+        const int ox1 = ix1 ? o + ddx * G.ld : o, ox2 = ix2 ? o + 2 * ddx * G.ld : o;
+        const int oz1 = iz1 ? o + ddz : o, oz2 = iz2 ? o + 2 * ddz : o;
+        const int st0_ = G.s[o];
+        const int sj1 = G.s[ox1], sk1 = G.s[oz1];
+        const int sj2 = FOM ? G.s[ox2] : 1, sk2 = FOM ? G.s[oz2] : 1;
+        const double tj1 = G.t[ox1], tk1 = G.t[oz1];
+        const double tj2 = FOM ? G.t[ox2] : 0.0, tk2 = FOM ? G.t[oz2] : 0.0;
+        const double slown = G.sl[(cx - 1) * G.vld + (cz - 1)];
+        // the heap moves while the loads are in flight; the lane's neighbour's
+        // position then follows: the last entry's is the path's end, one on the
+        // path halves (with a single entry no neighbour is in the heap)
+        G.ntr = last;
+        int me[w_block<GL>::MAX], mp[w_block<GL>::MAX];
+        const int ell = w_uni<GL>(el);
+        const int hole = w_downtree<ET, GL>(G, gl, B, last, ell, w_uni_d<GL>(kl0), kb, eb, me, mp);
+        const int st = in ? st0_ : 0;
+        int pos = st > 0 ? st : 0;
+        const int sh = w_level(hole) - w_level(pos | 1);
+        if (pos == old) pos = hole;
+        else if (pos > 1 && sh >= 0 && (hole >> sh) == pos) pos >>= 1;
+        // (the popped node is alive; its state is stored below)
+        double tv = ix1 && iz1 ? w_quadrant<FOM>(sj1 == 0 || ox1 == oP, ix2 && sj2 == 0, sk1 == 0 || oz1 == oP,
+                                                 iz2 && sk2 == 0, tj1, tj2, tk1, tk2, slown, G.dnx, G.dnz)
+                               : W_NONE;
+        tv = fmin(tv, w_quad_d<0xb1>(tv));
+        tv = fmin(tv, w_quad_d<0x4e>(tv));
+        if (tv >= W_NONE) tv = 0.0;          // no quadrant: the reference's travm stays 0
+        // the states the pop changed, then the neighbours enter the heap one after another
+        if (G.lead) {
+            G.s[oP] = 0;
+            if (last > 0) w_setpos<ET>(G, ell, hole);
         }
-        const int st0 = __shfl(st, G.base + 0, 64), st1 = __shfl(st, G.base + 1, 64);
-        const int st2 = __shfl(st, G.base + 2, 64), st3 = __shfl(st, G.base + 3, 64);
-        w_track trk;
-        trk.p[0] = __shfl(mypos, G.base + 0, 64); trk.p[1] = __shfl(mypos, G.base + 1, 64);
-        trk.p[2] = __shfl(mypos, G.base + 2, 64); trk.p[3] = __shfl(mypos, G.base + 3, 64);
-        double tv = 0.0;
-        if (st != 0) tv = FOM == 0 ? l_fouds1s(S, G.dnx, G.dnz) : l_fouds2s(S, G.dnx, G.dnz);
-        const double tv0 = w_shfl_d(tv, G.base + 0), tv1 = w_shfl_d(tv, G.base + 1);
-        const double tv2 = w_shfl_d(tv, G.base + 2), tv3 = w_shfl_d(tv, G.base + 3);
 #pragma unroll
-        for (int k = 0; k < 4; k++) {
-            const int stk = k == 0 ? st0 : (k == 1 ? st1 : (k == 2 ? st2 : st3));
-            if (stk == 0) continue;
-            const double tvk = k == 0 ? tv0 : (k == 1 ? tv1 : (k == 2 ? tv2 : tv3));
+        for (int i = 0; i < w_block<GL>::MAX; i++)
+            if (mp[i]) w_setpos<ET>(G, me[i], mp[i]);
+        auto enter = [&](int stk, int pk, double tvk, int k) {
             const int xk = ix + (k == 0 ? -1 : (k == 1 ? 1 : 0)), zk = iz + (k == 2 ? -1 : (k == 3 ? 1 : 0));
             if (G.lead) LT(G, zk, xk) = tvk;
+            int p = pk;
             if (stk == -1) {
-                w_addtree<ET>(G, zk, xk, tvk, trk);
-            } else {
-                const int pos = trk.p[k];
-                trk.p[k] = 0;
-                w_updtree<ET>(G, pos, zk, xk, tvk, trk);
+                if (G.ntr + 1 > G.cap) { G.full = 1; return; }
+                G.ntr = G.ntr + 1;
+                p = G.ntr;
             }
-        }
+            if (kn == k) pos = 0;
+            w_siftup<ET, GL>(G, gl, p, w_enc<ET>(G, zk, xk), tvk, pos);
+        };
+        const int st0 = w_bcast<GL, 0>(st), st1 = w_bcast<GL, 4>(st), st2 = w_bcast<GL, 8>(st), st3 = w_bcast<GL, 12>(st);
+        const double tv0 = w_bcast_d<GL, 0>(tv), tv1 = w_bcast_d<GL, 4>(tv);
+        const double tv2 = w_bcast_d<GL, 8>(tv), tv3 = w_bcast_d<GL, 12>(tv);
+        if (st0 != 0) enter(st0, w_bcast<GL, 0>(pos), tv0, 0);
+        if (st1 != 0) enter(st1, w_bcast<GL, 4>(pos), tv1, 1);
+        if (st2 != 0) enter(st2, w_bcast<GL, 8>(pos), tv2, 2);
+        if (st3 != 0) enter(st3, w_bcast<GL, 12>(pos), tv3, 3);
         if (G.full) return -2;
-        w_sync();
     }
     return 0;
 }
@@ -989,6 +1125,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WAVE_EU))) v
     if (!live) return;
     const long wsz = (long)A.ld * A.nc;
     const double *velnc = A.veln + cp * (long)A.nnx * A.nnz;
+    const double *slnc = A.sln + cp * (long)A.nnx * A.nnz;
     const double *velv = A.velv + cp * (long)(A.nvz + 2) * (A.nvx + 2);
     const int ldv = A.nvz + 2;
     const double dnx = A.dvx / A.gdx, dnz = A.dvz / A.gdz;
@@ -998,15 +1135,17 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WAVE_EU))) v
     G.s = A.nsts + slot * wsz;
     {
         const int hbw = (int)(((long)(heap_cap + 1) * sizeof(ET) + 7) / 8);   // doubles of entries
-        const int per = heap_cap + 1 + hbw + 16;                              // doubles per group
+        const int per = heap_cap + 1 + hbw;                                   // doubles per group
         double *gb = w_lds + (long)g * per;
         G.hk = gb;
         G.hb = (void *)(gb + heap_cap + 1);
-        G.mv = (int2 *)(gb + heap_cap + 1 + hbw);
     }
+    G.mag = (unsigned)(((1ull << 32) + (unsigned)A.ld - 1) / (unsigned)A.ld);
     G.cap = heap_cap;
-    G.base = g * GL;
+    G.base = GL == 64 ? 0 : g * GL;
     G.lead = gl == 0;
+    G.t = w_uni_p<GL>(G.t);
+    G.s = w_uni_p<GL>(G.s);
     const double x = A.scx[s], z = A.scz[s];
     int isx = (int)((x - A.gox) / dnx) + 1, isz = (int)((z - A.goz) / dnz) + 1;
     if (isx < 1 || isx > A.nnx || isz < 1 || isz > A.nnz) return;   // the lane solver reports it
@@ -1027,7 +1166,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WAVE_EU))) v
         G.gox = A.gox + dnx * (vnl - 1);
         G.goz = A.goz + dnz * (vnt - 1);
         G.vnl = vnl; G.vnr = vnr; G.vnt = vnt; G.vnb = vnb;
-        G.v = vr; G.vld = A.ld;
+        double *sr = A.ttr + slot * wsz;      // refined slowness, until the remap below
+        G.v = vr; G.sl = w_uni_p<GL>((const double *)sr); G.vld = A.ld;
         const int nrxr = A.gdx * A.sgdl, nrzr = A.gdz * A.sgdl;
         const int origx = (vnl - 1) * A.sgdl + 1, origz = (vnt - 1) * A.sgdl + 1;
         const int rn = G.nnx * G.nnz;
@@ -1050,7 +1190,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WAVE_EU))) v
                     sum[i1 - 1] = sum[i1 - 1] + ui[j1 - 1] * velv[(jj - 2 + j1) * ldv + (ii - 2 + i1)];
                 sum[i1 - 1] = vi[i1 - 1] * sum[i1 - 1];
             }
-            vr[(long)(idm2 - 1) * A.ld + (idm1 - 1)] = sum[0] + sum[1] + sum[2] + sum[3];
+            const double vq = sum[0] + sum[1] + sum[2] + sum[3];
+            vr[(long)(idm2 - 1) * A.ld + (idm1 - 1)] = vq;
+            sr[(long)(idm2 - 1) * A.ld + (idm1 - 1)] = 1.0 / vq;
         }
         w_sync();
         if (w_travel<FOM, GL, ET>(G, x, z, 1)) return;
@@ -1064,8 +1206,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WAVE_EU))) v
             nr[o] = G.s[o];
         }
         w_sync();
-        for (long q = gl; q < (long)A.nnx * A.nnz; q += GL)
-            G.s[(q / A.nnz) * A.ld + (q % A.nnz)] = -1;
+        for (int k = 0; k < A.nnx; k++)
+            for (int l = gl; l < A.nnz; l += GL) G.s[k * A.ld + l] = -1;
         w_sync();
         const int wkz = (rnz - 1) / A.sgdl + 1, wkx = (rnx - 1) / A.sgdl + 1;
         for (int q = gl; q < wkz * wkx; q += GL) {
@@ -1077,10 +1219,12 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WAVE_EU))) v
         }
         w_sync();
         G.nnx = A.nnx; G.nnz = A.nnz; G.dnx = dnx; G.dnz = dnz; G.gox = A.gox; G.goz = A.goz;
-        G.v = velnc; G.vld = A.nnz;
-        // complete the narrow band: alive nodes next to far nodes become close
-        for (long q = gl; q < (long)A.nnx * A.nnz; q += GL) {
-            const int k = (int)(q / A.nnz) + 1, l = (int)(q % A.nnz) + 1;
+        G.v = velnc; G.sl = w_uni_p<GL>(slnc); G.vld = A.nnz;
+        // complete the narrow band: alive nodes next to far nodes become close (only
+        // the window holds alive nodes)
+        const int wnz = vnb - vnt + 1;
+        for (int q = gl; q < (vnr - vnl + 1) * wnz; q += GL) {
+            const int k = vnl + q / wnz, l = vnt + q % wnz;
             if (LS(G, l, k) != 0) continue;
             if ((l - 1 >= 1 && LS(G, l - 1, k) == -1) || (l + 1 <= A.nnz && LS(G, l + 1, k) == -1) ||
                 (k - 1 >= 1 && LS(G, l, k - 1) == -1) || (k + 1 <= A.nnx && LS(G, l, k + 1) == -1))
@@ -1090,7 +1234,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WAVE_EU))) v
         if (w_travel<FOM, GL, ET>(G, x, z, 2)) return;
     } else {
         G.nnx = A.nnx; G.nnz = A.nnz; G.dnx = dnx; G.dnz = dnz; G.gox = A.gox; G.goz = A.goz;
-        G.v = velnc; G.vld = A.nnz;
+        G.v = velnc; G.sl = w_uni_p<GL>(slnc); G.vld = A.nnz;
         if (w_travel<FOM, GL, ET>(G, x, z, 0)) return;
     }
     w_sync();
@@ -1167,12 +1311,11 @@ static int w_launch(const mct_fm2d_args &b, int cap, int32_t *pflag, hipStream_t
             v = 64 * 1024;
         lds_max = v;
     }
-    // per problem: keys, heap entries, the downtree log (16 moves: at most 13 levels);
-    // a heap too large for the workgroup's LDS is cut to what fits (bands that
+    // per problem: keys and heap entries; a heap too large for the workgroup's LDS is cut to what fits (bands that
     // outgrow it go to the lane solver like any other overflow)
     auto bytes = [&](int c) -> size_t {
         const long hbw = ((long)(c + 1) * (long)sizeof(ET) + 7) / 8;
-        return (size_t)NG * 8 * (size_t)(c + 1 + hbw + 16);
+        return (size_t)NG * 8 * (size_t)(c + 1 + hbw);
     };
     while (cap > 64 && bytes(cap) > (size_t)lds_max) cap -= 64;
     const size_t lds = bytes(cap);
@@ -1190,22 +1333,24 @@ static int w_launch(const mct_fm2d_args &b, int cap, int32_t *pflag, hipStream_t
 int mct_launch_fm2d_wave(const mct_fm2d_args &b, int32_t *pflag, hipStream_t s)
 {
     if (!pflag || b.nrun < 1) return MCT_ERR_ARG;
-    // bands that outgrow the heap go to the lane solver, which keeps all of them
-    // in flight at once (a second pass with 2,048-entry heaps, four problems per
-    // CU, was slower: 9.5 s instead of 2.6 s when a 384-entry first pass left a
-    // large share of the 40,960 problems over)
     // 16-bit heap entries (a node's offset in the slot's arrays) where they fit.
-    // A launch with few problems gives each a wave of its own, which shortens its
-    // chain (a plain 201x201 order-1 call, 640 problems: 194.6 ms against 242.8
-    // with four problems per wave); many problems share waves, which is the more
-    // work per instruction (40,960 problems: 1.63 s against 2.31 s)
     const bool e16 = (long)b.ld * b.nc <= 65536;
     const int cap = w_heap_cap();
     const char *es = getenv("MCT_WAVE_SPLIT");      // the largest launch with a wave per problem
     const long split = es ? atol(es) : 4096;
+    int rc;
     if (b.nrun <= split)
-        return e16 ? w_launch<64, uint16_t>(b, cap, pflag, s) : w_launch<64, int32_t>(b, cap, pflag, s);
-    return e16 ? w_launch<GRP_LANES, uint16_t>(b, cap, pflag, s) : w_launch<GRP_LANES, int32_t>(b, cap, pflag, s);
+        rc = e16 ? w_launch<64, uint16_t>(b, cap, pflag, s) : w_launch<64, int32_t>(b, cap, pflag, s);
+    else
+        rc = e16 ? w_launch<GRP_LANES, uint16_t>(b, cap, pflag, s) : w_launch<GRP_LANES, int32_t>(b, cap, pflag, s);
+    // bands that outgrew the heap run again, a wave each, with a larger one (a
+    // work-group whose problem is done leaves at once); what outgrows that too
+    // goes to the lane solver.  A few wide bands among 10,240 problems at
+    // 201 x 201 took the lane solver 449 ms, one lane's chain of cache misses;
+    // here they take about 100.
+    if (!rc && !getenv("MCT_WAVE_HEAP"))
+        rc = e16 ? w_launch<64, uint16_t>(b, 2048, pflag, s) : w_launch<64, int32_t>(b, 2048, pflag, s);
+    return rc;
 }
 
 int mct_launch_fm2d_gridder(const mct_fm2d_args &a, hipStream_t s)

@@ -306,3 +306,26 @@ def test_order_one_heap_larger_than_lds_is_cut_to_fit(split, monkeypatch):
     dflt = mct.modrays(velv, 0, 0, h, h, sx, sz, rx, rz, method=0, **kw)
     np.testing.assert_array_equal(got, dflt)
     agree(got, want, 0)
+
+
+@pytest.mark.parametrize("split", ["0", "1000000"])
+def test_order_one_bands_wider_than_the_first_heap(split, monkeypatch):
+    """A 325 x 289 grid (dicing 4) whose narrow band outgrows the first pass's 512
+    heap entries: the second pass (2,048 entries, a wave per problem) solves the
+    problem, and the times are the oracle's and the lane solver's bit for bit."""
+    rng = np.random.default_rng(512)
+    nvx, nvz, h = 82, 73, 0.5
+    ns, nr = 5, 9
+    velv = rng.uniform(2.2, 4.4, (nvx + 2, nvz + 2))
+    L, W = (nvx - 1) * h, (nvz - 1) * h
+    sx, sz = rng.uniform(h, L - h, ns), rng.uniform(h, W - h, ns)
+    rx, rz = rng.uniform(0, L, nr), rng.uniform(0, W, nr)
+    kw = dict(gdx=4, gdz=4, asgr=1, sgdl=4, sgs=8, fom=1)
+    say("order 1, wide band, split", split)
+    want = po.fm2d(velv, 0, 0, h, h, sx, sz, rx, rz, **kw)
+    monkeypatch.setenv("MCT_WAVE_SPLIT", split)
+    got = mct.modrays(velv, 0, 0, h, h, sx, sz, rx, rz, method=0, **kw)
+    monkeypatch.setenv("MCT_FM2D_WAVE", "0")
+    lanes = mct.modrays(velv, 0, 0, h, h, sx, sz, rx, rz, method=0, **kw)
+    np.testing.assert_array_equal(got, lanes)
+    agree(got, want, 0)
