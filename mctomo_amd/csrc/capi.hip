@@ -228,11 +228,10 @@ static int body_pipeline(mct_ctx *C, int nchain, const double *d_points, const d
         E.flags[0] = P<uint8_t>(C->eik.flags0); E.flags[1] = P<uint8_t>(C->eik.flags1);
     E.any = P<uint32_t>(C->eik.counts);
     E.key[0] = P<uint32_t>(C->eik.key0); E.key[1] = P<uint32_t>(C->eik.key1);
-    E.band_dt = P<float>(C->eik.band);
+    E.vmax = P<float>(C->eik.band);
+    E.band_h = C->band_tiles * 4.f * (float)fmin(fmin(G.dx, G.dy), lz);
     E.band_rounds = mct_band_rounds(G, C->band_tiles);
-    if ((rc = mct_launch_band_dt(E.vel, E.vel64, (long)G.ntiles * MCT_TILE_N, nchain * C->nwave,
-                                 (float)fmin(fmin(G.dx, G.dy), lz), C->band_tiles,
-                                 P<float>(C->eik.band), s)))
+    if ((rc = mct_launch_vmax(E.vel, E.vel64, (long)G.ntiles * MCT_TILE_N, nchain * C->nwave, P<float>(C->eik.band), s)))
         return rc;
     const double *src_pts; int sstride; long schain;
     const double *pick_pts; int pstride; int pchain;

@@ -148,11 +148,10 @@ extern "C" int fastMarching3D(int nx, int ny, int nz, double dx, double dy, doub
         E.flags[0] = (uint8_t *)W.fl0.p; E.flags[1] = (uint8_t *)W.fl1.p;
     E.any = (uint32_t *)W.counts.p;
     E.key[0] = (uint32_t *)W.k0.p; E.key[1] = (uint32_t *)W.k1.p;
-    E.band_dt = (const float *)W.band.p;
+    E.vmax = (const float *)W.band.p;
+    E.band_h = mct_default_band_tiles() * 4.f * (float)fmin(fmin(dx, dy), dz);
     E.band_rounds = mct_band_rounds(G, mct_default_band_tiles());
-    if ((rc = mct_launch_band_dt(E.vel, E.vel64, tn, 1, (float)fmin(fmin(dx, dy), dz), mct_default_band_tiles(),
-                                 (float *)W.band.p, s)))
-        return rc;
+    if ((rc = mct_launch_vmax(E.vel, E.vel64, tn, 1, (float *)W.band.p, s))) return rc;
     if ((rc = mct_launch_eik_init(E, (const double *)W.src.p, 3, 0, xmin, ymin, zmin, dx, dy, dz, s))) return rc;
     if (E.order == 1 && f64 && mct_default_heap_order1()) {
         // the reference's heap loop replayed (its mixed-order times depend on the pop order)

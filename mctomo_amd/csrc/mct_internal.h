@@ -89,7 +89,8 @@ struct mct_eik_problem_set {
     uint8_t *flags[2];             // active-tile flags of the current / next round
     uint32_t *key[2];              // per tile: smallest activating time (float bits)
     uint32_t *any;                 // [3] rotating "some tile is active" flags
-    const float *band_dt;          // (nchain*nwave) band time step per round
+    const float *vmax;             // (nchain*nwave) largest velocity
+    float band_h;                  // distance the band advances per round: band_h / vmax is its time step
     int band_rounds;               // rounds with the band schedule, then plain FIM
     int32_t *status;               // (nprob) or NULL
 };
@@ -103,12 +104,11 @@ int mct_launch_eik_init(const mct_eik_problem_set &P, const double *src_pts, int
                         double lx, double ly, double lz, hipStream_t s);
 int mct_launch_eik_round(const mct_eik_problem_set &P, int round, double hx, double hy, double hz,
                          int grid_blocks, hipStream_t s);
-// band_dt[cw] = tiles_per_round * 4 * min(h) / max velocity of (chain, wave) cw
-// (from vel64 when given, else vel)
-int mct_launch_band_dt(const float *vel, const double *vel64, long tsz, int ncw, float hmin, float tiles_per_round,
-                       float *band_dt, hipStream_t s);
+// vmax[cw] = the largest velocity of (chain, wave) cw (from vel64 when given, else
+// vel)
+int mct_launch_vmax(const float *vel, const double *vel64, long tsz, int ncw, float *vmax, hipStream_t s);
 
-// Band schedule: the first band rounds advance tau by band_dt per round; then
+// Band schedule: the first band rounds advance tau by band_h / vmax per round; then
 // tau is lifted (plain fast-iterative rounds) until no tile is active.
 static inline int mct_band_rounds(const mct_geom &G, float band_tiles)
 {
