@@ -172,7 +172,7 @@ struct mct_ctx {
     mct_geom G;
     mct_body_setup S;
     int nwave, nsrc_eff, npick, reciprocal;
-    float band_tiles;                // eikonal schedule: tiles the band advances per round
+    float band_tiles;                // eikonal schedule: tiles the band advances per round (0: by size)
     int t64;                         // eikonal arrival times stored as double
     int f64;                         // eikonal velocities and local solves in FP64 (with t64)
     int heap_order1;                 // order 1: replay the reference's heap loop (needs f64)
@@ -229,8 +229,9 @@ static int body_pipeline(mct_ctx *C, int nchain, const double *d_points, const d
     E.any = P<uint32_t>(C->eik.counts);
     E.key[0] = P<uint32_t>(C->eik.key0); E.key[1] = P<uint32_t>(C->eik.key1);
     E.vmax = P<float>(C->eik.band);
-    E.band_h = C->band_tiles * 4.f * (float)fmin(fmin(G.dx, G.dy), lz);
-    E.band_rounds = mct_band_rounds(G, C->band_tiles);
+    const float band = mct_band_tiles(C->band_tiles, E.order, (long)E.nprob * G.ntiles);
+    E.band_h = band * 4.f * (float)fmin(fmin(G.dx, G.dy), lz);
+    E.band_rounds = mct_band_rounds(G, band);
     if ((rc = mct_launch_vmax(E.vel, E.vel64, (long)G.ntiles * MCT_TILE_N, nchain * C->nwave, P<float>(C->eik.band), s)))
         return rc;
     const double *src_pts; int sstride; long schain;
@@ -351,7 +352,7 @@ int mct_body_create(const mct_grid *grid, const mct_body_setup *setup, mct_ctx *
     C->reciprocal = setup->dynamic != 0 || setup->nsrc > setup->nrev;
     C->nsrc_eff = C->reciprocal ? setup->nrev : setup->nsrc;
     C->npick = C->reciprocal ? setup->nsrc : setup->nrev;
-    C->band_tiles = mct_default_band_tiles();
+    C->band_tiles = 0.f;
     C->f64 = mct_default_f64();
     C->t64 = C->f64 ? 1 : mct_default_t64();
     C->heap_order1 = mct_default_heap_order1();

@@ -84,10 +84,10 @@ int eik_rounds(const mct_eik_problem_set &E, uint32_t *h_count, double hx, doubl
 {
     const mct_geom &G = E.G;
     const int max_rounds = E.band_rounds + 8 * (G.ntx + G.nty + G.ntz) + 256;
-    int dev = 0, cus = 256;
-    hipDeviceProp_t prop;
-    if (hipGetDevice(&dev) == hipSuccess && hipGetDeviceProperties(&prop, dev) == hipSuccess)
-        cus = prop.multiProcessorCount;
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+        cus = 256;
     int r = 0;
     for (;;) {
         for (int k = 0; k < 8; k++, r++) {
@@ -149,8 +149,9 @@ extern "C" int fastMarching3D(int nx, int ny, int nz, double dx, double dy, doub
     E.any = (uint32_t *)W.counts.p;
     E.key[0] = (uint32_t *)W.k0.p; E.key[1] = (uint32_t *)W.k1.p;
     E.vmax = (const float *)W.band.p;
-    E.band_h = mct_default_band_tiles() * 4.f * (float)fmin(fmin(dx, dy), dz);
-    E.band_rounds = mct_band_rounds(G, mct_default_band_tiles());
+    const float band = mct_band_tiles(0.f, E.order, G.ntiles);
+    E.band_h = band * 4.f * (float)fmin(fmin(dx, dy), dz);
+    E.band_rounds = mct_band_rounds(G, band);
     if ((rc = mct_launch_vmax(E.vel, E.vel64, tn, 1, (float *)W.band.p, s))) return rc;
     if ((rc = mct_launch_eik_init(E, (const double *)W.src.p, 3, 0, xmin, ymin, zmin, dx, dy, dz, s))) return rc;
     if (E.order == 1 && f64 && mct_default_heap_order1()) {

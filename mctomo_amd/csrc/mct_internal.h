@@ -115,8 +115,9 @@ static inline int mct_band_rounds(const mct_geom &G, float band_tiles)
     float bt = band_tiles > 0.05f ? band_tiles : 0.05f;
     return (int)(6.0f * (G.ntx + G.nty + G.ntz) / bt) + 8;
 }
-// Tiles per round of the band schedule (environment MCT_BAND_TILES, else 0.5).
-float mct_default_band_tiles();
+// Tiles per round of the band schedule: `set` if positive, else the environment's
+// MCT_BAND_TILES, else by the number of tiles of all problems.
+float mct_band_tiles(float set, int order, long tiles);
 // Arrival-time storage: double unless the environment sets MCT_EIK_F32=1.
 int mct_default_t64();
 // FP64 velocities and local solves: on unless the environment sets MCT_EIK_F64=0.

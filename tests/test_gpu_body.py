@@ -104,6 +104,27 @@ def test_fast_marching_3d_vs_oracle(order, rtol):
     say("fm3d order", order, "worst receiver rel err", worst)
 
 
+@pytest.mark.parametrize("dims,h", [((2, 2, 2), (0.3, 0.3, 0.3)), ((4, 5, 9), (0.2, 0.2, 0.2)),
+                                    ((13, 8, 21), (0.25, 0.25, 0.25)), ((13, 8, 21), (0.25, 0.4, 0.15)),
+                                    ((4, 17, 3), (0.1, 0.1, 0.05)), ((64, 3, 5), (0.2, 0.1, 0.2))])
+def test_first_order_field_on_ragged_tiles(dims, h):
+    """The first-order update on one spacing and on different ones, over grids that
+    end inside a 4^3 tile and at its edge, with the source inside a cell, on a
+    node and at both corners.  The reference keeps a time unless it falls by
+    2.2e-11 (COMP_MARGIN), the parallel relaxation takes every decrease: 1e-9."""
+    rng = np.random.default_rng(sum(dims))
+    h = np.array(h)
+    ext = h * (np.array(dims) - 1)
+    vel = rng.uniform(3.0, 7.0, dims)
+    rev = rng.uniform(0, 1, (5, 3)) * ext
+    for src in (rng.uniform(0, 1, 3) * ext, h * 1, ext.copy(), np.zeros(3)):
+        say("ragged", dims, h, src)
+        tt, f = mct.fast_marching_3d(vel, *h, 0, 0, 0, src, rev, 0, field=True)
+        to, fo = po.fast_marching_3d(vel, *h, 0, 0, 0, src, rev, 0, field=True)
+        np.testing.assert_allclose(f, fo, rtol=1e-9, atol=1e-10)
+        np.testing.assert_allclose(tt, to, rtol=1e-9, atol=1e-10)
+
+
 def test_fast_marching_3d_offset_grid_and_anisotropic_spacing():
     say("fm3d offset grid")
     rng = np.random.default_rng(3)
