@@ -44,7 +44,7 @@ template <class T> T *P(dbuf &b) { return (T *)b.p; }
 // Eikonal workspace for a set of problems on one geometry.
 struct eik_ws {
     dbuf T, flags0, flags1, key0, key1, counts, band;
-    dbuf heap, err;                  // heap replay (order 1): per-problem heaps, error bits
+    dbuf heap, err, lin;             // heap replay (order 1): per-problem heaps, error bits, padded grids
     uint32_t *h_count = nullptr;     // pinned
     int alloc(const mct_geom &G, long nprob)
     {
@@ -64,7 +64,7 @@ struct eik_ws {
     void release()
     {
         dfree(T); dfree(flags0); dfree(flags1); dfree(key0); dfree(key1); dfree(counts); dfree(band);
-        dfree(heap); dfree(err);
+        dfree(heap); dfree(err); dfree(lin);
         if (h_count) (void)hipHostFree(h_count);
         h_count = nullptr;
     }
@@ -160,6 +160,12 @@ int sfmm_solve(const mct_eik_problem_set &E, eik_ws &ws, const double *src_pts, 
     if ((rc = dalloc(ws.heap, sizeof(uint32_t) * (size_t)a.hcap * (size_t)E.nprob))) return rc;
     if ((rc = dalloc(ws.err, 4 * sizeof(uint32_t)))) return rc;
     a.heap = (uint32_t *)ws.heap.p; a.err = (uint32_t *)ws.err.p;
+    // (without room for it the replay runs with its heaps in global memory)
+    const size_t lin = mct_sfmm_lin_bytes(E.G, E.nprob, E.nprob / E.nsrc_eff);
+    if (lin) {
+        if (dalloc(ws.lin, lin) == MCT_OK) a.lin = ws.lin.p;
+        else (void)hipGetLastError();
+    }
     if ((rc = mct_launch_sfmm(a, s))) return rc;
     MCT_CHECK(hipMemcpyAsync(ws.h_count, a.err, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
     MCT_CHECK(hipStreamSynchronize(s));

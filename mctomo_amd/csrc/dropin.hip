@@ -30,7 +30,7 @@ struct dropin_ws {
     std::mutex mu;
     hipStream_t s = nullptr;
     ws_buf vel_d, vel_t, T, fl0, fl1, k0, k1, band, counts, src, rev, tt, field, pts, prm,
-        sid, vp, vs, rho, pm, fcount, fnodes, kdn, kdi, kdr, heap, err;
+        sid, vp, vs, rho, pm, fcount, fnodes, kdn, kdi, kdr, heap, err, lin;
     uint32_t *h_count = nullptr;
     int init()
     {
@@ -166,6 +166,11 @@ extern "C" int fastMarching3D(int nx, int ny, int nz, double dx, double dy, doub
         if ((rc = W.heap.need(sizeof(uint32_t) * (size_t)a.hcap)) || (rc = W.err.need(4 * sizeof(uint32_t))))
             return rc;
         a.heap = (uint32_t *)W.heap.p; a.err = (uint32_t *)W.err.p;
+        const size_t lin = mct_sfmm_lin_bytes(G, 1, 1);
+        if (lin) {
+            if (W.lin.need(lin) == MCT_OK) a.lin = W.lin.p;
+            else (void)hipGetLastError();
+        }
         if ((rc = mct_launch_sfmm(a, s))) return rc;
         MCT_CHECK(hipMemcpyAsync(W.h_count, a.err, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
         MCT_CHECK(hipStreamSynchronize(s));

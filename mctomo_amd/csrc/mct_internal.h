@@ -142,7 +142,11 @@ struct mct_sfmm_args {
     long hcap;
     uint32_t *err;
     uint32_t *pops;
+    void *lin;                     // mct_sfmm_lin_bytes of scratch for the replay in LDS, or NULL
+    const uint32_t *done;          // set by the launcher: problems already solved there
 };
+// Scratch of the replay with its heap in LDS (padded grids), 0 where it is not used.
+size_t mct_sfmm_lin_bytes(const mct_geom &G, long nprob, long ncw);
 long mct_sfmm_heap_cap(const mct_geom &G);
 int mct_launch_sfmm(const mct_sfmm_args &a, hipStream_t s);
 int mct_sfmm_status(uint32_t err_bits);

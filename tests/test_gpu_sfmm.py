@@ -141,3 +141,20 @@ def test_order1_batch_equals_single_calls():
     assert (dst.numpy() == 0).all()
     np.testing.assert_array_equal(dout.numpy(), np.array(single))
     like.close()
+
+
+@pytest.mark.parametrize("shape,h,where", [((3, 4, 5), (0.2, 0.2, 0.2), "LDS"), ((24, 2, 9), (0.1, 0.3, 0.2), "LDS"),
+                                           ((70, 66, 64), (0.2, 0.2, 0.1), "LDS or handed over"),
+                                           ((90, 88, 86), (0.2, 0.2, 0.2), "global")])
+def test_heap_replay_by_size(shape, h, where):
+    """The replay keeps its heap and keys in LDS where the band fits (small grids to
+    about 70^3), hands a band that outgrows them to the replay in global memory, and
+    starts there on larger grids: the fields are the oracle's bit for bit."""
+    vel, ext, rng = _voronoi(shape, h, 12, sum(shape))
+    rev = rng.uniform(0, 1, (4, 3)) * ext
+    for src in (rng.uniform(0, 1, 3) * ext, ext * [0.5, 0.5, 0.0]):
+        say("heap replay by size", shape, where, src)
+        tg, fg = mct.fast_marching_3d(vel, h[0], h[1], h[2], 0, 0, 0, src, rev, 1, field=True)
+        to, fo = po.fast_marching_3d(vel, h[0], h[1], h[2], 0, 0, 0, src, rev, 1, field=True)
+        assert np.array_equal(fg, fo)
+        np.testing.assert_allclose(tg, to, rtol=1e-12)
