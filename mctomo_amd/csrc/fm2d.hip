@@ -1432,8 +1432,8 @@ extern "C" int mct_modrays(int nvx, int nvz, double goxd, double gozd, double dv
     a.nnx = (nvx - 1) * gdx + 1; a.nnz = (nvz - 1) * gdz + 1;   // for the LDS check below
     const bool fast = method == 0 && mct_fm2d_fast_ok(a);
     void *bufs[16] = {nullptr};
-    size_t sizes[16] = {nv * 8, 2 * nn * 8, 8 * (size_t)nsrc, 8 * (size_t)nsrc, 8 * (size_t)nrc, 8 * (size_t)nrc,
-                        4 * (size_t)np * nsrc * nrc, 8 * (size_t)(nprob * wsz), 8 * (size_t)(nprob * wsz),
+    size_t sizes[16] = {nv * 8, 8 * (2 * nn + MCT_FM2D_PAD), 8 * (size_t)nsrc, 8 * (size_t)nsrc, 8 * (size_t)nrc, 8 * (size_t)nrc,
+                        4 * (size_t)np * nsrc * nrc, 8 * (size_t)(nprob * wsz + 2 * MCT_FM2D_PAD), 8 * (size_t)(nprob * wsz),
                         8 * (size_t)(nprob * wsz), 4 * (size_t)(nprob * wsz), 4 * (size_t)(nprob * wsz),
                         4 * (size_t)(nprob * (wsz + 8)), 8 * (size_t)nprob * nrc, 4, 4 * (size_t)nprob};
     int rc = MCT_OK;
@@ -1453,7 +1453,7 @@ extern "C" int mct_modrays(int nvx, int nvz, double goxd, double gozd, double dv
         a.scx = (const double *)bufs[2]; a.scz = (const double *)bufs[3];
         a.rcx = (const double *)bufs[4]; a.rcz = (const double *)bufs[5];
         a.srs = (const int32_t *)bufs[6];
-        a.ttn = (double *)bufs[7]; a.ttr = (double *)bufs[8]; a.vr = (double *)bufs[9];
+        a.ttn = (double *)bufs[7] + MCT_FM2D_PAD; a.ttr = (double *)bufs[8]; a.vr = (double *)bufs[9];
         a.nsts = (int32_t *)bufs[10]; a.nstr = (int32_t *)bufs[11]; a.heap = (int32_t *)bufs[12];
         a.ttime = (double *)bufs[13]; a.status = (int32_t *)bufs[14];
         a.srs_pstride = (long)nsrc * nrc;

@@ -240,10 +240,10 @@ __device__ __forceinline__ double ff_fouds2(const fview &V, const AL &al, int iz
     return travm;
 }
 
-template <class AL>
-__device__ __forceinline__ double ff_fouds(const fview &V, const AL &al, int iz, int ix, double slown, int fom)
+template <int FOM, class AL>
+__device__ __forceinline__ double ff_fouds(const fview &V, const AL &al, int iz, int ix, double slown)
 {
-    return fom == 0 ? ff_fouds1(V, al, iz, ix, slown) : ff_fouds2(V, al, iz, ix, slown);
+    return FOM == 0 ? ff_fouds1(V, al, iz, ix, slown) : ff_fouds2(V, al, iz, ix, slown);
 }
 
 // The same updates on a register copy of the node's axis stencil: [0] the
@@ -506,44 +506,52 @@ __host__ __device__ __forceinline__ double ff_q2(double tj, double tk, const ff_
     return tj + (K.a2p ? num * K.ia2 : fp_quot(num, K.a2, K.ra2));
 }
 
-__host__ __device__ __forceinline__ double ff_cands0_all(const ff_sten &S, const ff_k0 &K, double slown)
+__host__ __device__ __forceinline__ double ff_cands0_all(double x0, double x1, double z0, double z1, bool ix0, bool ix1,
+                                                         bool iz0, bool iz1, const ff_k0 &K, double slown)
 {
-    unsigned mp = ff_mask(S, FF_THR0);
-    if (!(mp & 0x33u)) return FF_BIG;
+    // rolled over the quadrants: few nodes come here (see ff_cands0_min), and
+    // four copies in each of a strip's unrolled steps cost it half its registers
     const double ss = slown * slown;
     // one alive neighbour: a = 1, b = 0, so tdsh = sqrt(-4c) / 2
     const double hx = fp_sqrt(ss * K.uu);       // sqrt(4.0 * (ss * K.uu)) * 0.5
     const double sdz = slown * K.dnz;
     const double hz = K.hsame ? hx : fp_sqrt(sdz * sdz);
-    double q[2][2];
-    for (int sj = 0; sj < 2; sj++)
-        for (int sk = 0; sk < 2; sk++)
-            q[sj][sk] = (S.ix1[sj] && S.iz1[sk] && FF_AX1_(mp, sj) && FF_AZ1_(mp, sk))
-                            ? ff_q2(S.tx1[sj], S.tz1[sk], K, ss) : 0.0;
-    auto sel = [&](unsigned m) -> double {
-        int any = 0;
-        double travm = 0.0;
-        for (int sj = 0; sj < 2; sj++)
-            for (int sk = 0; sk < 2; sk++) {
-                if (!(S.ix1[sj] && S.iz1[sk])) continue;
+    double thr = FF_THR0, c = FF_BIG;
+    unsigned mp = 0;
+#pragma unroll 1
+    for (int k = 0; k < 9; k++) {
+        const unsigned m = (unsigned)ff_al(x0, ix0, thr) | (unsigned)ff_al(x1, ix1, thr) << 1 |
+                           (unsigned)ff_al(z0, iz0, thr) << 2 | (unsigned)ff_al(z1, iz1, thr) << 3;
+        if (k > 0 && m == mp) break;            // the update would return c again
+        mp = m;
+        double c2 = FF_BIG;
+        if (m) {
+            int any = 0;
+            double travm = 0.0;
+#pragma unroll 1
+            for (int q = 0; q < 4; q++) {
+                const bool sj = (q & 2) != 0, sk = (q & 1) != 0;
+                if (!((sj ? ix1 : ix0) && (sk ? iz1 : iz0))) continue;
+                const bool aj = (m >> (sj ? 1 : 0)) & 1u, ak = (m >> (sk ? 3 : 2)) & 1u;
+                const double tj = sj ? x1 : x0, tk = sk ? z1 : z0;
                 double trav;
-                if (FF_AX1_(m, sj)) trav = FF_AZ1_(m, sk) ? q[sj][sk] : S.tx1[sj] + hx;
-                else if (FF_AZ1_(m, sk)) trav = S.tz1[sk] + hz;
+                if (aj) trav = ak ? ff_q2(tj, tk, K, ss) : tj + hx;
+                else if (ak) trav = tk + hz;
                 else continue;
                 travm = any ? fmin(trav, travm) : trav;
                 any = 1;
             }
-        return travm;
-    };
-    double c = sel(mp);
-    for (int k = 0; k < 8; k++) {
-        if (c >= FF_THR0) break;
-        unsigned m = ff_mask(S, c);
-        if (m == mp) break;
-        double c2 = (m & 0x33u) ? sel(m) : FF_BIG;
-        if (c2 == c || c2 >= FF_THR0) break;
-        c = c2;
-        mp = m;
+            c2 = travm;
+        }
+        if (k == 0) {
+            if (!m) return FF_BIG;
+            c = c2;
+            if (c >= FF_THR0) break;
+        } else {
+            if (c2 == c || c2 >= FF_THR0) break;
+            c = c2;
+        }
+        thr = c;
     }
     return c;
 }
@@ -587,7 +595,7 @@ __host__ __device__ __forceinline__ double ff_cands0f(const ff_sten &S, const ff
     if (in && ff_cands0_min(S.ix1[0] ? S.tx1[0] : FF_BIG, S.ix1[1] ? S.tx1[1] : FF_BIG,
                             S.iz1[0] ? S.tz1[0] : FF_BIG, S.iz1[1] ? S.tz1[1] : FF_BIG, K, slown, c))
         return c;
-    return ff_cands0_all(S, K, slown);
+    return ff_cands0_all(S.tx1[0], S.tx1[1], S.tz1[0], S.tz1[1], S.ix1[0], S.ix1[1], S.iz1[0], S.iz1[1], K, slown);
 }
 
 template <int FOM>
@@ -876,8 +884,8 @@ __device__ __forceinline__ bool ff_gen_get(const fview &V, const uint32_t *b, in
 // popped node's four neighbours read frozen nodes only, which none of the four
 // is, so lanes 0-3 compute them at once and lane 0 then enters them into the
 // heap in the reference's order (x-1, x+1, z-1, z+1).
-template <class VL>
-__device__ __forceinline__ void ff_heap_loop(const fview &V, ff_heap &H, const VL &vel, int fom, ff_stop &S)
+template <int FOM, class VL>
+__device__ __forceinline__ void ff_heap_loop(const fview &V, ff_heap &H, const VL &vel, ff_stop &S)
 {
     const int lane = threadIdx.x;
     auto al = [&](int z, int x) -> bool { return V.n(z, x) == 0; };
@@ -934,7 +942,7 @@ __device__ __forceinline__ void ff_heap_loop(const fview &V, ff_heap &H, const V
         const bool inb = lane < 4 && nx >= 1 && nx <= V.nnx && nz >= 1 && nz <= V.nnz;
         const int st = inb ? (int)V.n(nz, nx) : 0;
         double tv = 0.0;
-        if (st != 0) tv = ff_fouds(V, al, nz, nx, 1.0 / vel(nz, nx), fom);
+        if (st != 0) tv = ff_fouds<FOM>(V, al, nz, nx, 1.0 / vel(nz, nx));
 #pragma unroll
         for (int k = 0; k < 4; k++) {
             const int stk = __shfl(st, k, 64);
@@ -1126,6 +1134,7 @@ __device__ __forceinline__ void ff_srtimes(const mct_fm2d_args &A, const near_ge
 // One wave per problem.  LDS: region (doubles + int16 states) sized for the
 // larger of the refined grid and the coarse neighbourhood, the heap, and the
 // remap staging of the refined window's coarse nodes.
+template <int FOM>
 __global__ __launch_bounds__(64) void k_fm2d_near(mct_fm2d_args A, int region_nodes, int heap_cap,
                                                   int win_nodes, int32_t *pflag)
 {
@@ -1230,7 +1239,7 @@ __global__ __launch_bounds__(64) void k_fm2d_near(mct_fm2d_args A, int region_no
                 S.x1 = risx + 1 + FF_SEED_RINGS > R.nnx ? R.nnx : risx + 1 + FF_SEED_RINGS;
                 S.z0 = risz - FF_SEED_RINGS < 1 ? 1 : risz - FF_SEED_RINGS;
                 S.z1 = risz + 1 + FF_SEED_RINGS > R.nnz ? R.nnz : risz + 1 + FF_SEED_RINGS;
-                if (A.fom != 0) {
+                if (FOM != 0) {
                     // mixed order: the refined grid's answer depends on the heap's
                     // history (keys rise, nodes pop out of time order), and the
                     // heap-order check covers the coarse grid only, so the heap loop
@@ -1244,7 +1253,7 @@ __global__ __launch_bounds__(64) void k_fm2d_near(mct_fm2d_args A, int region_no
         }
         __syncthreads();
         if (!sh_ovf) {
-            ff_heap_loop(R, H, rvel, A.fom, S);
+            ff_heap_loop<FOM>(R, H, rvel, S);
             if (lane == 0) {
                 sh_exit = S.exited ? 1 : 0;
                 if (H.full || S.overflow) sh_ovf = 2;
@@ -1270,8 +1279,7 @@ __global__ __launch_bounds__(64) void k_fm2d_near(mct_fm2d_args A, int region_no
             ff_edges RE;
             RE.bound = &sh_bound;
             RE.left = g.vnl != 1; RE.right = g.vnr != R.nnx; RE.top = g.vnt != 1; RE.bottom = g.vnb != R.nnz;
-            int rounds = A.fom == 0 ? ff_sweep<0, true>(R, rfixed, rvel, &sh_flag, &RW, nullptr, &RE)
-                                    : ff_sweep<1, true>(R, rfixed, rvel, &sh_flag, &RW);
+            int rounds = ff_sweep<FOM, true>(R, rfixed, rvel, &sh_flag, &RW, nullptr, FOM == 0 ? &RE : nullptr);
             if (rounds < 0) {
                 if (lane == 0) pflag[slot] = 1;
                 return;
@@ -1317,7 +1325,7 @@ __global__ __launch_bounds__(64) void k_fm2d_near(mct_fm2d_args A, int region_no
                 auto alt = [&](int zz, int xx) -> bool {
                     return R.n(zz, xx) == 0 && !(zz == ex_z && xx == ex_x) && R.t(zz, xx) <= tlast;
                 };
-                double tv = ff_fouds(R, alt, j, i, 1.0 / rvel(j, i), A.fom);
+                double tv = ff_fouds<FOM>(R, alt, j, i, 1.0 / rvel(j, i));
                 RT[q] = tv;
                 RN[q] = 1;
             };
@@ -1422,7 +1430,7 @@ __global__ __launch_bounds__(64) void k_fm2d_near(mct_fm2d_args A, int region_no
             }
         }
         __syncthreads();
-        ff_heap_loop(C, H, cvel, A.fom, S);
+        ff_heap_loop<FOM>(C, H, cvel, S);
         if (lane == 0) sh_ovf = S.overflow || H.full;
         __syncthreads();
     } else {
@@ -1442,7 +1450,7 @@ __global__ __launch_bounds__(64) void k_fm2d_near(mct_fm2d_args A, int region_no
             S.have = 0;
         }
         __syncthreads();
-        ff_heap_loop(C, H, cvel, A.fom, S);
+        ff_heap_loop<FOM>(C, H, cvel, S);
         if (lane == 0) sh_ovf = S.overflow || H.full;
         __syncthreads();
     }
@@ -1573,7 +1581,13 @@ __global__ __launch_bounds__(256) void k_fm2d_sweep(mct_fm2d_args A, int32_t *pf
 // and streams its column's old times and velocities from memory FF_PF to
 // 2*FF_PF steps ahead; the strip's outer neighbour columns are staged in LDS.
 // A strip without dirty nodes is skipped.
-#define FF_PF 4
+// With many grids in flight the sweep is bound by memory, not by its arithmetic:
+// 4 doubles of a column at a time fetch each 128-byte line four times over, and
+// the lines do not stay in the L2 between.  48 chains of 201x201 grids (1440
+// problems, order 0): one 8-byte load a step 128 ms, 4 nodes in two 16-byte loads
+// 83 ms, 8 nodes 71 ms, 12 nodes 81 ms and 16 nodes 79 ms (registers).
+#define FF_PF 8
+typedef double ff_pair __attribute__((ext_vector_type(2), aligned(8)));
 
 // Lane i takes lane i-1's value (wave_shr:1) / lane i+1's (wave_shl:1) by DPP
 // moves, two per double; a lane without a source keeps its own value, as
@@ -1610,8 +1624,8 @@ __global__ __launch_bounds__(64) void k_fm2d_strip(mct_fm2d_args A, int32_t *pfl
     const double *slnc = A.sln ? A.sln + cp * (long)nnx * nnz : nullptr;
     double *T = A.ttn + slot * wsz;
     const int32_t *F = A.nsts + slot * wsz;
-    const long nn = (long)nnx * nnz;
-    const int nw = (int)((nn + 31) / 32);
+    const int nn = nnx * nnz;               // the bitmaps fit LDS, so node indices fit 32 bits
+    const int nw = (nn + 31) / 32;
     const int ns = (nnx + 63) / 64;
     constexpr int NSIDE = FOM == 0 ? 2 : 4;
     constexpr int reach = FOM == 0 ? 1 : 2;
@@ -1645,7 +1659,7 @@ __global__ __launch_bounds__(64) void k_fm2d_strip(mct_fm2d_args A, int32_t *pfl
         return (FB[q >> 5] >> (q & 31)) & 1u;
     };
     auto mark = [&](int z, int x) {
-        long q = (long)(x - 1) * nnz + (z - 1);
+        const int q = (x - 1) * nnz + (z - 1);
         atomicOr(&DB[q >> 5], 1u << (q & 31));
         cnt[(x - 1) >> 6] = 1;
     };
@@ -1678,21 +1692,21 @@ __global__ __launch_bounds__(64) void k_fm2d_strip(mct_fm2d_args A, int32_t *pfl
                 const int xl63 = xs > 0 ? xl0 + 63 : xl0 - 63;
                 const int x = xs > 0 ? xl0 + lane : xl0 - lane;
                 const bool xin = x >= 1 && x <= nnx;
-                const long colT = (long)(x - 1) * ld, colV = (long)(x - 1) * nnz;
+                const int colT = (x - 1) * ld, colV = (x - 1) * nnz;
                 // the strip's marked nodes as pipeline steps t = b + lane: the visit runs
                 // from the first to the last of them, and on while its changes mark
                 // nodes further on
                 int tl = 0x7fffffff, th = -1;
                 if (xin) {
                     int zlo = -1, zhi = -1;
-                    const long q0 = colV, q1 = colV + nnz;
-                    for (long w = q0 >> 5; w <= (q1 - 1) >> 5; w++) {
+                    const int q0 = colV, q1 = colV + nnz;
+                    for (int w = q0 >> 5; w <= (q1 - 1) >> 5; w++) {
                         uint32_t v = DB[w];
                         if (w == (q0 >> 5)) v &= ~0u << (q0 & 31);
                         if (w == ((q1 - 1) >> 5) && (q1 & 31)) v &= ~(~0u << (q1 & 31));
                         if (v) {
-                            const int lo = (int)(w * 32 - q0) + __ffs((int)v) - 1;
-                            const int hi = (int)(w * 32 - q0) + 31 - __clz((int)v);
+                            const int lo = w * 32 - q0 + __ffs((int)v) - 1;
+                            const int hi = w * 32 - q0 + 31 - __clz((int)v);
                             if (zlo < 0) zlo = lo;
                             zhi = hi;
                         }
@@ -1722,11 +1736,6 @@ __global__ __launch_bounds__(64) void k_fm2d_strip(mct_fm2d_args A, int32_t *pfl
                 const int tmax = nnz - 1 + last;
                 const int tstart = tl > first ? tl : first;
                 int tend = th < tmax ? th : tmax;
-                // The stream's loads have no condition: a lane whose node is outside
-                // the grid reads the slot's first element (one line that every such
-                // lane of the instruction shares), and the value is replaced where it
-                // is used, so the loads stay in flight until then (a load under a
-                // condition would be waited for at once).
                 auto inb = [&](int bb) -> bool { return xin && bb >= 0 && bb < nnz; };
                 auto zrow = [&](int bb) -> int { return zs > 0 ? bb : nnz - 1 - bb; };
                 auto tload = [&](int bb) -> double {
@@ -1738,13 +1747,22 @@ __global__ __launch_bounds__(64) void k_fm2d_strip(mct_fm2d_args A, int32_t *pfl
                     const double v = tload(bb);
                     return inb(bb) ? v : FF_BIG;
                 };
-                // the node's slowness 1.0 / veln (fouds' slown); used only where the
-                // node is in the column
-                auto vload = [&](int bb) -> double {
-                    double v = 1.0;
-                    if (inb(bb)) v = slnc[colV + zrow(bb)];
-                    return v;
+                // The stream: FF_PF nodes of the lane's column at once, in memory order
+                // (two to a load), from T or from the slowness 1.0 / veln (fouds' slown).
+                // A group that lies partly outside the column brings values of other
+                // nodes along, which are replaced or left unused.
+                auto group = [&](const double *col, int bb, double (&o)[FF_PF]) {
+                    const int lo = zs > 0 ? bb : nnz - bb - FF_PF;
+                    if (xin && bb > -FF_PF && bb < nnz) {
+#pragma unroll
+                        for (int k = 0; k < FF_PF; k += 2) {
+                            const ff_pair v = *(const ff_pair *)(col + lo + k);
+                            o[k] = v.x;
+                            o[k + 1] = v.y;
+                        }
+                    }
                 };
+                const double *Tcol = T + colT, *Vcol = slnc + colV;
                 constexpr int D = 2 + FOM;      // the stream delivers the old time D nodes ahead
                 const int b0 = tstart - lane;
                 // behind the start nothing has changed in this visit: the stored times
@@ -1752,7 +1770,9 @@ __global__ __launch_bounds__(64) void k_fm2d_strip(mct_fm2d_args A, int32_t *pfl
                 double c0 = told(b0), o1 = told(b0 + 1), o2 = FOM ? told(b0 + 2) : 0.0;
                 double sa[FF_PF], sb[FF_PF], va[FF_PF], vb[FF_PF];
 #pragma unroll
-                for (int j = 0; j < FF_PF; j++) { sa[j] = tload(b0 + j + D); va[j] = vload(b0 + j); }
+                for (int j = 0; j < FF_PF; j++) { sa[j] = sb[j] = FF_BIG; va[j] = vb[j] = 1.0; }
+                group(Tcol, b0 + D, sa);
+                group(Vcol, b0, va);
                 // the window and the first chunk in registers before the step loop, so the
                 // loop's waits are for the chunk in flight only
                 __builtin_amdgcn_s_waitcnt(0);
@@ -1767,7 +1787,7 @@ __global__ __launch_bounds__(64) void k_fm2d_strip(mct_fm2d_args A, int32_t *pfl
                     if (FOM) { xm2 = ff_from_below(ff_from_below(pn2)); xp2 = ff_from_above(ff_from_above(o2)); }
                     double newv = c0;
                     if (act) {
-                        const long q = colV + z0;
+                        const int q = colV + z0;
                         const uint32_t m = 1u << (q & 31);
                         if (DB[q >> 5] & m) {        // fixed nodes are never marked
                             atomicAnd(&DB[q >> 5], ~m);
@@ -1781,27 +1801,27 @@ __global__ __launch_bounds__(64) void k_fm2d_strip(mct_fm2d_args A, int32_t *pfl
                                 if (lane == 62) xp2 = side[nnz + z0];
                             }
                             double c;
-                            // values off the grid are FF_BIG here
-                            if (FOM != 0 || !ff_cands0_min(xm1, xp1, pn1, o1, K0, scur, c)) {
-                            // the stencil in grid orientation: [0] the x-1 / z-1 side
-                            ff_sten S;
-                            S.ix1[0] = x - 1 >= 1; S.ix1[1] = x + 1 <= nnx;
-                            S.iz1[0] = z0 >= 1; S.iz1[1] = z0 + 1 < nnz;
-                            S.ix2[0] = FOM != 0 && x - 2 >= 1; S.ix2[1] = FOM != 0 && x + 2 <= nnx;
-                            S.iz2[0] = FOM != 0 && z0 >= 2; S.iz2[1] = FOM != 0 && z0 + 2 < nnz;
-                            const double lx1 = xs > 0 ? xm1 : xp1, hx1 = xs > 0 ? xp1 : xm1;
-                            const double lz1 = zs > 0 ? pn1 : o1, hz1 = zs > 0 ? o1 : pn1;
-                            S.tx1[0] = S.ix1[0] ? lx1 : FF_BIG; S.tx1[1] = S.ix1[1] ? hx1 : FF_BIG;
-                            S.tz1[0] = S.iz1[0] ? lz1 : FF_BIG; S.tz1[1] = S.iz1[1] ? hz1 : FF_BIG;
-                            if (FOM) {
+                            if (FOM == 0) {
+                                // values off the grid are FF_BIG here
+                                if (!ff_cands0_min(xm1, xp1, pn1, o1, K0, scur, c))
+                                    c = ff_cands0_all(xm1, xp1, pn1, o1, x - xs >= 1 && x - xs <= nnx,
+                                                      x + xs >= 1 && x + xs <= nnx, b >= 1, b + 1 < nnz, K0, scur);
+                            } else {
+                                // the stencil in grid orientation: [0] the x-1 / z-1 side
+                                ff_sten S;
+                                S.ix1[0] = x - 1 >= 1; S.ix1[1] = x + 1 <= nnx;
+                                S.iz1[0] = z0 >= 1; S.iz1[1] = z0 + 1 < nnz;
+                                S.ix2[0] = x - 2 >= 1; S.ix2[1] = x + 2 <= nnx;
+                                S.iz2[0] = z0 >= 2; S.iz2[1] = z0 + 2 < nnz;
+                                const double lx1 = xs > 0 ? xm1 : xp1, hx1 = xs > 0 ? xp1 : xm1;
+                                const double lz1 = zs > 0 ? pn1 : o1, hz1 = zs > 0 ? o1 : pn1;
+                                S.tx1[0] = S.ix1[0] ? lx1 : FF_BIG; S.tx1[1] = S.ix1[1] ? hx1 : FF_BIG;
+                                S.tz1[0] = S.iz1[0] ? lz1 : FF_BIG; S.tz1[1] = S.iz1[1] ? hz1 : FF_BIG;
                                 const double lx2 = xs > 0 ? xm2 : xp2, hx2 = xs > 0 ? xp2 : xm2;
                                 const double lz2 = zs > 0 ? pn2 : o2, hz2 = zs > 0 ? o2 : pn2;
                                 S.tx2[0] = S.ix2[0] ? lx2 : FF_BIG; S.tx2[1] = S.ix2[1] ? hx2 : FF_BIG;
                                 S.tz2[0] = S.iz2[0] ? lz2 : FF_BIG; S.tz2[1] = S.iz2[1] ? hz2 : FF_BIG;
-                            } else {
-                                S.tx2[0] = S.tx2[1] = S.tz2[0] = S.tz2[1] = FF_BIG;
-                            }
-                            c = FOM == 0 ? ff_cands0_all(S, K0, scur) : ff_cands<FOM>(S, dnx, dnz, scur);
+                                c = ff_cands<FOM>(S, dnx, dnz, scur);
                             }
                             if (c < FF_THR0 && c != c0) {
                                 if (fabs(c - c0) > 1e-14 * c) changed = 1;
@@ -1828,14 +1848,12 @@ __global__ __launch_bounds__(64) void k_fm2d_strip(mct_fm2d_args A, int32_t *pfl
                 // own FF_PF steps on the values the previous pass loaded (static
                 // register indices, so the waits count only the loads it needs)
                 for (int t0 = tstart; t0 <= tend; t0 += FF_PF) {
-#pragma unroll
-                    for (int j = 0; j < FF_PF; j++) {
-                        sb[j] = tload(t0 + FF_PF + j - lane + D);
-                        vb[j] = vload(t0 + FF_PF + j - lane);
-                    }
+                    group(Tcol, t0 + FF_PF - lane + D, sb);
+                    group(Vcol, t0 + FF_PF - lane, vb);
 #pragma unroll
                     for (int j = 0; j < FF_PF; j++)
-                        if (t0 + j <= tend) step(t0 + j, sa[j], va[j]);
+                        if (t0 + j <= tend)
+                            step(t0 + j, zs > 0 ? sa[j] : sa[FF_PF - 1 - j], zs > 0 ? va[j] : va[FF_PF - 1 - j]);
 #pragma unroll
                     for (int j = 0; j < FF_PF; j++) { sa[j] = sb[j]; va[j] = vb[j]; }
                 }
@@ -1844,8 +1862,8 @@ __global__ __launch_bounds__(64) void k_fm2d_strip(mct_fm2d_args A, int32_t *pfl
                 // of its own steps ahead of the pipeline were taken in this visit)
                 bool left = false;
                 if (xin) {
-                    const long q0 = colV, q1 = colV + nnz;
-                    for (long w = q0 >> 5; w <= (q1 - 1) >> 5; w++) {
+                    const int q0 = colV, q1 = colV + nnz;
+                    for (int w = q0 >> 5; w <= (q1 - 1) >> 5; w++) {
                         uint32_t v = DB[w];
                         if (w == (q0 >> 5)) v &= ~0u << (q0 & 31);
                         if (w == ((q1 - 1) >> 5) && (q1 & 31)) v &= ~(~0u << (q1 & 31));
@@ -2055,7 +2073,8 @@ int mct_launch_fm2d_fast(const mct_fm2d_args &a, long chunk, int32_t *pflag, hip
     int rc = mct_launch_fm2d_gridder(a, s);
     if (rc) return rc;
     if (lds > 64 * 1024)
-        MCT_CHECK(hipFuncSetAttribute((const void *)k_fm2d_near, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        MCT_CHECK(hipFuncSetAttribute(a.fom == 0 ? (const void *)k_fm2d_near<0> : (const void *)k_fm2d_near<1>,
+                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     // the sweep's dirty bitmap in LDS when it fits
     const size_t dirty_bytes = 2 * 4 * (((size_t)a.nnx * a.nnz + 31) / 32) + 4 * 2 * (size_t)(a.nnx + a.nnz);
     const int use_dirty = dirty_bytes <= 48 * 1024;
@@ -2114,7 +2133,10 @@ int mct_launch_fm2d_fast(const mct_fm2d_args &a, long chunk, int32_t *pflag, hip
         b.verify = verify > 0 ? 1 : -1;
         b.prob0 = p0;
         b.nrun = nprob - p0 < chunk ? nprob - p0 : chunk;
-        hipLaunchKernelGGL(k_fm2d_near, dim3((unsigned)b.nrun), dim3(64), lds, s, b, region, heap_cap, win, pflag);
+        if (a.fom == 0)
+            hipLaunchKernelGGL(k_fm2d_near<0>, dim3((unsigned)b.nrun), dim3(64), lds, s, b, region, heap_cap, win, pflag);
+        else
+            hipLaunchKernelGGL(k_fm2d_near<1>, dim3((unsigned)b.nrun), dim3(64), lds, s, b, region, heap_cap, win, pflag);
         MCT_CHECK(hipGetLastError());
         if (a.ev_sweep && p0 == 0) MCT_CHECK(hipEventRecord(a.ev_sweep, s));
         if (strip_lds && a.fom == 0)

@@ -192,6 +192,10 @@ struct mct_misfit_args {
 int mct_launch_misfit(const mct_misfit_args &a, hipStream_t s);
 
 // ---- 2-D phase traveltimes (fm2d) -------------------------------------------------
+// Doubles readable before and after ttn and sln (the sweeps read a column's nodes
+// in groups that may begin before its first and end after its last one).
+#define MCT_FM2D_PAD 16
+
 struct mct_fm2d_args {
     int nvx, nvz;               // control grid nodes (grid nx, ny)
     double gox, goz, dvx, dvz;  // origin and control spacing
@@ -201,7 +205,8 @@ struct mct_fm2d_args {
     int nchain, np, nsrc, nrc;
     const double *velv;         // (nchain*np, (nvx+2)*(nvz+2)) padded control grids, Fortran (nvz+2,nvx+2)
     double *veln;               // (nchain*np, nnx*nnz) coarse velocity, Fortran (nnz,nnx)
-    double *sln;                // the same layout: 1.0 / veln (the sweeps' slowness), or NULL
+    double *sln;                // the same layout: 1.0 / veln (the sweeps' slowness), or NULL; MCT_FM2D_PAD
+                                // doubles before and after may be read
     const double *scx, *scz, *rcx, *rcz;
     const int32_t *srs;         // per period srs_pstride entries; the first nsrc*nrc mark the pairs used (receiver fastest)
     long srs_pstride;

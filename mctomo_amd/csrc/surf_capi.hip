@@ -269,7 +269,7 @@ static int surf_pipeline(mct_surf_ctx *C, int c0, int nchain, int part, int npar
     fa.scx = C->scx.as<double>(); fa.scz = C->scz.as<double>();
     fa.rcx = C->rcx.as<double>(); fa.rcz = C->rcz.as<double>();
     fa.srs = C->raystat.as<int32_t>(); fa.srs_pstride = 2L * S.nsrc * S.nrev;
-    fa.ttn = C->ttn.as<double>() + soff * wsz; fa.ttr = C->ttr.as<double>() + soff * wsz;
+    fa.ttn = C->ttn.as<double>() + MCT_FM2D_PAD + soff * wsz; fa.ttr = C->ttr.as<double>() + soff * wsz;
     fa.vr = C->vr.as<double>() + soff * wsz;
     fa.nsts = C->nsts.as<int32_t>() + soff * wsz; fa.nstr = C->nstr.as<int32_t>() + soff * wsz;
     fa.heap = C->heap.as<int32_t>() + soff * (wsz + 8);
@@ -477,11 +477,11 @@ int mct_surf_create(const mct_grid *grid, const mct_surf_setup *setup, mct_surf_
     ALLOC(dsp_dup, sizeof(int32_t) * ncol * M);
     ALLOC(dsp_njobs, sizeof(int32_t) * MCT_SURF_SPLIT_MAX);
     ALLOC(velv, sizeof(double) * (grid->nx + 2) * (grid->ny + 2) * np * M);
-    ALLOC(veln, 2 * sizeof(double) * nnx * nnz * np * M);   // velocities, then slowness
+    ALLOC(veln, sizeof(double) * (2 * nnx * nnz * np * M + MCT_FM2D_PAD));   // velocities, then slowness
     ALLOC(phase_time, sizeof(double) * npair * np * M);
     ALLOC(srdist, sizeof(double) * npair * np);
     ALLOC(sigma, sizeof(double) * npair * np);
-    ALLOC(ttn, sizeof(double) * wsz * ch);
+    ALLOC(ttn, sizeof(double) * (wsz * ch + 2 * MCT_FM2D_PAD));
     ALLOC(ttr, sizeof(double) * wsz * ch);
     ALLOC(vr, sizeof(double) * wsz * ch);
     ALLOC(nsts, sizeof(int32_t) * wsz * ch);

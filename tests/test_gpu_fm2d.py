@@ -329,3 +329,29 @@ def test_order_one_bands_wider_than_the_first_heap(split, monkeypatch):
     lanes = mct.modrays(velv, 0, 0, h, h, sx, sz, rx, rz, method=0, **kw)
     np.testing.assert_array_equal(got, lanes)
     agree(got, want, 0)
+
+
+@pytest.mark.parametrize("nx,nz", [(70, 5), (5, 70), (66, 7), (64, 8), (65, 9), (129, 15), (9, 17)])
+def test_strip_sweep_on_columns_around_its_load_groups(nx, nz, monkeypatch):
+    """Columns shorter than, equal to and just over the 8 nodes that a lane loads at
+    once, the last strip full, one column over and one column wide, two problems'
+    grids side by side in memory: the anti-diagonal sweep's times bit for bit."""
+    rng = np.random.default_rng(100 * nx + nz)
+    h = 0.5
+    velv = rng.uniform(2.6, 3.6, (3, nx + 2, nz + 2))
+    L, W = (nx - 1) * h, (nz - 1) * h
+    ns, nr = 4, 7
+    sx, sz = rng.uniform(h, L - h, ns), rng.uniform(h, W - h, ns)
+    rx, rz = rng.uniform(0, L, nr), rng.uniform(0, W, nr)
+    monkeypatch.setenv("MCT_FM2D_ORDER1", "check")   # fom 1 sweeps too
+    for fom in (0, 1):
+        for asgr in (0, 1):
+            say("fm2d strip groups", nx, nz, "fom", fom, "asgr", asgr)
+            kw = dict(fom=fom, asgr=asgr, method=0)
+            monkeypatch.setenv("MCT_SWEEP_KIND", "diag")
+            want = mct.modrays(velv, 0, 0, h, h, sx, sz, rx, rz, **kw)
+            monkeypatch.setenv("MCT_SWEEP_KIND", "strip")
+            got = mct.modrays(velv, 0, 0, h, h, sx, sz, rx, rz, **kw)
+            np.testing.assert_array_equal(got, want)
+            for p in range(3):
+                agree(got[p], po.fm2d(velv[p], 0, 0, h, h, sx, sz, rx, rz, fom=fom, asgr=asgr), 0)
