@@ -4,10 +4,11 @@
 // :523-629), the surfdisp96 branch of surfmodes (surfmodes/surfmodes.f90
 // :79-95) and surfdisp96 itself (surfmodes/surfdisp96.f:52-382).
 //
-// Three launch shapes.  k_dispersion_sm (throughput): one lane per column,
-// columns taken from a queue, surfdisp96's control flow as a per-lane state
-// machine with one period-equation call site, so the 64 lanes of a wave share
-// every evaluation whatever stage of the root search each is in.
+// Three launch shapes.  k_dispersion_sm (the likelihood's): columns taken from a
+// queue, surfdisp96's control flow as a per-lane state machine with one
+// period-equation call site, so the 64 lanes of a wave share every evaluation
+// whatever stage of the root search each is in; a column has one lane where
+// there are many columns and up to 64 where there are few.
 // k_dispersion_lane: one lane per column running surfdisp96 as written (lanes
 // wait for the wave's longest walk at every branch).  k_dispersion: one
 // wave64 per column with the layer model in LDS (latency).  The expensive part of
@@ -26,6 +27,7 @@
 #include "mct_internal.h"
 #include "libm_glibc.h"
 #include <float.h>
+#include <type_traits>
 
 #pragma clang fp contract(off)
 
@@ -59,9 +61,8 @@ __device__ __forceinline__ void dsp_vprho(const mct_dsp_args &A, long cbase, int
 // with A.water > 0 the first layer's is A.water itself (:616-617: the water
 // layer's, or for 0 < water <= EPS the first solid layer's).  Returns the
 // layer count (at most nz + 1).
-template <int ST>
 __device__ __forceinline__ int dsp_convert(const mct_dsp_args &A, long cb, const double *vs, float *sd, float *sa,
-                                           float *sb, float *sr)
+                                           float *sb, float *sr, int ST)
 {
     const double EPS = (double)1.0e-10f;       // src/likelihood_surf.F90:37
     int nl = 0, last_k = 1;
@@ -101,6 +102,12 @@ __device__ __forceinline__ int dsp_convert(const mct_dsp_args &A, long cb, const
 template <int ST> struct dsp_model_t {
     static constexpr int st = ST;
     int mmax, llw;
+    const float *d, *a, *b, *rho;
+};
+
+// The same with the stride known at run time only.
+struct dsp_model_rt {
+    int st, mmax, llw;
     const float *d, *a, *b, *rho;
 };
 
@@ -478,7 +485,7 @@ __global__ __launch_bounds__(64) void k_dispersion(mct_dsp_args A)
     bool below = false;
     for (int k = 1 + lane; k < A.nz; k += 64) below |= vs[k] < vs[0];
     if (__ballot(below) != 0ull && lane == 0) A.bad_model[c] = 1;
-    if (lane == 0) s_nl = dsp_convert<1>(A, cb, vs, sd, sa, sb, sr);
+    if (lane == 0) s_nl = dsp_convert(A, cb, vs, sd, sa, sb, sr, 1);
     __syncthreads();
     dsp_model_t<1> M;
     M.mmax = s_nl;
@@ -630,7 +637,7 @@ __global__ __launch_bounds__(64) void k_dispersion_lane(mct_dsp_args A, float *l
     for (int k = 1; k < A.nz; k++) below |= vs[k] < top;
     if (below) A.bad_model[c] = 1;
     dsp_model_t<64> M;
-    M.mmax = dsp_convert<64>(A, cb, vs, sd, sa, sb, sr);
+    M.mmax = dsp_convert(A, cb, vs, sd, sa, sb, sr, 64);
     M.d = sd; M.a = sa; M.b = sb; M.rho = sr;
     M.llw = (sb[0] <= 0.0f) ? 2 : 1;
     double *cp = A.phase + ((long)c * A.ncol + col) * A.np;
@@ -713,13 +720,26 @@ __global__ __launch_bounds__(64) void k_dispersion_lane(mct_dsp_args A, float *l
     if (A.nlayer) A.nlayer[(long)c * A.ncol + col] = M.mmax;
 }
 
-// One lane per column, columns handed out from a queue, and surfdisp96's
-// control flow as a per-lane state machine with a single period-equation
-// call site: every iteration each lane advances its own column (walk step,
-// Neville step, next period, next column) until it needs dltar, then the
-// whole wave evaluates dltar together.  Lanes never wait for one another's
-// walks, and a lane that finishes a column takes the next one.  The sequence
-// of operations per column is surfdisp96's (the same as k_dispersion_lane).
+// Columns handed out from a queue, and surfdisp96's control flow as a per-lane
+// state machine with a single period-equation call site: every iteration each
+// lane advances its own column (walk step, Neville step, next period, next
+// column) until it needs dltar, then the whole wave evaluates dltar together.
+// Lanes never wait for one another's walks, and a lane that finishes a column
+// takes the next one.  The sequence of operations per column is surfdisp96's
+// (the same as k_dispersion_lane).
+//
+// GROUPED gives a column 2^lg neighbouring lanes, which hold the same state and
+// evaluate points that the search may come to next; it then goes on through
+// those that it does come to, in its own order.  On the bracketing walk these are
+// the next 2^lg steps (with getsol's first evaluation: the steps upwards, which
+// are dropped if the search turns out to go down).  In nevill 7 of 9 evaluations
+// halve the bracket, mostly one after the other, so the lanes take a point's
+// possible halvings as a binary tree.  A root takes about 51 evaluations one by
+// one (42 walk, 9 nevill), 17 rounds with 4 lanes, 10 with 8 and 7 with 16.
+// What bounds few columns is that chain: a column has about 1000 evaluations of
+// 2000 instructions, one after the other, whatever the number of lanes that idle.
+// 201x201 columns (30,000 different): 16.1 -> 6.2 ms; the perturbed boxes of a
+// 101x101 group-velocity grid: 17.5 -> 1.5 ms.
 enum {
     SM_NEXT, SM_PERIOD, SM_G0, SM_G1, SM_N0, SM_NLOOP, SM_N1, SM_NBODY, SM_N2, SM_N3,
     SM_NDONE, SM_GDONE, SM_FINISH, SM_DONE
@@ -932,12 +952,30 @@ __global__ void k_dsp_queue_reset(unsigned long long *q)
     if (threadIdx.x == 0) q[0] = 0ull;
 }
 
+// Lanes per column, as a power of two: as many as keep the columns' waves within
+// wave_target (0: one lane per column), which is what the device holds at once
+// (2 waves per SIMD at this kernel's registers): beyond it each further lane only
+// adds evaluations that may not be used, 1.3 times the work with 4 lanes and 2.2
+// times with 16.  48 chains of 201x201 columns stay with one lane (91 ms).
+__host__ __device__ __forceinline__ int dsp_group_log(long ncolumns, long wave_target)
+{
+    int lg = 0;
+    while (lg < 6 && ncolumns << (lg + 1) <= 64 * wave_target) lg++;
+    return lg;
+}
+
+template <bool GROUPED>
 __global__ __launch_bounds__(64) void k_dispersion_sm(mct_dsp_args A, float *lay, int nlmax, long total)
 {
     const int lane = threadIdx.x;
     const long ntot = A.njobs ? (long)A.njobs[0] : total;   // duplicates are not queued
-    const long plane = (long)nlmax * 64;
-    float *base = lay + (long)blockIdx.x * 4 * plane + lane;
+    const int lg = dsp_group_log(ntot, A.wave_target);
+    if ((lg > 0) != GROUPED) return;
+    const int G = GROUPED ? 1 << lg : 1, sub = lane & (G - 1), g0 = lane - sub, ncw = GROUPED ? 64 >> lg : 64;
+    if ((long)blockIdx.x * ncw >= ntot) return;
+    const unsigned long long gmask = (~0ull >> (64 - G)) << g0;
+    const long plane = (long)nlmax * ncw;
+    float *base = lay + (long)blockIdx.x * 4 * plane + (lane >> (GROUPED ? lg : 0));
     float *sd = base, *sa = base + plane, *sb = base + 2 * plane, *sr = base + 3 * plane;
     const double twopi = 2.0 * 3.141592653589793;
     const float sone = 1.500f, h = 0.005f;
@@ -946,7 +984,9 @@ __global__ __launch_bounds__(64) void k_dispersion_sm(mct_dsp_args A, float *lay
     const double dc = fabs((double)ddc);
     const int ifunc = A.iwave;
 
-    dsp_model_t<64> M;
+    typename std::conditional<GROUPED, dsp_model_rt, dsp_model_t<64>>::type M;
+    if constexpr (GROUPED) M.st = ncw;
+    auto from = [](auto v, int l) { return GROUPED ? __shfl(v, l, 64) : v; };   // a lane of the group
     M.d = sd; M.a = sa; M.b = sb; M.rho = sr;
     M.mmax = 1; M.llw = 1;
     // column state
@@ -960,24 +1000,53 @@ __global__ __launch_bounds__(64) void k_dispersion_sm(mct_dsp_args A, float *lay
     float t1a = 0.0f, t1b = 0.0f;
     double t1 = 0.0, omega = 0.0;
     // getsol / nevill state
-    double c1 = 0.0, c2 = 0.0, del1 = 0.0, del2 = 0.0, clow = 0.0;
+    double c1 = 0.0, del1 = 0.0, clow = 0.0;
     int idir = 1, gret = 0, walk = 0;
     double gc = 0.0;
     double nc1 = 0.0, nc2 = 0.0, nd1 = 0.0, nd2 = 0.0, c3 = 0.0, del3 = 0.0;
     int nev = 0, nctrl = 0, m = 1;
+    double cprv = 0.0;                 // the lane's own step of the walk: from cprv to ceval
+    int dd = 1, skip = 0, node = 0, hi = 0;
     // Neville tables in LDS, lane-interleaved
     __shared__ double xs[12 * 64], ys[12 * 64];
 #define X(j) xs[(j) * 64 + lane]
 #define Y(j) ys[(j) * 64 + lane]
     double res = 0.0, ceval = 0.0;
     int pc = SM_NEXT;
+    // getsol's walk from c1: the lane's step is the (sub + 1 - skip)th
+    auto walk_points = [&]() {
+        double cc2 = c1;
+        cprv = c1; ceval = c1; dd = idir;
+        for (int s = skip; s <= sub; s++) {
+            for (;;) {
+                ceval = dd > 0 ? cc2 + dc : cc2 - dc;
+                if (ceval <= clow) { dd = 1; cc2 = clow; continue; }
+                break;
+            }
+            cprv = cc2;
+            cc2 = ceval;
+        }
+    };
+    // nevill at c3 and the halvings that can follow it: node 1 is c3, nodes 2n and
+    // 2n + 1 halve what is left below and above node n's point; lane sub has node sub + 1
+    auto halving_points = [&]() {
+        double a = nc1, b = nc2;
+        const int n = sub + 1;
+        ceval = c3;
+        for (int l = 30 - __clz(n); l >= 0; l--) {
+            if ((n >> l) & 1) a = ceval; else b = ceval;
+            ceval = 0.5 * (a + b);
+        }
+        node = 1;
+    };
 
     for (;;) {
         bool need = false;
         while (!need && pc != SM_DONE) {
             switch (pc) {
             case SM_NEXT: {
-                job = (long)atomicAdd((unsigned long long *)A.queue, 1ull);
+                if (sub == 0) job = (long)atomicAdd((unsigned long long *)A.queue, 1ull);
+                job = from(job, g0);
                 if (job >= ntot) { pc = SM_DONE; break; }
                 if (A.jobs) job = A.jobs[job];
                 c = (int)(job / A.ncol);
@@ -989,7 +1058,7 @@ __global__ __launch_bounds__(64) void k_dispersion_sm(mct_dsp_args A, float *lay
                 const double top = vs[0];
                 for (int kk = 1; kk < A.nz; kk++) below |= vs[kk] < top;
                 if (below) A.bad_model[c] = 1;
-                M.mmax = dsp_convert<64>(A, cb, vs, sd, sa, sb, sr);
+                M.mmax = dsp_convert(A, cb, vs, sd, sa, sb, sr, ncw);
                 M.llw = (sb[0] <= 0.0f) ? 2 : 1;
                 cp = A.phase + ((long)c * A.ncol + col) * A.np;
                 cg = A.group + ((long)c * A.ncol + col) * A.np;
@@ -998,12 +1067,12 @@ __global__ __launch_bounds__(64) void k_dispersion_sm(mct_dsp_args A, float *lay
                 betmx = -1.e20f;
                 float betmn = 1.e20f;
                 for (int ii = 1; ii <= M.mmax; ii++) {
-                    float bi = sb[64 * (ii - 1)], ai = sa[64 * (ii - 1)];
+                    float bi = sb[ncw * (ii - 1)], ai = sa[ncw * (ii - 1)];
                     if (bi > 0.01f && bi < betmn) { betmn = bi; jmn = ii; jsol = 1; }
                     else if (bi <= 0.01f && ai < betmn) { betmn = ai; jmn = ii; jsol = 0; }
                     if (bi > betmx) betmx = bi;
                 }
-                float cc1 = jsol == 0 ? betmn : d_gtsolh(sa[64 * (jmn - 1)], sb[64 * (jmn - 1)]);
+                float cc1 = jsol == 0 ? betmn : d_gtsolh(sa[ncw * (jmn - 1)], sb[ncw * (jmn - 1)]);
                 cc1 = 0.95f * cc1;
                 cc1 = 0.90f * cc1;
                 cc = (double)cc1;
@@ -1027,47 +1096,56 @@ __global__ __launch_bounds__(64) void k_dispersion_sm(mct_dsp_args A, float *lay
                 else { ifirst = 0; c1 = cprev > 0 ? cprev - onea * dc : cc; clow = cm; }
                 pass = 0;
                 omega = twopi / t1;          // getsol: wvno = omega / c1
-                ceval = c1; need = true; pc = SM_G0;
+                idir = 1; skip = 1; walk_points();
+                need = true; pc = SM_G0;
                 break;
             }
             case SM_G0: {
-                del1 = res; ndl++;
+                // lane 0 of the group has c1, the others the first steps upwards from it
+                del1 = from(res, g0); ndl++;
                 if (ifirst == 1) del1st = del1;
                 double plmn = dsgn(del1st) * dsgn(del1);
                 idir = (ifirst == 1) ? 1 : (plmn >= 0.0 ? 1 : -1);
-                for (;;) {
-                    c2 = idir > 0 ? c1 + dc : c1 - dc;
-                    if (c2 <= clow) { idir = 1; c1 = clow; continue; }
-                    break;
-                }
                 walk = 0;
-                omega = twopi / t1;
-                ceval = c2; need = true; pc = SM_G1;
+                pc = SM_G1;
+                if (GROUPED && idir > 0) break;
+                skip = 0; walk_points();
+                need = true;
                 break;
             }
             case SM_G1: {
-                del2 = res; ndl++;
-                if (dsgn(del1) != dsgn(del2)) {
-                    nc1 = c1; nc2 = c2; nd1 = del1; nd2 = del2;
+                const double below = from(res, lane - 1);
+                const double dprev = sub == 0 ? del1 : below;
+                const bool change = sub >= skip && dsgn(dprev) != dsgn(res);
+                const bool stop = sub >= skip && !change &&
+                                  (ceval < cm || ceval >= cmax || walk + sub + 1 - skip >= (1 << 24));
+                const unsigned long long chg = __builtin_amdgcn_ballot_w64(change) & gmask;
+                const unsigned long long ev = chg | (__builtin_amdgcn_ballot_w64(stop) & gmask);
+                if (ev) {
+                    const int e = __ffsll(ev) - 1;       // the walk ends at this lane's step
+                    ndl += e - g0 + 1 - skip;
+                    const double ce = from(ceval, e), cb = from(cprv, e);
+                    const double db = from(dprev, e), de = from(res, e);
+                    if (!((chg >> e) & 1ull)) { gret = -1; gc = ce; pc = SM_GDONE; break; }
+                    nc1 = cb; nc2 = ce; nd1 = db; nd2 = de;
                     omega = twopi / t1;      // nevill (surfdisp96.f:903-1020)
                     c3 = 0.5 * (nc1 + nc2);
-                    ceval = c3; need = true; pc = SM_N0;
+                    halving_points();
+                    need = true; pc = SM_N0;
                     break;
                 }
-                c1 = c2;
-                del1 = del2;
-                if (c1 < cm || c1 >= cmax || ++walk >= (1 << 24)) { gret = -1; gc = c1; pc = SM_GDONE; break; }
-                for (;;) {
-                    c2 = idir > 0 ? c1 + dc : c1 - dc;
-                    if (c2 <= clow) { idir = 1; c1 = clow; continue; }
-                    break;
-                }
+                ndl += G - skip;
+                walk += G - skip;
+                c1 = from(ceval, g0 + G - 1);
+                del1 = from(res, g0 + G - 1);
+                idir = from(dd, g0 + G - 1);
                 omega = twopi / t1;
-                ceval = c2; need = true; pc = SM_G1;
+                skip = 0; walk_points();
+                need = true; pc = SM_G1;
                 break;
             }
             case SM_N0:
-                del3 = res; ndl++;
+                del3 = from(res, g0); ndl++;
                 nev = 1; nctrl = 1; m = 1;
                 pc = SM_NLOOP;
                 break;
@@ -1077,20 +1155,21 @@ __global__ __launch_bounds__(64) void k_dispersion_sm(mct_dsp_args A, float *lay
                 if (c3 < fmin(nc1, nc2) || c3 > fmax(nc1, nc2)) {
                     nev = 0;
                     c3 = 0.5 * (nc1 + nc2);
-                    ceval = c3; need = true; pc = SM_N1;
+                    halving_points();
+                    need = true; pc = SM_N1;
                     break;
                 }
                 pc = SM_NBODY;
                 break;
             case SM_N1:
-                del3 = res; ndl++;
+                del3 = from(res, g0); ndl++;
                 pc = SM_NBODY;
                 break;
             case SM_NBODY: {
                 double s13 = nd1 - del3;
                 double s32 = del3 - nd2;
-                if (dsgn(del3) * dsgn(nd1) < 0.0) { nc2 = c3; nd2 = del3; }
-                else { nc1 = c3; nd1 = del3; }
+                if (dsgn(del3) * dsgn(nd1) < 0.0) { nc2 = c3; nd2 = del3; hi = 0; }
+                else { nc1 = c3; nd1 = del3; hi = 1; }
                 if (fabs(nc1 - nc2) <= 1.0e-6 * nc1) { pc = SM_NDONE; break; }
                 if (dsgn(s13) != dsgn(s32)) nev = 0;
                 double ss1 = fabs(nd1);
@@ -1116,23 +1195,33 @@ __global__ __launch_bounds__(64) void k_dispersion_sm(mct_dsp_args A, float *lay
                     }
                     if (!bad) {
                         c3 = X(1);
-                        ceval = c3; need = true; pc = SM_N2;
+                        halving_points();
+                        need = true; pc = SM_N2;
                         break;
                     }
                 }
                 c3 = 0.5 * (nc1 + nc2);
-                ceval = c3; need = true; pc = SM_N3;
+                node = 2 * node + hi;
+                if (node <= G) {             // a lane has evaluated this point already
+                    del3 = from(res, g0 + node - 1); ndl++;
+                    nev = 1;
+                    m = 1;
+                    pc = SM_NLOOP;
+                    break;
+                }
+                halving_points();
+                need = true; pc = SM_N3;
                 break;
             }
             case SM_N2:
-                del3 = res; ndl++;
+                del3 = from(res, g0); ndl++;
                 nev = 2;
                 m = m + 1;
                 if (m > 10) m = 10;
                 pc = SM_NLOOP;
                 break;
             case SM_N3:
-                del3 = res; ndl++;
+                del3 = from(res, g0); ndl++;
                 nev = 1;
                 m = 1;
                 pc = SM_NLOOP;
@@ -1147,7 +1236,8 @@ __global__ __launch_bounds__(64) void k_dispersion_sm(mct_dsp_args A, float *lay
                     if (gret == -1) {
                         // no root at period k: the rest keep cp=100, cg=0 (labels 1700/1750)
                         ierr = 1;
-                        for (int ii = k; ii <= A.np; ii++) { cp[ii - 1] = 100.0; cg[ii - 1] = 0.0; }
+                        if (sub == 0)
+                            for (int ii = k; ii <= A.np; ii++) { cp[ii - 1] = 100.0; cg[ii - 1] = 0.0; }
                         pc = SM_FINISH;
                         break;
                     }
@@ -1160,18 +1250,23 @@ __global__ __launch_bounds__(64) void k_dispersion_sm(mct_dsp_args A, float *lay
                         clow = 0.0 + one * dc;
                         c1 = croot - onea * dc;
                         omega = twopi / t1;
-                        ceval = c1; need = true; pc = SM_G0;
+                        idir = 1; skip = 1; walk_points();
+                        need = true; pc = SM_G0;
                         break;
                     }
-                    cp[k - 1] = (double)(float)croot;
-                    cg[k - 1] = 100.0;
+                    if (sub == 0) {
+                        cp[k - 1] = (double)(float)croot;
+                        cg[k - 1] = 100.0;
+                    }
                 } else {
                     double cgr = gret == -1 ? croot : gc;
                     if (gret == -1) ierr = 1;
                     float cc0 = (float)croot, cc1k = (float)cgr;
                     float gvel = (1.0f / t1a - 1.0f / t1b) / (1.0f / (t1a * cc0) - 1.0f / (t1b * cc1k));
-                    cg[k - 1] = (double)gvel;
-                    cp[k - 1] = (double)cc0;
+                    if (sub == 0) {
+                        cg[k - 1] = (double)gvel;
+                        cp[k - 1] = (double)cc0;
+                    }
                     if (gvel < 0 || croot == 0) ierr = 1;
                     pass = 0;
                 }
@@ -1179,9 +1274,11 @@ __global__ __launch_bounds__(64) void k_dispersion_sm(mct_dsp_args A, float *lay
                 pc = k > A.np ? SM_FINISH : SM_PERIOD;
                 break;
             case SM_FINISH:
-                A.ierr[(long)c * A.ncol + col] = ierr;
-                if (A.ndltar) A.ndltar[(long)c * A.ncol + col] = ndl;
-                if (A.nlayer) A.nlayer[(long)c * A.ncol + col] = M.mmax;
+                if (sub == 0) {
+                    A.ierr[(long)c * A.ncol + col] = ierr;
+                    if (A.ndltar) A.ndltar[(long)c * A.ncol + col] = ndl;
+                    if (A.nlayer) A.nlayer[(long)c * A.ncol + col] = M.mmax;
+                }
                 pc = SM_NEXT;
                 break;
             default:
@@ -1189,11 +1286,20 @@ __global__ __launch_bounds__(64) void k_dispersion_sm(mct_dsp_args A, float *lay
                 break;
             }
         }
-        if (__ballot(need) == 0ull) break;     // every lane has run out of columns
+        if (__builtin_amdgcn_ballot_w64(need) == 0ull) break;     // every lane has run out of columns
         if (need) res = d_dltar(omega / ceval, omega, ifunc, M);
     }
 #undef X
 #undef Y
+}
+
+long mct_dispersion_wave_target()
+{
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
+        return 0;
+    return 8L * cus;
 }
 
 int mct_launch_dispersion(const mct_dsp_args &a, hipStream_t s)
@@ -1236,9 +1342,16 @@ int mct_launch_dispersion(const mct_dsp_args &a, hipStream_t s)
             b.jobs = nullptr; b.dup = nullptr; b.njobs = nullptr;
             hipLaunchKernelGGL(k_dsp_queue_reset, dim3(1), dim3(64), 0, s, b.queue);
         }
+        // dsp_group_log() of the columns left after the duplicates: at most
+        // wave_target waves, or one lane per column
         long nw = (total + 63) / 64;
-        if (nw > b.lay_waves) nw = b.lay_waves;
-        hipLaunchKernelGGL(k_dispersion_sm, dim3((unsigned)nw), dim3(64), 0, s, b, b.lay, b.nz + 1, total);
+        if (nw < b.wave_target) nw = total < b.wave_target ? total : b.wave_target;
+        if (b.max_waves > 0 && nw > b.max_waves) nw = b.max_waves;
+        // the duplicates are known on the device only: of many columns the one that
+        // has no work returns at once
+        hipLaunchKernelGGL(k_dispersion_sm<true>, dim3((unsigned)nw), dim3(64), 0, s, b, b.lay, b.nz + 1, total);
+        if (dsp_group_log(total, b.wave_target) == 0)
+            hipLaunchKernelGGL(k_dispersion_sm<false>, dim3((unsigned)nw), dim3(64), 0, s, b, b.lay, b.nz + 1, total);
         if (b.dup) {
             MCT_CHECK(hipGetLastError());
             hipLaunchKernelGGL(k_dsp_dup_copy, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, b, total);
@@ -1439,7 +1552,7 @@ extern "C" int mct_dispersion_columns(int ncol, int nz, double dz, double scalin
         if (mode == 1 || mode == 3) a.lay = (float *)b[6];
         if (mode == 3) {
             a.queue = (unsigned long long *)b[7];
-            a.lay_waves = (ncol + 63) / 64;
+            a.wave_target = mct_dispersion_wave_target();
             a.jobs = (int32_t *)b[8]; a.keys = (int32_t *)b[9]; a.hist = (int32_t *)b[10];
             a.hlog = hlog; a.hkey = (unsigned long long *)b[11]; a.hrep = (int32_t *)b[12];
             a.dup = (int32_t *)b[13]; a.njobs = (int32_t *)b[14];

@@ -288,7 +288,9 @@ struct mct_dsp_args {
     float *lay;                   // lane-per-column scratch (mct_dispersion_lay_floats) or NULL
                                   // for one wave per column
     unsigned long long *queue;    // column queue counter: with lay, persistent waves
-    long lay_waves;               // waves the scratch holds (queue mode)
+    long wave_target;             // queue mode: up to this many waves share few columns
+                                  // (mct_dispersion_wave_target), 0: a lane per column
+    long max_waves;               // queue mode: at most this many waves, 0: no limit
     int32_t *jobs, *keys;         // queue mode: (nchain*ncol) columns ordered by layer count, or NULL
     int32_t *hist;                // (nz + 1) bins for that order
     // sorted queue mode, optional: columns whose Vs profiles are bit-identical
@@ -310,5 +312,7 @@ struct mct_dsp_args {
 // One wave per (column, chain): check_model, convert_to_layer, surfdisp96.
 // Requires np <= 60 and nz <= 100.
 int mct_launch_dispersion(const mct_dsp_args &a, hipStream_t s);
-// Floats of layer scratch the lane-per-column kernel needs.
+// The waves that a launch spreads few columns over, from the device's size.
+long mct_dispersion_wave_target();
+// Floats of layer scratch the lane-per-column and queue kernels need.
 long mct_dispersion_lay_floats(int ncol, int nz, int nchain);

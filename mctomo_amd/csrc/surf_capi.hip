@@ -87,7 +87,8 @@ struct mct_surf_ctx {
     mct_fm2d_args F;                 // geometry part of the 2-D solve
     long fm2d_chunk;
     int fm2d_method;                 // 0 parallel sweeps, 1 sequential heap loop
-    long dsp_waves;                  // queue mode: at most this many waves (0: one per 64 columns)
+    long dsp_waves;                  // queue mode: at most this many waves (0: no limit)
+    long dsp_wave_target;            // queue mode: waves that few columns are spread over
     long fm2d_run_chunk = 0;         // 2-D problems per launch (0: the workspace's capacity)
     // the batched call captured in HIP graphs, one per set of arguments (a
     // server lane replays one per batch size), oldest evicted beyond 64
@@ -192,10 +193,8 @@ static int surf_pipeline(mct_surf_ctx *C, int c0, int nchain, int part, int npar
     da.ndltar = C->ndltar.as<int32_t>() + (long)c0 * ncol;
     da.nlayer = C->nlayer.as<int32_t>() + (long)c0 * ncol;
     if (joint) { da.vp = na.vp; da.rho = na.rho; }
-    // many columns: one lane per column from a column queue (throughput); few:
-    // one wave per column (latency)
     int dmode = C->dsp_mode;
-    if (dmode == 0) dmode = (long)ncol * nchain >= 16384 ? 3 : 2;
+    if (dmode == 0) dmode = 3;
     if (d_box) {
         // a perturbed-box call (src/likelihood_surf.F90:155-170): the box's
         // columns are recomputed, the others keep the accepted phase velocities
@@ -211,8 +210,8 @@ static int surf_pipeline(mct_surf_ctx *C, int c0, int nchain, int part, int npar
     da.lay = (dmode == 1 || dmode == 3) ? C->lay.as<float>() + (long)c0 * wpc * 4 * (G.nz + 1) * 64 : nullptr;
     if (da.lay && dmode == 3) {
         da.queue = C->dsp_queue.as<unsigned long long>() + part;
-        da.lay_waves = (long)nchain * wpc;
-        if (C->dsp_waves > 0 && da.lay_waves > C->dsp_waves) da.lay_waves = C->dsp_waves;
+        da.wave_target = C->dsp_wave_target;
+        da.max_waves = C->dsp_waves;
         if (!C->dsp_unsorted || d_box) {
             da.jobs = C->dsp_jobs.as<int32_t>() + (long)c0 * ncol;
             da.keys = C->dsp_keys.as<int32_t>() + (long)c0 * ncol;
@@ -409,6 +408,7 @@ int mct_surf_create(const mct_grid *grid, const mct_surf_setup *setup, mct_surf_
         if (C->dsp_mode < 0 || C->dsp_mode > 3) C->dsp_mode = 0;
         const char *w = getenv("MCT_DSP_WAVES");
         C->dsp_waves = w ? atol(w) : 0;
+        C->dsp_wave_target = mct_dispersion_wave_target();
         const char *u = getenv("MCT_DSP_UNSORTED");     // columns in grid order (tuning)
         C->dsp_unsorted = u && atoi(u) != 0;
         const char *dd = getenv("MCT_DSP_DEDUP");       // 0: solve every column (tuning)

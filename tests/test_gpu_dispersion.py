@@ -176,3 +176,25 @@ def test_columns_under_a_water_layer(mode, water, iw, igr):
         nexact += same
     say("water columns", mode, water, iw, igr, "exact", nexact, "/", ncol, "bad_model", bad)
     assert nexact == ncol
+
+
+@pytest.mark.parametrize("ncol,iw,igr", [(1, 2, 1), (3, 1, 0), (2047, 1, 1), (2500, 2, 1), (5000, 1, 0), (9001, 2, 0),
+                                         (20001, 1, 1), (40003, 2, 1), (66000, 1, 0), (66000, 2, 1)])
+def test_lanes_per_column_by_size(ncol, iw, igr):
+    """The queue kernel gives a column 64 lanes where there are few columns, one
+    where there are many and each power of two between: the root search visits
+    other points ahead of time and uses the same ones, so the results are the
+    one-lane walk's bit for bit, with columns that have no root, searches that
+    start downwards and identical columns among them."""
+    rng = np.random.default_rng(ncol + 2 * iw + igr)
+    dz, nz = 0.8, 14
+    vs = np.repeat(rng.uniform(1.2, 4.8, (ncol, 5)), [3, 2, 4, 1, 4], axis=1)
+    vs[::2] = np.sort(vs[::2], axis=1)
+    vs[9::10] = vs[8:8 + vs[9::10].shape[0] * 10:10]
+    per = np.geomspace(0.6, 9, 6)
+    say("lanes per column", ncol, iw, igr)
+    want = mct.dispersion_columns(vs, dz, per, iw, igr, mode=1)
+    got = mct.dispersion_columns(vs, dz, per, iw, igr, mode=3)
+    for g, w in zip(got[:3], want[:3]):
+        np.testing.assert_array_equal(g, w)
+    assert got[3] == want[3]
