@@ -25,6 +25,7 @@
 // C library's numbers, which the reference's build uses) and sqrt and division
 // from the hardware's correctly rounded operations.
 #include "mct_internal.h"
+#include "fp64_ops.h"
 #include "libm_glibc.h"
 #include <float.h>
 #include <type_traits>
@@ -132,31 +133,45 @@ __device__ static float d_gtsolh(float a, float b)
     return c;
 }
 
+// Division, square root and the quotients of one denominator, y = dsp_rcp(d):
+// with NORM the operands are known to be far from the ends of the exponent range
+// (dsp_in_range) and fp64_ops.h's shorter forms give the same bits.
+template <bool NORM> __device__ __forceinline__ double dsp_rcp(double d) { return NORM ? fp_recip(d) : 0.0; }
+template <bool NORM> __device__ __forceinline__ double dsp_quot(double n, double d, double y)
+{
+    return NORM ? fp_quot(n, d, y) : n / d;
+}
+template <bool NORM> __device__ __forceinline__ double dsp_div(double n, double d)
+{
+    return NORM ? fp_div(n, d) : n / d;
+}
+template <bool NORM> __device__ __forceinline__ double dsp_sqrt(double x) { return NORM ? fp_sqrt(x) : sqrt(x); }
+
 // SH period equation, dltar1 (surfdisp96.f:1056-1115)
-template <class MD>
+template <bool NORM, class MD>
 __device__ static double d_dltar1(double wvno, double omega, const MD &M)
 {
     double beta1 = (double)M.b[M.st * (M.mmax - 1)];
     double rho1 = (double)M.rho[M.st * (M.mmax - 1)];
-    double xkb = omega / beta1;
+    double xkb = dsp_div<NORM>(omega, beta1);
     double wvnop = wvno + xkb;
     double wvnom = fabs(wvno - xkb);
-    double rb = sqrt(wvnop * wvnom);
+    double rb = dsp_sqrt<NORM>(wvnop * wvnom);
     double e1 = rho1 * rb;
-    double e2 = 1.0 / (beta1 * beta1);
+    double e2 = dsp_div<NORM>(1.0, beta1 * beta1);
     for (int m = M.mmax - 1; m >= M.llw; m--) {
         beta1 = (double)M.b[M.st * (m - 1)];
         rho1 = (double)M.rho[M.st * (m - 1)];
         double xmu = rho1 * beta1 * beta1;
-        xkb = omega / beta1;
+        xkb = dsp_div<NORM>(omega, beta1);
         wvnop = wvno + xkb;
         wvnom = fabs(wvno - xkb);
-        rb = sqrt(wvnop * wvnom);
+        rb = dsp_sqrt<NORM>(wvnop * wvnom);
         double q = (double)M.d[M.st * (m - 1)] * rb;
         double sinq, y, z, cosq;
         if (wvno < xkb) {
             mct_libm::libm_sincos(q, &sinq, &cosq);
-            y = sinq / rb;
+            y = dsp_div<NORM>(sinq, rb);
             z = -(rb * sinq);
         } else if (wvno == xkb) {
             cosq = 1.0;
@@ -167,37 +182,39 @@ __device__ static double d_dltar1(double wvno, double omega, const MD &M)
             if (q < 16) fac = mct_libm::libm_exp(-2.0 * q);
             cosq = (1.0 + fac) * 0.5;
             sinq = (1.0 - fac) * 0.5;
-            y = sinq / rb;
+            y = dsp_div<NORM>(sinq, rb);
             z = rb * sinq;
         }
         double e10 = e1 * cosq + e2 * xmu * z;
-        double e20 = e1 * y / xmu + e2 * cosq;
+        double e20 = dsp_div<NORM>(e1 * y, xmu) + e2 * cosq;
         double xnor = fabs(e10), ynor = fabs(e20);
         if (ynor > xnor) xnor = ynor;
         if (xnor < 1.0e-40) xnor = 1.0;
-        e1 = e10 / xnor;
-        e2 = e20 / xnor;
+        const double rnor = dsp_rcp<NORM>(xnor);
+        e1 = dsp_quot<NORM>(e10, xnor, rnor);
+        e2 = dsp_quot<NORM>(e20, xnor, rnor);
     }
     return e1;
 }
 
 // P-SV period equation, dltar4 with var and dnka inlined (surfdisp96.f:1119-1414)
-template <class MD>
+template <bool NORM, class MD>
 __device__ static double d_dltar4(double wvno, double omga, const MD &M)
 {
     double omega = omga;
     if (omega < 1.0e-4) omega = 1.0e-4;
     const double one = 1.0, two = 2.0;
+    const double romega = dsp_rcp<NORM>(omega);
     double wvno2 = wvno * wvno;
     int mm = M.mmax - 1;
-    double xka = omega / (double)M.a[M.st * (mm)];
-    double xkb = omega / (double)M.b[M.st * (mm)];
+    double xka = dsp_div<NORM>(omega, (double)M.a[M.st * (mm)]);
+    double xkb = dsp_div<NORM>(omega, (double)M.b[M.st * (mm)]);
     double wvnop = wvno + xka, wvnom = fabs(wvno - xka);
-    double ra = sqrt(wvnop * wvnom);
+    double ra = dsp_sqrt<NORM>(wvnop * wvnom);
     wvnop = wvno + xkb;
     wvnom = fabs(wvno - xkb);
-    double rb = sqrt(wvnop * wvnom);
-    double t = (double)M.b[M.st * (mm)] / omega;
+    double rb = dsp_sqrt<NORM>(wvnop * wvnom);
+    double t = dsp_quot<NORM>((double)M.b[M.st * (mm)], omega, romega);
     double gammk = 2.0 * t * t;
     double gam = gammk * wvno2;
     double gamm1 = gam - 1.0;
@@ -209,17 +226,17 @@ __device__ static double d_dltar4(double wvno, double omga, const MD &M)
     double e4 = wvno2 - ra * rb;
     for (int m = M.mmax - 1; m >= M.llw; m--) {
         int i0 = m - 1;
-        xka = omega / (double)M.a[M.st * (i0)];
-        xkb = omega / (double)M.b[M.st * (i0)];
-        t = (double)M.b[M.st * (i0)] / omega;
+        xka = dsp_div<NORM>(omega, (double)M.a[M.st * (i0)]);
+        xkb = dsp_div<NORM>(omega, (double)M.b[M.st * (i0)]);
+        t = dsp_quot<NORM>((double)M.b[M.st * (i0)], omega, romega);
         gammk = 2.0 * t * t;
         gam = gammk * wvno2;
         wvnop = wvno + xka;
         wvnom = fabs(wvno - xka);
-        ra = sqrt(wvnop * wvnom);
+        ra = dsp_sqrt<NORM>(wvnop * wvnom);
         wvnop = wvno + xkb;
         wvnom = fabs(wvno - xkb);
-        rb = sqrt(wvnop * wvnom);
+        rb = dsp_sqrt<NORM>(wvnop * wvnom);
         double dpth = (double)M.d[M.st * (i0)];
         rho1 = (double)M.rho[M.st * (i0)];
         double p = ra * dpth, q = rb * dpth;
@@ -227,7 +244,7 @@ __device__ static double d_dltar4(double wvno, double omga, const MD &M)
         double pex = 0.0, sex = 0.0, sinp, w = 0, x = 0, cosp = 0, sinq, y = 0, z = 0, cosq = 0;
         if (wvno < xka) {
             mct_libm::libm_sincos(p, &sinp, &cosp);
-            w = sinp / ra;
+            w = dsp_div<NORM>(sinp, ra);
             x = -(ra * sinp);
         } else if (wvno == xka) {
             cosp = 1.0;
@@ -239,12 +256,12 @@ __device__ static double d_dltar4(double wvno, double omga, const MD &M)
             if (p < 16) fac = mct_libm::libm_exp(-2.0 * p);
             cosp = (1.0 + fac) * 0.5;
             sinp = (1.0 - fac) * 0.5;
-            w = sinp / ra;
+            w = dsp_div<NORM>(sinp, ra);
             x = ra * sinp;
         }
         if (wvno < xkb) {
             mct_libm::libm_sincos(q, &sinq, &cosq);
-            y = sinq / rb;
+            y = dsp_div<NORM>(sinq, rb);
             z = -(rb * sinq);
         } else if (wvno == xkb) {
             cosq = 1.0;
@@ -256,7 +273,7 @@ __device__ static double d_dltar4(double wvno, double omga, const MD &M)
             if (q < 16) fac = mct_libm::libm_exp(-2.0 * q);
             cosq = (1.0 + fac) * 0.5;
             sinq = (1.0 - fac) * 0.5;
-            y = sinq / rb;
+            y = dsp_div<NORM>(sinq, rb);
             z = rb * sinq;
         }
         double exa = pex + sex;
@@ -273,10 +290,11 @@ __device__ static double d_dltar4(double wvno, double omga, const MD &M)
         double rho2 = rho1 * rho1;
         double a0pq = a0 - cpcq;
         double c11 = cpcq - two * gmgm1 * a0pq - gmgmk * xz - wvno2 * gm1sq * wy;
-        double c12 = (wvno2 * cpy - cqx) / rho1;
-        double c13 = -((twgm1 * a0pq + gammk * xz + wvno2 * g1 * wy) / rho1);
-        double c14 = (cpz - wvno2 * cqw) / rho1;
-        double c15 = -((two * wvno2 * a0pq + xz + wvno2 * wvno2 * wy) / rho2);
+        const double rrho1 = dsp_rcp<NORM>(rho1);
+        double c12 = dsp_quot<NORM>(wvno2 * cpy - cqx, rho1, rrho1);
+        double c13 = -dsp_quot<NORM>(twgm1 * a0pq + gammk * xz + wvno2 * g1 * wy, rho1, rrho1);
+        double c14 = dsp_quot<NORM>(cpz - wvno2 * cqw, rho1, rrho1);
+        double c15 = -dsp_div<NORM>(two * wvno2 * a0pq + xz + wvno2 * wvno2 * wy, rho2);
         double c21 = (gmgmk * cpz - gm1sq * cqw) * rho1;
         double c22 = cpcq;
         double c23 = gammk * cpz - g1 * cqw;
@@ -313,24 +331,29 @@ __device__ static double d_dltar4(double wvno, double omga, const MD &M)
         if (fabs(ee3) > t1) t1 = fabs(ee3);
         if (fabs(ee4) > t1) t1 = fabs(ee4);
         if (t1 < 1.0e-40) t1 = 1.0;
-        e0 = ee0 / t1; e1 = ee1 / t1; e2 = ee2 / t1; e3 = ee3 / t1; e4 = ee4 / t1;
+        const double rt1 = dsp_rcp<NORM>(t1);
+        e0 = dsp_quot<NORM>(ee0, t1, rt1);
+        e1 = dsp_quot<NORM>(ee1, t1, rt1);
+        e2 = dsp_quot<NORM>(ee2, t1, rt1);
+        e3 = dsp_quot<NORM>(ee3, t1, rt1);
+        e4 = dsp_quot<NORM>(ee4, t1, rt1);
     }
     if (M.llw != 1) {   // water layer on top
-        xka = omega / (double)M.a[M.st * (0)];
+        xka = dsp_div<NORM>(omega, (double)M.a[M.st * (0)]);
         wvnop = wvno + xka;
         wvnom = fabs(wvno - xka);
-        ra = sqrt(wvnop * wvnom);
+        ra = dsp_sqrt<NORM>(wvnop * wvnom);
         double dpth = (double)M.d[M.st * (0)];
         rho1 = (double)M.rho[M.st * (0)];
         double p = ra * dpth;
         double w = 0, cosp = 0;
-        if (wvno < xka) { double sp; mct_libm::libm_sincos(p, &sp, &cosp); w = sp / ra; }
+        if (wvno < xka) { double sp; mct_libm::libm_sincos(p, &sp, &cosp); w = dsp_div<NORM>(sp, ra); }
         else if (wvno == xka) { cosp = 1.0; w = dpth; }
         else {
             double fac = 0.0;
             if (p < 16) fac = mct_libm::libm_exp(-2.0 * p);
             cosp = (1.0 + fac) * 0.5;
-            w = ((1.0 - fac) * 0.5) / ra;
+            w = dsp_div<NORM>((1.0 - fac) * 0.5, ra);
         }
         double w0 = -(rho1 * w);
         return cosp * e0 + w0 * e1;
@@ -338,10 +361,10 @@ __device__ static double d_dltar4(double wvno, double omga, const MD &M)
     return e0;
 }
 
-template <class MD>
+template <bool NORM = false, class MD>
 __device__ __forceinline__ double d_dltar(double wvno, double omega, int ifunc, const MD &M)
 {
-    return ifunc == 1 ? d_dltar1(wvno, omega, M) : d_dltar4(wvno, omega, M);
+    return ifunc == 1 ? d_dltar1<NORM>(wvno, omega, M) : d_dltar4<NORM>(wvno, omega, M);
 }
 
 // nevill (surfdisp96.f:903-1020), run identically by every lane of the wave
@@ -738,8 +761,13 @@ __global__ __launch_bounds__(64) void k_dispersion_lane(mct_dsp_args A, float *l
 // one (42 walk, 9 nevill), 17 rounds with 4 lanes, 10 with 8 and 7 with 16.
 // What bounds few columns is that chain: a column has about 1000 evaluations of
 // 2000 instructions, one after the other, whatever the number of lanes that idle.
-// 201x201 columns (30,000 different): 16.1 -> 6.2 ms; the perturbed boxes of a
-// 101x101 group-velocity grid: 17.5 -> 1.5 ms.
+// 201x201 columns (30,000 different): 16.1 -> 5.4 ms; the perturbed boxes of a
+// 101x101 group-velocity grid: 17.5 -> 1.4 ms.
+//
+// Many columns are bound by the FP64 instructions, which 3 waves per SIMD issue at
+// 79 % of the time and 2 at 70 %: hence the search's state in LDS, one kernel per
+// wave type, and the shorter quotients and sines.  1.4 million different columns of
+// 48 chains, Rayleigh: 91 -> 78 ms; 410,000 columns, Love group: 40 -> 34.7 ms.
 enum {
     SM_NEXT, SM_PERIOD, SM_G0, SM_G1, SM_N0, SM_NLOOP, SM_N1, SM_NBODY, SM_N2, SM_N3,
     SM_NDONE, SM_GDONE, SM_FINISH, SM_DONE
@@ -952,11 +980,16 @@ __global__ void k_dsp_queue_reset(unsigned long long *q)
     if (threadIdx.x == 0) q[0] = 0ull;
 }
 
+// 2^-40 <= x <= 2^40.  Layers, periods and trial velocities in this range keep the
+// period equations' quotients and square roots within 2^-700..2^700 (or at 0).
+template <class T> __device__ __forceinline__ bool dsp_in_range(T x) { return x >= (T)0x1p-40 && x <= (T)0x1p40; }
+
 // Lanes per column, as a power of two: as many as keep the columns' waves within
-// wave_target (0: one lane per column), which is what the device holds at once
-// (2 waves per SIMD at this kernel's registers): beyond it each further lane only
-// adds evaluations that may not be used, 1.3 times the work with 4 lanes and 2.2
-// times with 16.  48 chains of 201x201 columns stay with one lane (91 ms).
+// wave_target (0: one lane per column), 16 per CU where 12 are resident at once:
+// with fewer lanes the chain of evaluations bounds the call, with more the
+// evaluations that are not used (1.3 times the work with 4 lanes, 2.2 times with
+// 16).  201x201 columns (30,000 different, 8 lanes): 5.4 ms, with 8 or 12 waves per
+// CU as the line (4 lanes) 6.1 ms.
 __host__ __device__ __forceinline__ int dsp_group_log(long ncolumns, long wave_target)
 {
     int lg = 0;
@@ -964,8 +997,8 @@ __host__ __device__ __forceinline__ int dsp_group_log(long ncolumns, long wave_t
     return lg;
 }
 
-template <bool GROUPED>
-__global__ __launch_bounds__(64) void k_dispersion_sm(mct_dsp_args A, float *lay, int nlmax, long total)
+template <bool GROUPED, int IFUNC>
+__global__ __launch_bounds__(64, 3) void k_dispersion_sm(mct_dsp_args A, float *lay, int nlmax, long total)
 {
     const int lane = threadIdx.x;
     const long ntot = A.njobs ? (long)A.njobs[0] : total;   // duplicates are not queued
@@ -982,7 +1015,6 @@ __global__ __launch_bounds__(64) void k_dispersion_sm(mct_dsp_args A, float *lay
     const float ddc = (float)A.dphase;
     const double one = 1.0e-2, onea = (double)sone;
     const double dc = fabs((double)ddc);
-    const int ifunc = A.iwave;
 
     typename std::conditional<GROUPED, dsp_model_rt, dsp_model_t<64>>::type M;
     if constexpr (GROUPED) M.st = ncw;
@@ -993,24 +1025,25 @@ __global__ __launch_bounds__(64) void k_dispersion_sm(mct_dsp_args A, float *lay
     long job = -1;
     int c = 0;
     long col = 0;
-    double *cp = nullptr, *cg = nullptr;
     int ierr = 0, ndl = 0, k = 1, pass = 0, ifirst = 0;
-    float betmx = 0.0f;
-    double cc = 0.0, cm = 0.0, cmax = 0.0, cprev = 0.0, del1st = 0.0, croot = 0.0;
-    float t1a = 0.0f, t1b = 0.0f;
-    double t1 = 0.0, omega = 0.0;
+    // The search's state lies in LDS, a row of 64 lanes each: it is touched between
+    // evaluations only, and in registers it would cost a wave per SIMD.
+    __shared__ double rows[18 * 64];
+    double &cc = rows[lane], &cm = rows[64 + lane], &cmax = rows[2 * 64 + lane], &cprev = rows[3 * 64 + lane];
+    double &del1st = rows[4 * 64 + lane], &croot = rows[5 * 64 + lane], &t1 = rows[6 * 64 + lane];
     // getsol / nevill state
-    double c1 = 0.0, del1 = 0.0, clow = 0.0;
+    double &c1 = rows[7 * 64 + lane], &del1 = rows[8 * 64 + lane], &clow = rows[9 * 64 + lane];
+    double &gc = rows[10 * 64 + lane], &nc1 = rows[11 * 64 + lane], &nc2 = rows[12 * 64 + lane];
+    double &nd1 = rows[13 * 64 + lane], &nd2 = rows[14 * 64 + lane], &c3 = rows[15 * 64 + lane];
+    double &del3 = rows[16 * 64 + lane];
+    double &cprv = rows[17 * 64 + lane];    // the lane's own step of the walk: from cprv to ceval
+    float betmx = 0.0f, t1a = 0.0f, t1b = 0.0f;
+    double omega = 0.0;
     int idir = 1, gret = 0, walk = 0;
-    double gc = 0.0;
-    double nc1 = 0.0, nc2 = 0.0, nd1 = 0.0, nd2 = 0.0, c3 = 0.0, del3 = 0.0;
     int nev = 0, nctrl = 0, m = 1;
-    double cprv = 0.0;                 // the lane's own step of the walk: from cprv to ceval
     int dd = 1, skip = 0, node = 0, hi = 0;
-    // Neville tables in LDS, lane-interleaved
-    __shared__ double xs[12 * 64], ys[12 * 64];
-#define X(j) xs[(j) * 64 + lane]
-#define Y(j) ys[(j) * 64 + lane]
+    bool norm = false;                 // the column's layers are dsp_in_range
+    double XY[32];                // Neville tables: two or three entries as a rule
     double res = 0.0, ceval = 0.0;
     int pc = SM_NEXT;
     // getsol's walk from c1: the lane's step is the (sub + 1 - skip)th
@@ -1060,14 +1093,16 @@ __global__ __launch_bounds__(64) void k_dispersion_sm(mct_dsp_args A, float *lay
                 if (below) A.bad_model[c] = 1;
                 M.mmax = dsp_convert(A, cb, vs, sd, sa, sb, sr, ncw);
                 M.llw = (sb[0] <= 0.0f) ? 2 : 1;
-                cp = A.phase + ((long)c * A.ncol + col) * A.np;
-                cg = A.group + ((long)c * A.ncol + col) * A.np;
                 ierr = 0; ndl = 0;
                 int jmn = 1, jsol = 1;
                 betmx = -1.e20f;
                 float betmn = 1.e20f;
+                norm = true;
                 for (int ii = 1; ii <= M.mmax; ii++) {
                     float bi = sb[ncw * (ii - 1)], ai = sa[ncw * (ii - 1)];
+                    norm &= dsp_in_range(ai) && dsp_in_range(sr[ncw * (ii - 1)]) &&
+                            (dsp_in_range(bi) || ii < M.llw) &&
+                            (dsp_in_range(sd[ncw * (ii - 1)]) || sd[ncw * (ii - 1)] == 0.0f);
                     if (bi > 0.01f && bi < betmn) { betmn = bi; jmn = ii; jsol = 1; }
                     else if (bi <= 0.01f && ai < betmn) { betmn = ai; jmn = ii; jsol = 0; }
                     if (bi > betmx) betmx = bi;
@@ -1179,22 +1214,22 @@ __global__ __launch_bounds__(64) void k_dispersion_sm(mct_dsp_args A, float *lay
                 bool halve = s1 > ss2 || s2 > ss1 || nev == 0;
                 if (!halve) {
                     if (nev == 2) {
-                        X(m + 1) = c3;
-                        Y(m + 1) = del3;
+                        XY[2 * (m + 1)] = c3;
+                        XY[2 * (m + 1) + 1] = del3;
                     } else {
-                        X(1) = nc1; Y(1) = nd1;
-                        X(2) = nc2; Y(2) = nd2;
+                        XY[2 * (1)] = nc1; XY[2 * (1) + 1] = nd1;
+                        XY[2 * (2)] = nc2; XY[2 * (2) + 1] = nd2;
                         m = 1;
                     }
                     bool bad = false;
                     for (int kk = 1; kk <= m; kk++) {
                         int j = m - kk + 1;
-                        double denom = Y(m + 1) - Y(j);
-                        if (fabs(denom) < 1.0e-10 * fabs(Y(m + 1))) { bad = true; break; }
-                        X(j) = (-(Y(j) * X(j + 1)) + Y(m + 1) * X(j)) / denom;
+                        double denom = XY[2 * (m + 1) + 1] - XY[2 * (j) + 1];
+                        if (fabs(denom) < 1.0e-10 * fabs(XY[2 * (m + 1) + 1])) { bad = true; break; }
+                        XY[2 * (j)] = (-(XY[2 * (j) + 1] * XY[2 * (j + 1)]) + XY[2 * (m + 1) + 1] * XY[2 * (j)]) / denom;
                     }
                     if (!bad) {
-                        c3 = X(1);
+                        c3 = XY[2 * (1)];
                         halving_points();
                         need = true; pc = SM_N2;
                         break;
@@ -1231,7 +1266,9 @@ __global__ __launch_bounds__(64) void k_dispersion_sm(mct_dsp_args A, float *lay
                 gret = (c3 > (double)betmx) ? -1 : 1;
                 pc = SM_GDONE;
                 break;
-            case SM_GDONE:
+            case SM_GDONE: {
+                double *cp = A.phase + ((long)c * A.ncol + col) * A.np;
+                double *cg = A.group + ((long)c * A.ncol + col) * A.np;
                 if (pass == 0) {
                     if (gret == -1) {
                         // no root at period k: the rest keep cp=100, cg=0 (labels 1700/1750)
@@ -1273,6 +1310,7 @@ __global__ __launch_bounds__(64) void k_dispersion_sm(mct_dsp_args A, float *lay
                 k++;
                 pc = k > A.np ? SM_FINISH : SM_PERIOD;
                 break;
+            }
             case SM_FINISH:
                 if (sub == 0) {
                     A.ierr[(long)c * A.ncol + col] = ierr;
@@ -1287,10 +1325,12 @@ __global__ __launch_bounds__(64) void k_dispersion_sm(mct_dsp_args A, float *lay
             }
         }
         if (__builtin_amdgcn_ballot_w64(need) == 0ull) break;     // every lane has run out of columns
-        if (need) res = d_dltar(omega / ceval, omega, ifunc, M);
+        if (need) {
+            const double wvno = omega / ceval;
+            if (norm && dsp_in_range(ceval) && dsp_in_range(omega)) res = d_dltar<true>(wvno, omega, IFUNC, M);
+            else res = d_dltar(wvno, omega, IFUNC, M);
+        }
     }
-#undef X
-#undef Y
 }
 
 long mct_dispersion_wave_target()
@@ -1299,7 +1339,7 @@ long mct_dispersion_wave_target()
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
         return 0;
-    return 8L * cus;
+    return 16L * cus;
 }
 
 int mct_launch_dispersion(const mct_dsp_args &a, hipStream_t s)
@@ -1349,9 +1389,11 @@ int mct_launch_dispersion(const mct_dsp_args &a, hipStream_t s)
         if (b.max_waves > 0 && nw > b.max_waves) nw = b.max_waves;
         // the duplicates are known on the device only: of many columns the one that
         // has no work returns at once
-        hipLaunchKernelGGL(k_dispersion_sm<true>, dim3((unsigned)nw), dim3(64), 0, s, b, b.lay, b.nz + 1, total);
+        auto *few = b.iwave == 1 ? k_dispersion_sm<true, 1> : k_dispersion_sm<true, 2>;
+        auto *many = b.iwave == 1 ? k_dispersion_sm<false, 1> : k_dispersion_sm<false, 2>;
+        hipLaunchKernelGGL(few, dim3((unsigned)nw), dim3(64), 0, s, b, b.lay, b.nz + 1, total);
         if (dsp_group_log(total, b.wave_target) == 0)
-            hipLaunchKernelGGL(k_dispersion_sm<false>, dim3((unsigned)nw), dim3(64), 0, s, b, b.lay, b.nz + 1, total);
+            hipLaunchKernelGGL(many, dim3((unsigned)nw), dim3(64), 0, s, b, b.lay, b.nz + 1, total);
         if (b.dup) {
             MCT_CHECK(hipGetLastError());
             hipLaunchKernelGGL(k_dsp_dup_copy, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, b, total);

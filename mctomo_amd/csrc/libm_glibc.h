@@ -113,70 +113,69 @@ __host__ __device__ __forceinline__ double lm_copysign(double a, double s)
 }
 __host__ __device__ __forceinline__ double lm_fabs(double a) { return lm_dbl(lm_bits(a) & 0x7fffffffffffffffull); }
 
-// sin(a + da), |a| < 0.855
-__host__ __device__ __forceinline__ double lm_do_sin(double x, double dx)
+// sin(x + dx) and cos(x + dx), |x| < 0.855
+__host__ __device__ __forceinline__ void lm_do_sincos(double x, double dx, double *sinx, double *cosx)
 {
-    const double xold = x;
+    const double dxs = dx, u = lm_sc::big + lm_fabs(x);
+    const double r = lm_fabs(x) - (u - lm_sc::big);
+    const int k = (int)(uint32_t)lm_bits(u) << 2;
+    const double sn = LIBM_SC_TAB[k], ssn = LIBM_SC_TAB[k + 1], cs = LIBM_SC_TAB[k + 2], ccs = LIBM_SC_TAB[k + 3];
+    if (x < 0) dx = -dx;
+    {
+        const double y = r + dx;
+        const double yy = y * y;
+        const double s = y + y * yy * (lm_sc::sn3 + yy * lm_sc::sn5);
+        const double c = yy * (lm_sc::cs2 + yy * (lm_sc::cs4 + yy * lm_sc::cs6));
+        const double cor = (ccs - s * ssn - cs * c) - sn * s;
+        *cosx = cs + cor;
+    }
     if (lm_fabs(x) < 0.126) {
         const double xx = x * x;
         const double p = ((((lm_sc::s5 * xx + lm_sc::s4) * xx + lm_sc::s3) * xx + lm_sc::s2) * xx) + lm_sc::s1;
-        const double t = ((p * x - 0.5 * dx) * xx + dx);
-        return x + t;
+        const double t = ((p * x - 0.5 * dxs) * xx + dxs);
+        *sinx = x + t;
+    } else {
+        const double xx = r * r;
+        const double s = r + (dx + r * xx * (lm_sc::sn3 + xx * lm_sc::sn5));
+        const double c = r * dx + xx * (lm_sc::cs2 + xx * (lm_sc::cs4 + xx * lm_sc::cs6));
+        const double cor = (ssn + s * ccs - sn * c) + cs * s;
+        *sinx = lm_copysign(sn + cor, x);
     }
-    if (x <= 0) dx = -dx;
-    const double u = lm_sc::big + lm_fabs(x);
-    x = lm_fabs(x) - (u - lm_sc::big);
-    const double xx = x * x;
-    const double s = x + (dx + x * xx * (lm_sc::sn3 + xx * lm_sc::sn5));
-    const double c = x * dx + xx * (lm_sc::cs2 + xx * (lm_sc::cs4 + xx * lm_sc::cs6));
-    const int k = (int)(uint32_t)lm_bits(u) << 2;
-    const double sn = LIBM_SC_TAB[k], ssn = LIBM_SC_TAB[k + 1], cs = LIBM_SC_TAB[k + 2], ccs = LIBM_SC_TAB[k + 3];
-    const double cor = (ssn + s * ccs - sn * c) + cs * s;
-    return lm_copysign(sn + cor, xold);
 }
 
-// cos(a + da), |a| < 0.855
-__host__ __device__ __forceinline__ double lm_do_cos(double x, double dx)
-{
-    if (x < 0) dx = -dx;
-    const double u = lm_sc::big + lm_fabs(x);
-    x = lm_fabs(x) - (u - lm_sc::big) + dx;
-    const double xx = x * x;
-    const double s = x + x * xx * (lm_sc::sn3 + xx * lm_sc::sn5);
-    const double c = xx * (lm_sc::cs2 + xx * (lm_sc::cs4 + xx * lm_sc::cs6));
-    const int k = (int)(uint32_t)lm_bits(u) << 2;
-    const double sn = LIBM_SC_TAB[k], ssn = LIBM_SC_TAB[k + 1], cs = LIBM_SC_TAB[k + 2], ccs = LIBM_SC_TAB[k + 3];
-    const double cor = (ccs - s * ssn - cs * c) - sn * s;
-    return cs + cor;
-}
-
-// sin(x) and cos(x) for |x| < 105414350 (larger |x| is not reduced: NaN).
+// sin(x) and cos(x) for |x| < 105414350 (larger |x| is not reduced: NaN).  The
+// argument is brought to (a, da) with |a| < 0.855 by the range's own rule, chosen
+// by selects: a wave whose lanes lie in different ranges runs the polynomials once
+// instead of once per range (281 -> 172 instructions).
 __host__ __device__ __forceinline__ void libm_sincos(double x, double *sinx, double *cosx)
 {
     const uint32_t k = (uint32_t)(lm_bits(x) >> 32) & 0x7fffffffu;
-    if (k < 0x400368fdu) {
-        if (k < 0x3e400000u) { *sinx = x; *cosx = 1.0; return; }
-        if (k < 0x3feb6000u) { *sinx = lm_do_sin(x, 0); *cosx = lm_do_cos(x, 0); return; }
-        const double y = lm_sc::hp0 - lm_fabs(x), a = y + lm_sc::hp1, da = (y - a) + lm_sc::hp1;
-        *sinx = lm_copysign(lm_do_cos(a, da), x);
-        *cosx = lm_do_sin(a, da);
-        return;
-    }
-    if (k >= 0x419921fbu) { *sinx = *cosx = __builtin_nan(""); return; }
     // pi/2 in four parts; the quadrant from the low bits of the shifted multiple
     const double t = (x * lm_sc::hpinv + lm_sc::toint);
     const double xn = t - lm_sc::toint;
     const double y = (x - xn * lm_sc::mp1) - xn * lm_sc::mp2;
-    const unsigned n = (unsigned)lm_bits(t) & 3u;
+    unsigned n = (unsigned)lm_bits(t) & 3u;
     double t1 = xn * lm_sc::pp3, t2 = y - t1;
-    double db = (y - t2) - t1;
+    double da = (y - t2) - t1;
     t1 = xn * lm_sc::pp4;
     double a = t2 - t1;
-    db += (t2 - a) - t1;
-    if (n == 1 || n == 2) { a = -a; db = -db; }
-    const double s = lm_do_sin(a, db), c = lm_do_cos(a, db);
-    if (n & 1) { *cosx = s; *sinx = (n & 2) ? -c : c; }
-    else { *sinx = s; *cosx = (n & 2) ? -c : c; }
+    da += (t2 - a) - t1;
+    if (n == 1 || n == 2) { a = -a; da = -da; }
+    if (k < 0x400368fdu) {              // |x| < 2.426: pi/2 - |x|, the quadrant by x's sign
+        const double h = lm_sc::hp0 - lm_fabs(x);
+        a = h + lm_sc::hp1;
+        da = (h - a) + lm_sc::hp1;
+        n = x < 0 ? 3 : 1;
+    }
+    if (k < 0x3feb6000u) { a = x; da = 0; n = 0; }      // |x| < 0.855
+    if (k >= 0x419921fbu) a = 0;
+    double s, c;
+    lm_do_sincos(a, da, &s, &c);
+    if (k >= 0x419921fbu) { s = c = __builtin_nan(""); n = 0; }
+    if (k < 0x3e400000u) { s = x; c = 1.0; }            // |x| < 2^-27
+    const double o = (n & 2) ? -c : c;
+    *sinx = (n & 1) ? o : s;
+    *cosx = (n & 1) ? s : o;
 }
 
 }   // namespace mct_libm

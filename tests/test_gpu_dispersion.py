@@ -198,3 +198,19 @@ def test_lanes_per_column_by_size(ncol, iw, igr):
     for g, w in zip(got[:3], want[:3]):
         np.testing.assert_array_equal(g, w)
     assert got[3] == want[3]
+
+
+@pytest.mark.parametrize("dz,pmin", [(1e-13, 0.6), (2e12, 0.6), (0.8, 1e-13)])
+@pytest.mark.parametrize("iw,igr", [(2, 0), (1, 1)])
+def test_columns_outside_the_short_forms_range(dz, pmin, iw, igr):
+    """Layer thicknesses and periods beyond 2^+-40, where the queue kernel leaves the
+    short quotients and square roots for the compiler's: the lane kernel's results,
+    which has no other, bit for bit."""
+    rng = np.random.default_rng(77 + iw)
+    vs = np.sort(np.repeat(rng.uniform(1.2, 4.8, (130, 3)), [3, 2, 4], axis=1), axis=1)
+    per = np.r_[0.6 if pmin > 0.1 else pmin, 2.0, 9.0]
+    say("columns out of range", dz, pmin, iw, igr)
+    want = mct.dispersion_columns(vs, dz, per, iw, igr, mode=1)
+    got = mct.dispersion_columns(vs, dz, per, iw, igr, mode=3)
+    for g, w in zip(got[:3], want[:3]):
+        np.testing.assert_array_equal(g, w)
