@@ -16,6 +16,7 @@
 // The coarse B-spline velocity of a period is computed once by a separate
 // kernel (one thread per node) and shared by all sources of that period.
 #include "mct_internal.h"
+#include "fm2d_wave.h"
 #include <stdlib.h>
 #include <string.h>
 
@@ -682,14 +683,6 @@ struct wave_grid {
     bool lead;              // this lane is it
 };
 
-// Lanes of one wave read what others of it wrote: keep the accesses in order.
-__device__ __forceinline__ void w_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // the group's bits of a ballot
 template <int GL>
 __device__ __forceinline__ unsigned long long w_ballot(const wave_grid &G, bool p)
@@ -731,16 +724,6 @@ __device__ __forceinline__ double w_bcast_d(double v)
     const int lo = w_bcast<GL, SRC>((int)b), hi = w_bcast<GL, SRC>((int)(b >> 32));
     return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
-// the value of the lane whose index differs in bit 0 (0xb1) or bit 1 (0x4e)
-template <int CTRL>
-__device__ __forceinline__ double w_quad_d(double v)
-{
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_update_dpp((int)b, (int)b, CTRL, 0xf, 0xf, false);
-    const int hi = __builtin_amdgcn_update_dpp((int)(b >> 32), (int)(b >> 32), CTRL, 0xf, 0xf, false);
-    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-}
-
 // A heap entry names its node as (ix << 16) | iz (ET = int32_t), or, where the
 // slot's arrays hold fewer than 65,536 words, as the node's offset in them
 // (ET = uint16_t: half the LDS, so more problems fit on a CU).
@@ -770,8 +753,6 @@ __device__ __forceinline__ void w_setpos(const wave_grid &G, int e, int pos)
     if (sizeof(ET) == 2) G.s[e] = pos;
     else LS(G, BPZ(e), BPX(e)) = pos;
 }
-__device__ __forceinline__ int w_level(int p) { return 31 - __clz(p); }
-
 // A lane's place in a downtree block: the node `off` of level `lv` under the
 // hole (its index in the block is 2^lv - 2 + off, so siblings are lanes i, i^1),
 // and the bits of itself and its ancestors in the block.
@@ -874,67 +855,6 @@ __device__ __forceinline__ int w_downtree(wave_grid &G, int gl, const w_block<GL
     }
     w_sync();
     return hole;
-}
-
-// One quadrant of fouds1 (fm2d_ttime.f90:248-332) or fouds2 (:342-518): tj, tk the
-// x and z neighbours' times, tj2, tk2 the ones behind them, a* whether alive.
-// Returns W_NONE when neither neighbour is alive.
-#define W_NONE 1e300
-template <int FOM>
-__device__ __forceinline__ double w_quadrant(bool aj, bool aj2, bool ak, bool ak2, double tj, double tj2, double tk,
-                                             double tk2, double slown, double dnx, double dnz)
-{
-    const bool J = FOM != 0 && aj && aj2 && tj > tj2, K = FOM != 0 && ak && ak2 && tk > tk2;
-    const double ss = slown * slown, xx = dnx * dnx, zz = dnz * dnz;
-    double a = 1.0, b = 0.0, c, tref, tdiv = 1.0;
-    if (aj && ak) {
-        double uu, vv, em;
-        if (J && K) {
-            uu = 4.0 * xx; vv = 4.0 * zz;
-            tref = 4.0 * tj - tj2;
-            em = tref - 4.0 * tk;
-            em = em + tk2;
-            a = vv + uu;
-            b = 2.0 * em * uu;
-            tdiv = 3.0;
-        } else if (J) {
-            uu = zz; vv = 4.0 * xx;
-            em = 3.0 * tk - 4.0 * tj + tj2;
-            a = vv + 9.0 * uu;
-            b = 6.0 * em * uu;
-            tref = tk;
-        } else if (K) {
-            uu = xx; vv = 4.0 * zz;
-            em = 3.0 * tj - 4.0 * tk + tk2;
-            a = vv + 9.0 * uu;
-            b = 6.0 * em * uu;
-            tref = tj;
-        } else {
-            uu = xx; vv = zz;
-            em = tk - tj;
-            a = uu + vv;
-            b = -(2.0 * uu * em);
-            tref = tj;
-        }
-        c = uu * (em * em - vv * ss);
-    } else if (aj) {
-        c = -((J ? 4.0 * xx : xx) * ss);
-        tref = J ? 4.0 * tj - tj2 : tj;
-        tdiv = J ? 3.0 : 1.0;
-    } else if (ak) {
-        // fouds1 squares slown * dnz as one product, fouds2 the squares of each
-        const double sz = slown * dnz;
-        c = FOM == 0 ? -(sz * sz) : -((K ? 4.0 * zz : zz) * ss);
-        tref = K ? 4.0 * tk - tk2 : tk;
-        tdiv = K ? 3.0 : 1.0;
-    } else {
-        return W_NONE;
-    }
-    double rd1 = b * b - 4.0 * a * c;
-    if (rd1 < 0.0) rd1 = 0.0;
-    const double tdsh = (-b + sqrt(rd1)) / (2.0 * a);
-    const double trav = tref + tdsh;
-    return FOM == 0 ? trav : trav / tdiv;
 }
 
 // travel (fm2d_ttime.f90:41-238) on a group; -1 source outside, -2 heap full.

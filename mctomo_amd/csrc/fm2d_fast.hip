@@ -33,6 +33,7 @@
 // A problem whose heap loop would leave the LDS neighbourhood is flagged and
 // solved by the sequential kernel instead.
 #include "mct_internal.h"
+#include "fm2d_wave.h"
 #include "fp64_ops.h"
 #include <string.h>
 #include <stdlib.h>
@@ -749,9 +750,8 @@ __device__ __forceinline__ int ff_sweep(const fview &V, const FX &fixed, const V
 }
 
 // ---- heap on an LDS view (fm2d_ttime.f90:527-680) ---------------------------------
-#define HPX(e) ((e) >> 16)
-#define HPZ(e) ((e) & 0xffff)
-
+// Every lane of the wave holds the heap's bookkeeping and calls these; an entry is
+// its node's place in the view's storage, the keys are the nodes' times.
 struct ff_heap {
     int32_t *btg;    // 1-based
     int ntr;
@@ -759,88 +759,80 @@ struct ff_heap {
     int full;        // an insertion did not fit
 };
 
-__device__ __forceinline__ void ff_addtree(const fview &V, ff_heap &H, int iz, int ix)
+// The sift-up of addtree (:527-564) and updtree (:653-680): node e with time tv
+// starts at position p.  Lane j looks at the ancestor p >> (j + 1); those up to
+// the first that is not later move down a level.
+__device__ __forceinline__ void ff_siftup(const fview &V, const ff_heap &H, int p, int e, double tv)
+{
+    const int lane = threadIdx.x & 63;
+    const int m = w_level(p);
+    const bool act = lane < m;
+    const int ee = H.btg[act ? p >> (lane + 1) : 1];
+    const double k = V.T[act ? ee : e];
+    const unsigned long long stop = __builtin_amdgcn_ballot_w64(act && !(tv < k));
+    const int n = stop ? __builtin_ctzll(stop) : m;
+    if (lane <= n) {
+        const int to = p >> lane, ew = lane == n ? e : ee;
+        H.btg[to] = ew;
+        V.ns[ew] = (int16_t)to;
+    }
+    w_sync();
+}
+
+// addtree (:527-564); the node's time is tv already
+__device__ __forceinline__ void ff_addtree(const fview &V, ff_heap &H, int e, double tv)
 {
     if (H.ntr + 1 > H.cap) { H.full = 1; return; }
     H.ntr = H.ntr + 1;
-    V.n(iz, ix) = (int16_t)H.ntr;
-    H.btg[H.ntr] = (ix << 16) | iz;
-    int tpc = H.ntr, tpp = tpc / 2;
-    const double tv = V.t(iz, ix);
-    while (tpp > 0) {
-        int ep = H.btg[tpp];
-        if (tv < V.t(HPZ(ep), HPX(ep))) {
-            V.n(iz, ix) = (int16_t)tpp;
-            V.n(HPZ(ep), HPX(ep)) = (int16_t)tpc;
-            H.btg[tpp] = (ix << 16) | iz;      // the moving entry: the node's own
-            H.btg[tpc] = ep;
-            tpc = tpp;
-            tpp = tpc / 2;
-        } else {
-            tpp = 0;
-        }
-    }
+    ff_siftup(V, H, H.ntr, e, tv);
 }
 
+// downtree (:575-644): the last entry moves down from the root.  The lanes hold the
+// five levels under the hole: lane i has the node `off` of level `lv` (siblings are
+// lanes i and i ^ 1); a node is on the way if it and its ancestors up to the hole
+// are each the smaller sibling and earlier than the moving entry.
 __device__ __forceinline__ void ff_downtree(const fview &V, ff_heap &H)
 {
-    if (H.ntr == 1) { H.ntr = H.ntr - 1; return; }
-    const int el = H.btg[H.ntr];
-    V.n(HPZ(el), HPX(el)) = 1;
-    H.btg[1] = el;
+    const int lane = threadIdx.x & 63;
+    const int lv = w_level(lane + 2), off = lane + 2 - (1 << lv);
+    unsigned long long anc = 0;
+    for (int j = lane + 2; j >= 2; j >>= 1) anc |= 1ull << (j - 2);
+    const int el = __builtin_amdgcn_readfirstlane(H.btg[H.ntr]);
     H.ntr = H.ntr - 1;
-    // the entry moving down is el at every step (each comparison is against it
-    // as the parent), so its key is read once and the chosen child's entry and
-    // key are the ones just read
-    const double kel = V.t(HPZ(el), HPX(el));
-    int tpp = 1, tpc = 2 * tpp;
-    while (tpc < H.ntr) {
-        const int e0 = H.btg[tpc], e1 = H.btg[tpc + 1];
-        const double rd1 = V.t(HPZ(e0), HPX(e0));
-        const double rd2 = V.t(HPZ(e1), HPX(e1));
-        const bool right = rd1 > rd2;
-        if (right) tpc = tpc + 1;
-        const int ec = right ? e1 : e0;
-        const double kc = right ? rd2 : rd1;
-        if (kc < kel) {
-            V.n(HPZ(el), HPX(el)) = (int16_t)tpc;
-            V.n(HPZ(ec), HPX(ec)) = (int16_t)tpp;
-            H.btg[tpc] = el;
-            H.btg[tpp] = ec;
-            tpp = tpc;
-            tpc = 2 * tpp;
-        } else {
-            tpc = H.ntr + 1;
+    const int last = H.ntr;
+    if (last == 0) return;
+    const double kl = V.T[el];
+    int hole = 1;
+    for (bool more = true; more;) {
+        const int c = (hole << lv) + off;
+        const bool ok = lane < 62 && c <= last;
+        const int e = H.btg[ok ? c : 1];
+        double k = V.T[ok ? e : el];
+        if (!ok) k = __builtin_huge_val();
+        const double ks = w_quad_d<0xb1>(k);
+        // the right child when the left one's time is larger, else the left one
+        const bool sel = (lane & 1) ? ks > k : !(k > ks);
+        const unsigned long long P = __builtin_amdgcn_ballot_w64(ok && sel && k < kl);
+        const bool on = ok && (P & anc) == anc;
+        const unsigned long long path = __builtin_amdgcn_ballot_w64(on);
+        if (on) {
+            H.btg[c >> 1] = e;
+            V.ns[e] = (int16_t)(c >> 1);
         }
-    }
-    if (tpc == H.ntr) {
-        const int ec = H.btg[tpc];
-        if (V.t(HPZ(ec), HPX(ec)) < kel) {
-            V.n(HPZ(el), HPX(el)) = (int16_t)tpc;
-            V.n(HPZ(ec), HPX(ec)) = (int16_t)tpp;
-            H.btg[tpc] = el;
-            H.btg[tpp] = ec;
+        more = false;
+        if (path) {
+            const int j = 63 - __builtin_clzll(path) + 2;   // the deepest, as 2^level + offset
+            const int l = w_level(j);
+            hole = (hole << l) + j - (1 << l);
+            more = l == 5 && 2 * hole <= last;
         }
+        w_sync();
     }
-}
-
-__device__ __forceinline__ void ff_updtree(const fview &V, ff_heap &H, int iz, int ix)
-{
-    int tpc = V.n(iz, ix), tpp = tpc / 2;
-    const double tv = V.t(iz, ix);
-    while (tpp > 0) {
-        int ep = H.btg[tpp];
-        if (tv < V.t(HPZ(ep), HPX(ep))) {
-            V.n(iz, ix) = (int16_t)tpp;
-            V.n(HPZ(ep), HPX(ep)) = (int16_t)tpc;
-            H.btg[tpp] = (ix << 16) | iz;      // the moving entry: the node's own
-            H.btg[tpc] = ep;
-            tpc = tpp;
-            tpp = tpc / 2;
-        } else {
-            tpp = 0;
-        }
+    if (lane == 0) {
+        H.btg[hole] = el;
+        V.ns[el] = (int16_t)hole;
     }
+    w_sync();
 }
 
 __device__ __forceinline__ double ff_bilinear(const double nv[2][2], double dsx, double dsz, double dnx, double dnz)
@@ -867,96 +859,100 @@ struct ff_stop {
     int gen;                  // mode 3: 0 first generation, 1 second
 };
 
-__device__ __forceinline__ void ff_gen_set(const fview &V, uint32_t *b, int iz, int ix)
-{
-    long q = V.at(iz, ix);
-    b[q >> 5] |= 1u << (q & 31);
-}
-__device__ __forceinline__ bool ff_gen_get(const fview &V, const uint32_t *b, int iz, int ix)
-{
-    long q = V.at(iz, ix);
-    return (b[q >> 5] >> (q & 31)) & 1u;
-}
-
-// The reference's heap loop over the view (travel's :137-237) with fouds and
-// velocities vel(z,x); stops by rule S.  Called by the whole wave: lane 0
-// keeps the heap and the stop rule (H and S are lane 0's); the updates of the
-// popped node's four neighbours read frozen nodes only, which none of the four
-// is, so lanes 0-3 compute them at once and lane 0 then enters them into the
-// heap in the reference's order (x-1, x+1, z-1, z+1).
+// The reference's heap loop over the view (travel's :137-237) with velocities
+// vel(z,x); stops by rule S.  The whole wave runs it, every lane with the same H
+// and S: the moves of a pop and of each insertion are made by all lanes at once,
+// and lanes 4k + 2 sj + sk compute quadrant (sj, sk) of neighbour k's update (x-1,
+// x+1, z-1, z+1: the reference's order), the smallest of which fouds takes; the
+// four updates read frozen nodes only, which none of the four is.  A pop is a chain
+// of LDS round trips and FP64 operations: with one lane for the heap and a lane
+// per neighbour it took 8,000 cycles, so it took half of k_fm2d_near.
 template <int FOM, class VL>
 __device__ __forceinline__ void ff_heap_loop(const fview &V, ff_heap &H, const VL &vel, ff_stop &S)
 {
-    const int lane = threadIdx.x;
-    auto al = [&](int z, int x) -> bool { return V.n(z, x) == 0; };
+    const int lane = threadIdx.x & 63;
+    const int kn = (lane >> 2) & 3;
+    const int dx = kn == 0 ? -1 : (kn == 1 ? 1 : 0), dz = kn == 2 ? -1 : (kn == 3 ? 1 : 0);
+    const int ddx = (lane & 2) ? 1 : -1, ddz = (lane & 1) ? 1 : -1;
+    // er / ld below as a high product: the view lies in LDS, so er * ld < 2^32
+    const unsigned mag = (unsigned)(((1ull << 32) + (unsigned)V.ld - 1) / (unsigned)V.ld);
     for (;;) {
-        int go = 0, ix = 0, iz = 0;
-        if (lane == 0) {
-            do {
-                if (H.ntr <= 0) break;
-                if (H.full) { S.overflow = 1; break; }
-                int e = H.btg[1];
-                ix = HPX(e); iz = HPZ(e);
-                if (S.mode == 1 || S.mode == 4) {
-                    int swrg = 0;
-                    if (ix == 1 && S.vnl != 1) swrg = 1;
-                    if (ix == V.nnx && S.vnr != V.nnx) swrg = 1;
-                    if (iz == 1 && S.vnt != 1) swrg = 1;
-                    if (iz == V.nnz && S.vnb != V.nnz) swrg = 1;
-                    if (swrg == 1) { V.n(iz, ix) = 0; S.exited = 1; break; }
-                }
-                if ((S.mode == 2 || S.mode == 4) && S.have >= S.need) break;
-                if (S.mode == 3 && S.have >= S.need) {
-                    // every node of the generation is frozen: the second generation is
-                    // the band at this moment; after it the heap loop is a plain one
-                    if (S.gen == 1 || H.ntr == 0) break;
-                    for (int q = 1; q <= H.ntr; q++) ff_gen_set(V, S.gen_bits, HPZ(H.btg[q]), HPX(H.btg[q]));
-                    S.need += H.ntr;
-                    S.gen = 1;
-                    e = H.btg[1];
-                    ix = HPX(e); iz = HPZ(e);
-                }
-                // the updates around a popped node read up to three nodes away
-                {
-                    int xa = ix - 3 < 1 ? 1 : ix - 3, xb = ix + 3 > V.nnx ? V.nnx : ix + 3;
-                    int za = iz - 3 < 1 ? 1 : iz - 3, zb = iz + 3 > V.nnz ? V.nnz : iz + 3;
-                    if (!V.local(za, xa) || !V.local(zb, xb)) { S.overflow = 1; break; }
-                }
-                V.n(iz, ix) = 0;
-                if ((S.mode == 2 || S.mode == 4) && ix >= S.x0 && ix <= S.x1 && iz >= S.z0 && iz <= S.z1) S.have++;
-                if (S.mode == 3 && ff_gen_get(V, S.gen_bits, iz, ix)) S.have++;
-                ff_downtree(V, H);
-                go = 1;
-            } while (0);
+        if (H.ntr <= 0) break;
+        if (H.full) { S.overflow = 1; break; }
+        if (S.mode == 3 && S.have >= S.need) {
+            // every node of the generation is frozen: the second generation is
+            // the band at this moment; after it the heap loop is a plain one
+            if (S.gen == 1) break;
+            for (int q = lane + 1; q <= H.ntr; q += 64) {
+                const int b = H.btg[q];
+                atomicOr(&S.gen_bits[b >> 5], 1u << (b & 31));
+            }
+            w_sync();
+            S.need += H.ntr;
+            S.gen = 1;
         }
-        go = __shfl(go, 0, 64);
-        if (!go) break;
-        ix = __shfl(ix, 0, 64);
-        iz = __shfl(iz, 0, 64);
-        __syncthreads();
-        int nx = ix, nz = iz;
-        if (lane == 0) nx = ix - 1;
-        else if (lane == 1) nx = ix + 1;
-        else if (lane == 2) nz = iz - 1;
-        else nz = iz + 1;
-        const bool inb = lane < 4 && nx >= 1 && nx <= V.nnx && nz >= 1 && nz <= V.nnz;
-        const int st = inb ? (int)V.n(nz, nx) : 0;
-        double tv = 0.0;
-        if (st != 0) tv = ff_fouds<FOM>(V, al, nz, nx, 1.0 / vel(nz, nx));
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-            const int stk = __shfl(st, k, 64);
-            const double tvk = __shfl(tv, k, 64);
-            if (lane == 0 && stk != 0) {
-                const int xk = k == 0 ? ix - 1 : (k == 1 ? ix + 1 : ix);
-                const int zk = k == 2 ? iz - 1 : (k == 3 ? iz + 1 : iz);
-                V.t(zk, xk) = tvk;
-                if (stk == -1) ff_addtree(V, H, zk, xk);
-                else ff_updtree(V, H, zk, xk);
+        const int er = __builtin_amdgcn_readfirstlane(H.btg[1]);
+        const int qx = (int)__umulhi((unsigned)er, mag), ix = qx + V.ox + 1, iz = er - qx * V.ld + V.oz + 1;
+        if (S.mode == 1 || S.mode == 4) {
+            int swrg = 0;
+            if (ix == 1 && S.vnl != 1) swrg = 1;
+            if (ix == V.nnx && S.vnr != V.nnx) swrg = 1;
+            if (iz == 1 && S.vnt != 1) swrg = 1;
+            if (iz == V.nnz && S.vnb != V.nnz) swrg = 1;
+            if (swrg == 1) {
+                if (lane == 0) V.ns[er] = 0;
+                S.exited = 1;
+                break;
             }
         }
-        __syncthreads();
+        if ((S.mode == 2 || S.mode == 4) && S.have >= S.need) break;
+        // the updates around a popped node read up to three nodes away
+        {
+            int xa = ix - 3 < 1 ? 1 : ix - 3, xb = ix + 3 > V.nnx ? V.nnx : ix + 3;
+            int za = iz - 3 < 1 ? 1 : iz - 3, zb = iz + 3 > V.nnz ? V.nnz : iz + 3;
+            if (!V.local(za, xa) || !V.local(zb, xb)) { S.overflow = 1; break; }
+        }
+        // the lane's neighbour (off the grid: the node itself) and its velocity,
+        // in flight during the heap's moves
+        const int nx = ix + dx, nz = iz + dz;
+        const bool in = lane < 16 && nx >= 1 && nx <= V.nnx && nz >= 1 && nz <= V.nnz;
+        const int cx = in ? nx : ix, cz = in ? nz : iz;
+        const double vz = vel(cz, cx);
+        if ((S.mode == 2 || S.mode == 4) && ix >= S.x0 && ix <= S.x1 && iz >= S.z0 && iz <= S.z1) S.have++;
+        if (S.mode == 3 && ((S.gen_bits[er >> 5] >> (er & 31)) & 1u)) S.have++;
+        if (lane == 0) V.ns[er] = 0;
+        ff_downtree(V, H);
+        const int x1 = cx + ddx, x2 = cx + 2 * ddx, z1 = cz + ddz, z2 = cz + 2 * ddz;
+        const bool ix1 = x1 >= 1 && x1 <= V.nnx, iz1 = z1 >= 1 && z1 <= V.nnz;
+        const bool ix2 = FOM != 0 && x2 >= 1 && x2 <= V.nnx, iz2 = FOM != 0 && z2 >= 1 && z2 <= V.nnz;
+        const int o = (int)V.at(cz, cx);
+        const int ox1 = ix1 ? o + ddx * V.ld : o, ox2 = ix2 ? o + 2 * ddx * V.ld : o;
+        const int oz1 = iz1 ? o + ddz : o, oz2 = iz2 ? o + 2 * ddz : o;
+        const int st = in ? (int)V.ns[o] : 0;
+        double tv = W_NONE;
+        if (ix1 && iz1)
+            tv = w_quadrant<FOM>(V.ns[ox1] == 0, ix2 && V.ns[ox2] == 0, V.ns[oz1] == 0, iz2 && V.ns[oz2] == 0,
+                                 V.T[ox1], FOM ? V.T[ox2] : 0.0, V.T[oz1], FOM ? V.T[oz2] : 0.0, 1.0 / vz, V.dnx,
+                                 V.dnz);
+        tv = fmin(tv, w_quad_d<0xb1>(tv));
+        tv = fmin(tv, w_quad_d<0x4e>(tv));
+        if (tv >= W_NONE) tv = 0.0;          // no quadrant: the reference's travm stays 0
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const int stk = __builtin_amdgcn_readlane(st, 4 * k);
+            if (stk == 0) continue;
+            const int ok = __builtin_amdgcn_readlane(o, 4 * k);
+            const long long tb = __double_as_longlong(tv);
+            const int tlo = __builtin_amdgcn_readlane((int)tb, 4 * k);
+            const int thi = __builtin_amdgcn_readlane((int)(tb >> 32), 4 * k);
+            const double tk = __longlong_as_double(((long long)thi << 32) | (unsigned int)tlo);
+            if (lane == 0) V.T[ok] = tk;
+            w_sync();
+            if (stk == -1) ff_addtree(V, H, ok, tk);
+            else ff_siftup(V, H, __builtin_amdgcn_readfirstlane((int)V.ns[ok]), ok, tk);
+        }
     }
+    w_sync();
 }
 
 // travel's corner initialisation (fm2d_ttime.f90:105-126) and heap start.
@@ -975,8 +971,11 @@ __device__ __forceinline__ void ff_corners(const fview &V, ff_heap &H, const VL 
         for (int j = 1; j <= 2; j++) {
             double ex = dsx - (i - 1) * V.dnx, ez = dsz - (j - 1) * V.dnz;
             double ds = sqrt(ex * ex + ez * ez);
-            V.t(isz - 1 + j, isx - 1 + i) = 2.0 * ds / (vss[i - 1][j - 1] + vsrc);
-            ff_addtree(V, H, isz - 1 + j, isx - 1 + i);
+            const double tc = 2.0 * ds / (vss[i - 1][j - 1] + vsrc);
+            const int o = (int)V.at(isz - 1 + j, isx - 1 + i);
+            if ((threadIdx.x & 63) == 0) V.T[o] = tc;
+            w_sync();
+            ff_addtree(V, H, o, tc);
         }
 }
 
@@ -1226,7 +1225,7 @@ __global__ __launch_bounds__(64) void k_fm2d_near(mct_fm2d_args A, int region_no
         // as the reference checks its exit first)
         ff_stop S;
         memset(&S, 0, sizeof S);
-        if (lane == 0) {
+        {
             int risx = (int)((x - gorx) / R.dnx) + 1, risz = (int)((z - gorz) / R.dnz) + 1;
             bool ok = !(risx < 1 || risx > R.nnx || risz < 1 || risz > R.nnz);
             if (ok) {
@@ -1248,7 +1247,7 @@ __global__ __launch_bounds__(64) void k_fm2d_near(mct_fm2d_args A, int region_no
                 }
                 S.need = (S.x1 - S.x0 + 1) * (S.z1 - S.z0 + 1);
             } else {
-                sh_ovf = 3;   // source outside the refined grid: use the sequential solver
+                if (lane == 0) sh_ovf = 3;   // source outside the refined grid: use the sequential solver
             }
         }
         __syncthreads();
@@ -1400,32 +1399,30 @@ __global__ __launch_bounds__(64) void k_fm2d_near(mct_fm2d_args A, int region_no
         for (int w = lane; w < (C.lnx * C.lnz + 31) / 32; w += 64) DB[w] = 0u;
         __syncthreads();
         memset(&S, 0, sizeof S);
-        if (lane == 0) {
-            S.mode = 3;
-            S.gen_bits = DB;
-            H.ntr = 0;
-            H.full = 0;
-        }
+        S.mode = 3;
+        S.gen_bits = DB;
+        H.ntr = 0;
+        H.full = 0;
+        __syncthreads();
         {
             // the band's nodes enter the heap in scan order (x outer, z inner): the
-            // wave tests 64 nodes at a time and lane 0 adds the band nodes among
-            // them in lane order (adding a node changes only the states of nodes
-            // already in the heap, which stay positive, so the tests stand)
+            // wave tests 64 nodes at a time and adds the band nodes among them in lane
+            // order (adding a node changes only the states of nodes already in the
+            // heap, which stay positive, so the tests stand)
             const int cz = lz1 - lz0 + 1, tot = (lx1 - lx0 + 1) * cz;
             for (int b0 = 0; b0 < tot; b0 += 64) {
                 const int q = b0 + lane;
                 const int i = lx0 + q / cz, j = lz0 + q % cz;
                 const bool band = q < tot && C.n(j, i) > 0;
                 unsigned long long m = __ballot(band);
+                const int o = band ? (int)C.at(j, i) : 0;
+                if (band) atomicOr(&DB[o >> 5], 1u << (o & 31));
+                S.need += __builtin_popcountll(m);
                 while (m) {
                     const int l = __builtin_ctzll(m);
                     m &= m - 1;
-                    const int il = __shfl(i, l, 64), jl = __shfl(j, l, 64);
-                    if (lane == 0) {
-                        ff_addtree(C, H, jl, il);
-                        ff_gen_set(C, DB, jl, il);
-                        S.need++;
-                    }
+                    const int ol = __builtin_amdgcn_readlane(o, l);
+                    ff_addtree(C, H, ol, C.T[ol]);
                 }
             }
         }
@@ -1439,7 +1436,7 @@ __global__ __launch_bounds__(64) void k_fm2d_near(mct_fm2d_args A, int region_no
         __syncthreads();
         ff_stop S;
         memset(&S, 0, sizeof S);
-        if (lane == 0) {
+        {
             ff_corners(C, H, cvel, x, z, A.gox, A.goz, g.isx, g.isz);
             S.mode = 2;
             S.x0 = g.isx - FF_SEED_RINGS < 1 ? 1 : g.isx - FF_SEED_RINGS;
@@ -1454,14 +1451,13 @@ __global__ __launch_bounds__(64) void k_fm2d_near(mct_fm2d_args A, int region_no
         if (lane == 0) sh_ovf = S.overflow || H.full;
         __syncthreads();
     }
-    if (A.verify > 0 && lane == 0 && !sh_ovf) {
+    if (A.verify > 0 && !sh_ovf) {
         // the band handed to the sweep must be a valid heap: fouds overwrites a
         // key and updtree only sifts up, so a raised key can leave it out of
         // order, and then the pops that follow are not in time order
-        for (int q = 2; q <= H.ntr; q++) {
-            const int ec = H.btg[q], ep = H.btg[q / 2];
-            if (C.t(HPZ(ec), HPX(ec)) < C.t(HPZ(ep), HPX(ep))) { sh_ovf = 4; break; }
-        }
+        bool bad = false;
+        for (int q = lane + 2; q <= H.ntr; q += 64) bad |= C.T[H.btg[q]] < C.T[H.btg[q / 2]];
+        if (__builtin_amdgcn_ballot_w64(bad) && lane == 0) sh_ovf = 4;
     }
     __syncthreads();
     if (sh_ovf) {
