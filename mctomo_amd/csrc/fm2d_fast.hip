@@ -643,15 +643,10 @@ struct ff_edges {
     bool left, right, top, bottom;   // which edges are inner edges
 };
 
-template <int FOM, bool FAST, class FX, class VL>
+template <int FOM, class FX, class VL>
 __device__ __forceinline__ int ff_sweep(const fview &V, const FX &fixed, const VL &vel, int *sh_flag,
-                        const ff_work *W, int *stat = nullptr, const ff_edges *E = nullptr)
+                        const ff_work *W, int *stat = nullptr)
 {
-    const bool prune = FOM == 0 && E != nullptr;
-    auto on_edge = [&](int iz, int ix) -> bool {
-        return (ix == 1 && E->left) || (ix == V.nnx && E->right) || (iz == 1 && E->top) || (iz == V.nnz && E->bottom);
-    };
-    const ff_k0 K0 = ff_k0_make(V.dnx, V.dnz);
     int n_steps = 0, n_evals = 0;
     const int nt = blockDim.x, tid = threadIdx.x;
     const int reach = FOM == 0 ? 1 : 2;
@@ -716,10 +711,8 @@ __device__ __forceinline__ int ff_sweep(const fview &V, const FX &fixed, const V
                     ff_load_sten<FOM>(V, z, x, S);
                     const double t = V.t(z, x);
                     double slown = 1.0 / vz;
-                    double c = (FAST && FOM == 0) ? ff_cands0f(S, K0, slown) : ff_cands<FOM>(S, V.dnx, V.dnz, slown);
+                    double c = ff_cands<FOM>(S, V.dnx, V.dnz, slown);
                     if (c < FF_THR0 && c != t) {
-                        if (prune && c > __longlong_as_double((long long)*E->bound)) continue;
-                        if (prune && on_edge(z, x)) atomicMin(E->bound, (unsigned long long)__double_as_longlong(c));
                         if (fabs(c - t) > 1e-14 * c) changed = 1;
                         V.t(z, x) = c;
                         if (W) {
@@ -745,6 +738,99 @@ __device__ __forceinline__ int ff_sweep(const fview &V, const FX &fixed, const V
             if (stat) { atomicAdd(&stat[1], tid == 0 ? n_steps : 0); atomicAdd(&stat[2], n_evals); }
             return round + 1;
         }
+    }
+    return -1;
+}
+
+// The first-order sweep of the refined grid in LDS by one wave: ff_sweep<0>'s rounds,
+// diagonals and updates.  A step is a chain (flags, work bits, stencil, update,
+// marks) that nothing else of the wave hides, so its reads are issued together,
+// 64 flags are looked at in one read, a changed node marks its neighbours without
+// looking whether they are fixed (a fixed node's mark is dropped when it comes up),
+// and a diagonal's flag is set once per node, not once per mark.  A problem of
+// 65 x 65 refined nodes takes 380 steps of about 16 updates.  With ff_sweep the
+// near-source kernel of 61,440 problems took 79.8 ms instead of 67.8.
+template <class VL>
+__device__ __forceinline__ int ff_sweep_wave(const fview &V, const VL &vel, const ff_work &W, const ff_edges &E)
+{
+    const ff_k0 K0 = ff_k0_make(V.dnx, V.dnz);
+    const int lane = threadIdx.x & 63;
+    const int nn = V.nnx * V.nnz, ND = V.nnx + V.nnz - 1, ld = V.nnz;
+    const unsigned mag = (unsigned)(((1ull << 32) + (unsigned)ld - 1) / (unsigned)ld);   // q / ld, q * ld < 2^32
+    for (int w = lane; w < (nn + 31) / 32; w += 64) W.bits[w] = 0u;
+    for (int d = lane; d < ND; d += 64) { W.cs[d] = 0; W.cd[d] = 0; }
+    w_sync();
+    for (int q = lane; q < nn; q += 64) {
+        const int x0 = (int)__umulhi((unsigned)q, mag), z0 = q - x0 * ld;
+        if (V.ns[q] == 0) continue;
+        const bool nb = (x0 > 0 && V.ns[q - ld] == 0) || (x0 + 1 < V.nnx && V.ns[q + ld] == 0) ||
+                        (z0 > 0 && V.ns[q - 1] == 0) || (z0 + 1 < V.nnz && V.ns[q + 1] == 0);
+        if (nb) {
+            atomicOr(&W.bits[q >> 5], 1u << (q & 31));
+            W.cs[x0 + z0] = 1;
+            W.cd[V.nnx - 1 - x0 + z0] = 1;
+        }
+    }
+    w_sync();
+    for (int round = 0; round < FF_MAX_ROUNDS; round++) {
+        bool changed = false;
+        for (int dir = 0; dir < 4; dir++) {
+            // sum diagonals upwards and downwards, difference diagonals likewise
+            int *fl = dir == 0 || dir == 3 ? W.cs : W.cd;
+            const bool back = dir >= 2;
+            for (int d = 0; d < ND; d++) {
+                unsigned long long m = 0;
+                for (; d < ND; d += 64) {
+                    const int df = d + lane < ND ? d + lane : ND - 1;
+                    m = __builtin_amdgcn_ballot_w64(fl[back ? ND - 1 - df : df] != 0 && d + lane < ND);
+                    if (m) break;
+                }
+                if (!m) break;
+                d += __builtin_ctzll(m);
+                if (lane == 0) fl[back ? ND - 1 - d : d] = 0;
+                const int a_lo = d - (V.nnz - 1) > 0 ? d - (V.nnz - 1) : 0;
+                const int a_hi = d < V.nnx - 1 ? d : V.nnx - 1;
+                for (int a = a_lo + lane; a <= a_hi; a += 64) {
+                    const int b = d - a;
+                    const int x0 = (dir & 1) ? V.nnx - 1 - a : a, z0 = (dir & 2) ? V.nnz - 1 - b : b;
+                    const int o = x0 * ld + z0;
+                    const double vz = vel(z0 + 1, x0 + 1);
+                    const bool ixl = x0 > 0, ixh = x0 + 1 < V.nnx, izl = z0 > 0, izh = z0 + 1 < V.nnz;
+                    unsigned word = W.bits[o >> 5];
+                    int st = V.ns[o];
+                    double t = V.T[o], xl = V.T[ixl ? o - ld : o], xh = V.T[ixh ? o + ld : o];
+                    double zl = V.T[izl ? o - 1 : o], zh = V.T[izh ? o + 1 : o];
+                    double bound = __longlong_as_double((long long)*E.bound);
+                    // (read before the branch that uses them)
+                    asm volatile("" : "+v"(word), "+v"(st), "+v"(t), "+v"(xl), "+v"(xh), "+v"(zl), "+v"(zh), "+v"(bound));
+                    const unsigned bm = 1u << (o & 31);
+                    if (!(word & bm)) continue;
+                    atomicAnd(&W.bits[o >> 5], ~bm);
+                    if (st == 0) continue;
+                    const double slown = 1.0 / vz;
+                    ff_sten S;
+                    S.ix1[0] = ixl; S.ix1[1] = ixh; S.iz1[0] = izl; S.iz1[1] = izh;
+                    S.tx1[0] = xl; S.tx1[1] = xh; S.tz1[0] = zl; S.tz1[1] = zh;
+                    const double c = ff_cands0f(S, K0, slown);
+                    if (!(c < FF_THR0 && c != t) || c > bound) continue;
+                    V.T[o] = c;
+                    if ((!ixl && E.left) || (!ixh && E.right) || (!izl && E.top) || (!izh && E.bottom))
+                        atomicMin(E.bound, (unsigned long long)__double_as_longlong(c));
+                    changed |= fabs(c - t) > 1e-14 * c;
+                    if (ixl) atomicOr(&W.bits[(o - ld) >> 5], 1u << ((o - ld) & 31));
+                    if (ixh) atomicOr(&W.bits[(o + ld) >> 5], 1u << ((o + ld) & 31));
+                    if (izl) atomicOr(&W.bits[(o - 1) >> 5], 1u << ((o - 1) & 31));
+                    if (izh) atomicOr(&W.bits[(o + 1) >> 5], 1u << ((o + 1) & 31));
+                    const int s = x0 + z0, e = V.nnx - 1 - x0 + z0;
+                    if (s > 0) W.cs[s - 1] = 1;
+                    if (s + 1 < ND) W.cs[s + 1] = 1;
+                    if (e > 0) W.cd[e - 1] = 1;
+                    if (e + 1 < ND) W.cd[e + 1] = 1;
+                }
+                w_sync();
+            }
+        }
+        if (!__builtin_amdgcn_ballot_w64(changed)) return round + 1;
     }
     return -1;
 }
@@ -981,10 +1067,11 @@ __device__ __forceinline__ void ff_corners(const fview &V, ff_heap &H, const VL 
 
 __device__ __forceinline__ void bspl_w4(double u, double w[4])
 {
-    w[0] = (1.0 - u) * (1.0 - u) * (1.0 - u) / 6.0;
-    w[1] = (4.0 - 6.0 * (u * u) + 3.0 * (u * u * u)) / 6.0;
-    w[2] = (1.0 + 3.0 * u + 3.0 * (u * u) - 3.0 * (u * u * u)) / 6.0;
-    w[3] = (u * u * u) / 6.0;
+    const double r6 = fp_recip(6.0);
+    w[0] = fp_quot((1.0 - u) * (1.0 - u) * (1.0 - u), 6.0, r6);
+    w[1] = fp_quot(4.0 - 6.0 * (u * u) + 3.0 * (u * u * u), 6.0, r6);
+    w[2] = fp_quot(1.0 + 3.0 * u + 3.0 * (u * u) - 3.0 * (u * u * u), 6.0, r6);
+    w[3] = fp_quot(u * u * u, 6.0, r6);
 }
 
 // Work-group -> problem slot map that keeps neighbouring slots (the sources
@@ -1278,7 +1365,10 @@ __global__ __launch_bounds__(64) void k_fm2d_near(mct_fm2d_args A, int region_no
             ff_edges RE;
             RE.bound = &sh_bound;
             RE.left = g.vnl != 1; RE.right = g.vnr != R.nnx; RE.top = g.vnt != 1; RE.bottom = g.vnb != R.nnz;
-            int rounds = ff_sweep<FOM, true>(R, rfixed, rvel, &sh_flag, &RW, nullptr, FOM == 0 ? &RE : nullptr);
+            int rounds;
+            if constexpr (FOM == 0) rounds = ff_sweep_wave(R, rvel, RW, RE);
+            else rounds = ff_sweep<FOM>(R, rfixed, rvel, &sh_flag, &RW);
+            __syncthreads();
             if (rounds < 0) {
                 if (lane == 0) pflag[slot] = 1;
                 return;
@@ -1544,7 +1634,7 @@ __global__ __launch_bounds__(256) void k_fm2d_sweep(mct_fm2d_args A, int32_t *pf
     int *stat = A.rounds_out ? A.rounds_out + 4 * slot : nullptr;
     if (stat && threadIdx.x == 0) { stat[1] = 0; stat[2] = 0; }
     __syncthreads();
-    int rounds = ff_sweep<FOM, false>(V, fixed, vel, &sh_flag, use_dirty ? &W : nullptr, stat);
+    int rounds = ff_sweep<FOM>(V, fixed, vel, &sh_flag, use_dirty ? &W : nullptr, stat);
     if (rounds < 0) {
         // the mixed-order update need not settle (it is not monotone): with the
         // heap-order check on, the sequential solver takes the problem
