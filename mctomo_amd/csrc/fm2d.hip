@@ -687,7 +687,7 @@ struct wave_grid {
 template <int GL>
 __device__ __forceinline__ unsigned long long w_ballot(const wave_grid &G, bool p)
 {
-    const unsigned long long m = __ballot(p);
+    const unsigned long long m = __builtin_amdgcn_ballot_w64(p);
     return GL == 64 ? m : ((m >> G.base) & 0xffffull);
 }
 // a value that every lane of the group holds (one wave: a scalar)

@@ -2,6 +2,7 @@
 // together: k_fm2d_wave's and k_fm2d_near's.
 #pragma once
 #include <hip/hip_runtime.h>
+#include "fp64_ops.h"
 
 #pragma clang fp contract(off)
 
@@ -83,9 +84,10 @@ __device__ __forceinline__ double w_quadrant(bool aj, bool aj2, bool ak, bool ak
     }
     double rd1 = b * b - 4.0 * a * c;
     if (rd1 < 0.0) rd1 = 0.0;
-    const double tdsh = (-b + sqrt(rd1)) / (2.0 * a);
+    const double tdsh = fp_div(-b + fp_sqrt(rd1), 2.0 * a);
     const double trav = tref + tdsh;
-    return FOM == 0 ? trav : trav / tdiv;
+    if (FOM == 0 || tdiv == 1.0) return trav;
+    return fp_quot(trav, 3.0, fp_recip(3.0));
 }
 
 } // namespace
