@@ -65,11 +65,11 @@ struct fview {
     int nnx, nnz;
     double dnx, dnz;
     double *T;
-    int16_t *ns;          // LDS states (-1 far, 0 frozen, >0 heap position) or null
+    int8_t *ns;           // LDS states (-1 far, 0 frozen, 1 in the heap) or null
     int ld, ox, oz, lnx, lnz;
     __device__ __forceinline__ long at(int iz, int ix) const { return (long)(ix - ox - 1) * ld + (iz - oz - 1); }
     __device__ __forceinline__ double &t(int iz, int ix) const { return T[at(iz, ix)]; }
-    __device__ __forceinline__ int16_t &n(int iz, int ix) const { return ns[at(iz, ix)]; }
+    __device__ __forceinline__ int8_t &n(int iz, int ix) const { return ns[at(iz, ix)]; }
     __device__ __forceinline__ bool local(int iz, int ix) const
     {
         return ix > ox && ix <= ox + lnx && iz > oz && iz <= oz + lnz;
@@ -837,9 +837,12 @@ __device__ __forceinline__ int ff_sweep_wave(const fview &V, const VL &vel, cons
 
 // ---- heap on an LDS view (fm2d_ttime.f90:527-680) ---------------------------------
 // Every lane of the wave holds the heap's bookkeeping and calls these; an entry is
-// its node's place in the view's storage, the keys are the nodes' times.
+// its node's place in the view's storage, the keys are the nodes' times.  A node
+// does not know its entry's position: 64 entries are searched in one read, so a
+// state takes one byte, and with 16-bit entries four problems of 65 x 65 refined
+// nodes fit a CU's LDS instead of three.
 struct ff_heap {
-    int32_t *btg;    // 1-based
+    uint16_t *btg;   // 1-based
     int ntr;
     int cap;         // entries the LDS heap holds
     int full;        // an insertion did not fit
@@ -859,10 +862,21 @@ __device__ __forceinline__ void ff_siftup(const fview &V, const ff_heap &H, int 
     const int n = stop ? __builtin_ctzll(stop) : m;
     if (lane <= n) {
         const int to = p >> lane, ew = lane == n ? e : ee;
-        H.btg[to] = ew;
-        V.ns[ew] = (int16_t)to;
+        H.btg[to] = (uint16_t)ew;
     }
     w_sync();
+}
+
+// the position of node e, which is in the heap
+__device__ __forceinline__ int ff_find(const ff_heap &H, int e)
+{
+    const int lane = threadIdx.x & 63;
+    for (int b = 1; b <= H.ntr; b += 64) {
+        const int q = b + lane <= H.ntr ? b + lane : b;
+        const unsigned long long m = __builtin_amdgcn_ballot_w64(H.btg[q] == e);
+        if (m) return b + __builtin_ctzll(m);
+    }
+    return 1;
 }
 
 // addtree (:527-564); the node's time is tv already
@@ -870,6 +884,7 @@ __device__ __forceinline__ void ff_addtree(const fview &V, ff_heap &H, int e, do
 {
     if (H.ntr + 1 > H.cap) { H.full = 1; return; }
     H.ntr = H.ntr + 1;
+    if ((threadIdx.x & 63) == 0) V.ns[e] = 1;
     ff_siftup(V, H, H.ntr, e, tv);
 }
 
@@ -883,7 +898,7 @@ __device__ __forceinline__ void ff_downtree(const fview &V, ff_heap &H)
     const int lv = w_level(lane + 2), off = lane + 2 - (1 << lv);
     unsigned long long anc = 0;
     for (int j = lane + 2; j >= 2; j >>= 1) anc |= 1ull << (j - 2);
-    const int el = __builtin_amdgcn_readfirstlane(H.btg[H.ntr]);
+    const int el = __builtin_amdgcn_readfirstlane((int)H.btg[H.ntr]);
     H.ntr = H.ntr - 1;
     const int last = H.ntr;
     if (last == 0) return;
@@ -902,8 +917,7 @@ __device__ __forceinline__ void ff_downtree(const fview &V, ff_heap &H)
         const bool on = ok && (P & anc) == anc;
         const unsigned long long path = __builtin_amdgcn_ballot_w64(on);
         if (on) {
-            H.btg[c >> 1] = e;
-            V.ns[e] = (int16_t)(c >> 1);
+            H.btg[c >> 1] = (uint16_t)e;
         }
         more = false;
         if (path) {
@@ -914,10 +928,7 @@ __device__ __forceinline__ void ff_downtree(const fview &V, ff_heap &H)
         }
         w_sync();
     }
-    if (lane == 0) {
-        H.btg[hole] = el;
-        V.ns[el] = (int16_t)hole;
-    }
+    if (lane == 0) H.btg[hole] = (uint16_t)el;
     w_sync();
 }
 
@@ -977,7 +988,7 @@ __device__ __forceinline__ void ff_heap_loop(const fview &V, ff_heap &H, const V
             S.need += H.ntr;
             S.gen = 1;
         }
-        const int er = __builtin_amdgcn_readfirstlane(H.btg[1]);
+        const int er = __builtin_amdgcn_readfirstlane((int)H.btg[1]);
         const int qx = (int)__umulhi((unsigned)er, mag), ix = qx + V.ox + 1, iz = er - qx * V.ld + V.oz + 1;
         if (S.mode == 1 || S.mode == 4) {
             int swrg = 0;
@@ -1035,7 +1046,7 @@ __device__ __forceinline__ void ff_heap_loop(const fview &V, ff_heap &H, const V
             if (lane == 0) V.T[ok] = tk;
             w_sync();
             if (stk == -1) ff_addtree(V, H, ok, tk);
-            else ff_siftup(V, H, __builtin_amdgcn_readfirstlane((int)V.ns[ok]), ok, tk);
+            else ff_siftup(V, H, ff_find(H, ok), ok, tk);
         }
     }
     w_sync();
@@ -1217,20 +1228,22 @@ __device__ __forceinline__ void ff_srtimes(const mct_fm2d_args &A, const near_ge
     }
 }
 
-// One wave per problem.  LDS: region (doubles + int16 states) sized for the
-// larger of the refined grid and the coarse neighbourhood, the heap, and the
-// remap staging of the refined window's coarse nodes.
+#define FF_W_FROZEN ((long long)0x8000000000000000ull)
+#define FF_W_FAR ((long long)0xffffffffffffffffull)      // no time's bits
+// One wave per problem.  LDS: region (doubles + int8 states) sized for the
+// larger of the refined grid and the coarse neighbourhood, the heap, the sweep's
+// work bits and diagonal flags.  The kernel is bound by its chains of LDS reads and
+// FP64 operations, so the number of problems on a CU is its speed: 4 with 65 x 65
+// refined nodes (40.7 KB); with 48.9 KB (two-byte states, 32-bit heap entries, the
+// window staged in LDS), 3, 61,440 problems took 66.9 ms instead of 51.6.
 template <int FOM>
-__global__ __launch_bounds__(64) void k_fm2d_near(mct_fm2d_args A, int region_nodes, int heap_cap,
-                                                  int win_nodes, int32_t *pflag)
+__global__ __launch_bounds__(64) void k_fm2d_near(mct_fm2d_args A, int region_nodes, int heap_cap, int32_t *pflag)
 {
     extern __shared__ double ff_lds[];
     double *RT = ff_lds;
-    int16_t *RN = (int16_t *)(RT + region_nodes);
-    int32_t *HB = (int32_t *)(RN + ((region_nodes + 3) & ~3));
-    double *WT = (double *)(HB + ((heap_cap + 2 + 1) & ~1));
-    int16_t *WN = (int16_t *)(WT + win_nodes);
-    uint32_t *DB = (uint32_t *)(WN + ((win_nodes + 1) & ~1));
+    int8_t *RN = (int8_t *)(RT + region_nodes);
+    uint16_t *HB = (uint16_t *)(RN + ((region_nodes + 3) & ~3));
+    uint32_t *DB = (uint32_t *)(HB + ((heap_cap + 2 + 1) & ~1));
     int *DC = (int *)(DB + (region_nodes + 31) / 32);   // 2 x diag_cap counts
     ff_work RW;
     RW.bits = DB;
@@ -1418,7 +1431,7 @@ __global__ __launch_bounds__(64) void k_fm2d_near(mct_fm2d_args A, int region_no
                 RT[q] = tv;
                 RN[q] = 1;
             };
-            int *BL = HB;
+            uint16_t *BL = HB;
             const int blcap = (heap_cap + 2 + 1) & ~1;
             if (lane == 0) sh_nbl = 0;
             __syncthreads();
@@ -1427,7 +1440,7 @@ __global__ __launch_bounds__(64) void k_fm2d_near(mct_fm2d_args A, int region_no
                 const double tlast = close_tlast(q);
                 if (tlast >= 0) {
                     const int k = atomicAdd(&sh_nbl, 1);
-                    if (k < blcap) BL[k] = q;
+                    if (k < blcap) BL[k] = (uint16_t)q;
                     else close_solve(q, tlast);
                 }
             }
@@ -1454,13 +1467,16 @@ __global__ __launch_bounds__(64) void k_fm2d_near(mct_fm2d_args A, int region_no
                 nr[o] = RN[q];
             }
         }
-        // stage the refined values at the window's coarse nodes (remap, :354-416)
+        // stage the refined values at the window's coarse nodes (remap, :354-416) in
+        // the slot's vr, whose velocities are no longer read: a lane reads back what it
+        // wrote; the state is the sign (frozen) or FF_W_FAR
+        long long *WT = (long long *)vr;
         const int wnx = g.vnr - g.vnl + 1, wnz = g.vnb - g.vnt + 1;
         for (int q = lane; q < wnx * wnz; q += 64) {
             int a = q / wnz, b = q % wnz;
             int l = a * A.sgdl + 1, k = b * A.sgdl + 1;
-            WN[q] = R.n(k, l);
-            WT[q] = R.t(k, l);
+            const long long w = __double_as_longlong(R.t(k, l));   // >= 0
+            WT[q] = R.n(k, l) == 0 ? (w | FF_W_FROZEN) : (R.n(k, l) > 0 ? w : FF_W_FAR);
         }
         __syncthreads();
         // coarse neighbourhood: far everywhere, then the remapped window
@@ -1469,9 +1485,9 @@ __global__ __launch_bounds__(64) void k_fm2d_near(mct_fm2d_args A, int region_no
         for (int q = lane; q < wnx * wnz; q += 64) {
             int a = q / wnz, b = q % wnz;
             int idm2 = g.vnl + a, idm1 = g.vnt + b;
-            int st = WN[q];
-            C.n(idm1, idm2) = (int16_t)st;
-            if (st >= 0) C.t(idm1, idm2) = WT[q];
+            const long long w = WT[q];
+            C.n(idm1, idm2) = w == FF_W_FAR ? -1 : (w < 0 ? 0 : 1);
+            if (w != FF_W_FAR) C.t(idm1, idm2) = __longlong_as_double(w & ~FF_W_FROZEN);
         }
         __syncthreads();
         // frozen nodes next to far nodes re-enter the band
@@ -2114,7 +2130,7 @@ static size_t ff_strip_lds(const mct_fm2d_args &a)
 }
 
 // LDS bytes of k_fm2d_near for the geometry in a.
-static size_t ff_near_lds(const mct_fm2d_args &a, int &region, int &heap_cap, int &win)
+static size_t ff_near_lds(const mct_fm2d_args &a, int &region, int &heap_cap)
 {
     const int rg = 2 * a.sgs * a.sgdl + 1;
     const int wn = 2 * a.sgs + 1;
@@ -2127,19 +2143,21 @@ static size_t ff_near_lds(const mct_fm2d_args &a, int &region, int &heap_cap, in
     // the heap holds a narrow band only; a problem whose band outgrows it goes
     // to the sequential solver
     heap_cap = region < 512 ? region : 512;
-    win = a.asgr == 1 ? wn * wn : 1;
-    // times and states of the region, heap, remap staging, bit set, diagonal flags
-    size_t b = 8 * (size_t)region + 2 * (size_t)((region + 3) & ~3) + 4 * (size_t)((heap_cap + 2 + 1) & ~1) +
-               8 * (size_t)win + 2 * (size_t)((win + 1) & ~1) + 4 * (size_t)((region + 31) / 32) +
-               4 * 2 * (size_t)(rgx + rgz) + 64;
+    // times and states of the region, heap, bit set, diagonal flags
+    const size_t b = 8 * (size_t)region + (size_t)((region + 3) & ~3) + 2 * (size_t)((heap_cap + 2 + 1) & ~1) +
+                     4 * (size_t)((region + 31) / 32) + 4 * 2 * (size_t)(rgx + rgz);
     return b;
 }
 
 int mct_fm2d_fast_ok(const mct_fm2d_args &a)
 {
-    int region, heap_cap, win;
-    size_t b = ff_near_lds(a, region, heap_cap, win);
-    // heap positions and coordinates are 16-bit; LDS within the device's limit per workgroup
+    int region, heap_cap;
+    const size_t wn = a.asgr == 1 ? 2 * (size_t)a.sgs + 1 : 1;
+    // The region with room to spare for a second byte per state, 32-bit heap entries
+    // and the window: beyond this line a problem would have a CU to itself, and the
+    // sequential solver takes it.  Heap entries and coordinates are 16-bit.
+    size_t b = ff_near_lds(a, region, heap_cap);
+    b += (size_t)region + 2 * (size_t)(heap_cap + 2) + 10 * wn * wn + 64;
     static int lds_max = 0;
     if (!lds_max) {
         int dev = 0, v = 0;
@@ -2154,8 +2172,8 @@ int mct_fm2d_fast_ok(const mct_fm2d_args &a)
 int mct_launch_fm2d_fast(const mct_fm2d_args &a, long chunk, int32_t *pflag, hipStream_t s)
 {
     if (!a.sln) return MCT_ERR_ARG;       // the sweeps read the gridder's slowness
-    int region, heap_cap, win;
-    size_t lds = ff_near_lds(a, region, heap_cap, win);
+    int region, heap_cap;
+    size_t lds = ff_near_lds(a, region, heap_cap);
     int rc = mct_launch_fm2d_gridder(a, s);
     if (rc) return rc;
     if (lds > 64 * 1024)
@@ -2220,9 +2238,9 @@ int mct_launch_fm2d_fast(const mct_fm2d_args &a, long chunk, int32_t *pflag, hip
         b.prob0 = p0;
         b.nrun = nprob - p0 < chunk ? nprob - p0 : chunk;
         if (a.fom == 0)
-            hipLaunchKernelGGL(k_fm2d_near<0>, dim3((unsigned)b.nrun), dim3(64), lds, s, b, region, heap_cap, win, pflag);
+            hipLaunchKernelGGL(k_fm2d_near<0>, dim3((unsigned)b.nrun), dim3(64), lds, s, b, region, heap_cap, pflag);
         else
-            hipLaunchKernelGGL(k_fm2d_near<1>, dim3((unsigned)b.nrun), dim3(64), lds, s, b, region, heap_cap, win, pflag);
+            hipLaunchKernelGGL(k_fm2d_near<1>, dim3((unsigned)b.nrun), dim3(64), lds, s, b, region, heap_cap, pflag);
         MCT_CHECK(hipGetLastError());
         if (a.ev_sweep && p0 == 0) MCT_CHECK(hipEventRecord(a.ev_sweep, s));
         if (strip_lds && a.fom == 0)
