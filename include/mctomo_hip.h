@@ -470,14 +470,15 @@ int mct_surf_split_parts(mct_surf_ctx *ctx, int nchain, int *first_part_chains);
  * source (default), 1 the sequential heap loop per (period, source). */
 int mct_surf_set_method(mct_surf_ctx *ctx, int fm2d_method);
 
-/* Dispersion launch shape: 0 by size (default), 1 one lane per column
- * (throughput), 2 one wave per column (latency), 3 one lane per column with
- * columns taken from a queue in layer-count order.  Results are the same. */
+/* Dispersion launch shape: 0 default (3), 1 one lane per column
+ * (throughput), 2 one wave per column (latency), 3 columns taken from a queue
+ * in layer-count order, one lane each or, where they are few, up to 64.  Results
+ * are the same. */
 int mct_surf_set_dispersion_mode(mct_surf_ctx *ctx, int mode);
 
 /* Launch shape of a context, for tuning (no counterpart in the reference;
  * results do not depend on it): MCT_TUNE_DSP_WAVES waves of the queue
- * dispersion kernel (0: one per 64 columns), MCT_TUNE_SWEEP_KIND the 2-D
+ * dispersion kernel at most (0: no limit), MCT_TUNE_SWEEP_KIND the 2-D
  * sweep (0 default, 1 strip-pipelined, 2 anti-diagonal), MCT_TUNE_SWEEP_THREADS
  * threads per problem of the anti-diagonal sweep (0 default, 64, 128, 256),
  * MCT_TUNE_FM2D_CHUNK 2-D problems per launch (0: all the workspace holds),
