@@ -722,7 +722,10 @@ __global__ __launch_bounds__(64) void k_sfmm_lds(sfl_args S)
     int hs = 0;                                       // heap entries
     int nb = 0;                                       // slots ever used
     int fh = -1;                                      // head of the free list
-    // push_heap (as in k_sfmm): lane j - 1 holds the ancestor j levels up
+    // push_heap (as in k_sfmm): lane j - 1 holds the ancestor j levels up.  The other
+    // lanes read entry 0 and its key too, so entry 0 names a slot before the first push.
+    if (lane == 0) H[0] = 0;
+    wave_sync();
     auto push = [&](int slot, double kc) {
         const int k1 = (int)first_u((uint32_t)hs) + 1;
         hs = k1;

@@ -158,3 +158,19 @@ def test_heap_replay_by_size(shape, h, where):
         to, fo = po.fast_marching_3d(vel, h[0], h[1], h[2], 0, 0, 0, src, rev, 1, field=True)
         assert np.array_equal(fg, fo)
         np.testing.assert_allclose(tg, to, rtol=1e-12)
+
+
+def test_heap_replays_of_different_sizes_in_turn():
+    """A replay starts on whatever the kernel before it left in LDS: after one whose
+    tables fill the LDS, grids of a few cells and of a few thousand give the
+    oracle's fields bit for bit, each the same when it runs first."""
+    runs = []
+    for shape, ncell, seed in (((64, 48, 40), 120, 8), ((3, 4, 5), 3, 2), ((21, 21, 21), 30, 1)):
+        vel, ext, rng = _voronoi(shape, (0.2, 0.2, 0.2), ncell, seed)
+        src, rev = rng.uniform(0, 1, 3) * ext, rng.uniform(0, 1, (4, 3)) * ext
+        runs.append((vel, src, rev, po.fast_marching_3d(vel, 0.2, 0.2, 0.2, 0, 0, 0, src, rev, 1, field=True)[1]))
+    for k in (1, 0, 1, 2, 0, 2, 1):
+        vel, src, rev, fo = runs[k]
+        say("heap replays in turn", vel.shape)
+        fg = mct.fast_marching_3d(vel, 0.2, 0.2, 0.2, 0, 0, 0, src, rev, 1, field=True)[1]
+        np.testing.assert_array_equal(fg, fo)
