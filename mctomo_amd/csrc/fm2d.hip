@@ -971,10 +971,9 @@ __device__ static int w_travel(wave_grid &G, double scx, double scz, int urg)
         // (the popped node is alive; its state is stored below)
         double tv = ix1 && iz1 ? w_quadrant<FOM>(sj1 == 0 || ox1 == oP, ix2 && sj2 == 0, sk1 == 0 || oz1 == oP,
                                                  iz2 && sk2 == 0, tj1, tj2, tk1, tk2, slown, G.dnx, G.dnz)
-                               : W_NONE;
+                               : __builtin_nan("");
         tv = fmin(tv, w_quad_d<0xb1>(tv));
         tv = fmin(tv, w_quad_d<0x4e>(tv));
-        if (tv >= W_NONE) tv = 0.0;          // no quadrant: the reference's travm stays 0
         // the states the pop changed, then the neighbours enter the heap one after another
         if (G.lead) {
             G.s[oP] = 0;

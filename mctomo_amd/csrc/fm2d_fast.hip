@@ -1026,14 +1026,13 @@ __device__ __forceinline__ void ff_heap_loop(const fview &V, ff_heap &H, const V
         const int ox1 = ix1 ? o + ddx * V.ld : o, ox2 = ix2 ? o + 2 * ddx * V.ld : o;
         const int oz1 = iz1 ? o + ddz : o, oz2 = iz2 ? o + 2 * ddz : o;
         const int st = in ? (int)V.ns[o] : 0;
-        double tv = W_NONE;
+        double tv = __builtin_nan("");
         if (ix1 && iz1)
             tv = w_quadrant<FOM>(V.ns[ox1] == 0, ix2 && V.ns[ox2] == 0, V.ns[oz1] == 0, iz2 && V.ns[oz2] == 0,
                                  V.T[ox1], FOM ? V.T[ox2] : 0.0, V.T[oz1], FOM ? V.T[oz2] : 0.0, 1.0 / vz, V.dnx,
                                  V.dnz);
         tv = fmin(tv, w_quad_d<0xb1>(tv));
         tv = fmin(tv, w_quad_d<0x4e>(tv));
-        if (tv >= W_NONE) tv = 0.0;          // no quadrant: the reference's travm stays 0
 #pragma unroll
         for (int k = 0; k < 4; k++) {
             const int stk = __builtin_amdgcn_readlane(st, 4 * k);

@@ -30,8 +30,9 @@ __device__ __forceinline__ double w_quad_d(double v)
 
 // One quadrant of fouds1 (fm2d_ttime.f90:248-332) or fouds2 (:342-518): tj, tk the
 // x and z neighbours' times, tj2, tk2 the ones behind them, a* whether alive.
-// Returns W_NONE when neither neighbour is alive.
-#define W_NONE 1e300
+// Returns a NaN when neither neighbour is alive: the minimum over the quadrants leaves
+// it out.  A node next to a popped one always has a quadrant with a time.  Where
+// the velocity is 0 the slowness, and with it the time, is infinite.
 template <int FOM>
 __device__ __forceinline__ double w_quadrant(bool aj, bool aj2, bool ak, bool ak2, double tj, double tj2, double tk,
                                              double tk2, double slown, double dnx, double dnz)
@@ -80,14 +81,14 @@ __device__ __forceinline__ double w_quadrant(bool aj, bool aj2, bool ak, bool ak
         tref = K ? 4.0 * tk - tk2 : tk;
         tdiv = K ? 3.0 : 1.0;
     } else {
-        return W_NONE;
+        return __builtin_nan("");
     }
     double rd1 = b * b - 4.0 * a * c;
     if (rd1 < 0.0) rd1 = 0.0;
-    const double tdsh = fp_div(-b + fp_sqrt(rd1), 2.0 * a);
+    const double tdsh = fp_div_any(-b + fp_sqrt(rd1), 2.0 * a);
     const double trav = tref + tdsh;
     if (FOM == 0 || tdiv == 1.0) return trav;
-    return fp_quot(trav, 3.0, fp_recip(3.0));
+    return fp_div_any(trav, 3.0);
 }
 
 } // namespace

@@ -10,9 +10,10 @@
 // correctly rounded results.  Quotients with one denominator share its refined
 // reciprocal, so each further one costs three instructions.
 //
-// They hold for finite arguments with 2^-700 < |n|, |d|, |n/d| < 2^700, or n = 0 (whose
-// sign is not kept), and for x = 0 or 2^-700 < x < 2^700.  On the host they are the
-// plain operations.
+// Quotients hold for finite arguments with 2^-700 < |n|, |d|, |n/d| < 2^700, or n = 0
+// (whose sign is not kept); fp_div_any's n may also be infinite or a NaN.  Square
+// roots hold for x = 0, 2^-700 < x < 2^700, +inf and NaN.  On the host they are the plain
+// operations.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <math.h>
@@ -43,6 +44,17 @@ __host__ __device__ __forceinline__ double fp_quot(double n, double d, double y)
 
 __host__ __device__ __forceinline__ double fp_div(double n, double d) { return fp_quot(n, d, fp_recip(d)); }
 
+// n / d where n may be infinite or a NaN: the division's last step, one instruction,
+// which replaces the quotient in these cases
+__host__ __device__ __forceinline__ double fp_div_any(double n, double d)
+{
+#ifdef __HIP_DEVICE_COMPILE__
+    return __builtin_amdgcn_div_fixup(fp_div(n, d), d, n);
+#else
+    return n / d;
+#endif
+}
+
 // sqrt(x), x >= 0
 __host__ __device__ __forceinline__ double fp_sqrt(double x)
 {
@@ -54,7 +66,7 @@ __host__ __device__ __forceinline__ double fp_sqrt(double x)
     h = __builtin_fma(h, e, h);
     g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
     g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
-    return x == 0.0 ? 0.0 : g;                    // rsq(0) is infinite
+    return __builtin_amdgcn_class(x, 0x260) ? x : g;   // +-0 and +inf, where x * rsq(x) is a NaN
 #else
     return sqrt(x);
 #endif

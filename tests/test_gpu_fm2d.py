@@ -355,3 +355,30 @@ def test_strip_sweep_on_columns_around_its_load_groups(nx, nz, monkeypatch):
             np.testing.assert_array_equal(got, want)
             for p in range(3):
                 agree(got[p], po.fm2d(velv[p], 0, 0, h, h, sx, sz, rx, rz, fom=fom, asgr=asgr), 0)
+
+
+@pytest.mark.parametrize("asgr", [0, 1])
+@pytest.mark.parametrize("fom", [0, 1])
+@pytest.mark.parametrize("split", ["0", "1000000"])
+def test_nodes_of_velocity_zero(fom, asgr, split, monkeypatch):
+    """Grids with a block of velocity 0, where slowness and times are infinite: sources
+    inside the block, beside it and away from it, receivers all over.  The finite
+    times are the oracle's (method 1: every time, bit for bit), the others stay
+    without a finite time."""
+    monkeypatch.setenv("MCT_WAVE_SPLIT", split)
+    for seed in (1, 2, 3):
+        rng = np.random.default_rng(seed)
+        velv = rng.uniform(2.5, 3.5, (18, 16))
+        velv[6:11, 5:10] = 0
+        rx, rz = rng.uniform(0, 7.5, 9), rng.uniform(0, 6.5, 9)
+        sx = np.r_[rng.uniform(0.5, 7, 3), 2.4, 2.5, 4.6]
+        sz = np.r_[rng.uniform(0.5, 6, 3), 2.2, 3.0, 3.1]
+        say("velocity zero", seed, "fom", fom, "asgr", asgr, "split", split)
+        want = po.fm2d(velv, 0, 0, 0.5, 0.5, sx, sz, rx, rz, fom=fom, asgr=asgr)
+        m = np.isfinite(want)
+        assert np.count_nonzero(~m) < want.size // 3
+        seq = mct.modrays(velv, 0, 0, 0.5, 0.5, sx, sz, rx, rz, fom=fom, asgr=asgr, method=1)
+        np.testing.assert_array_equal(seq, want)
+        got = mct.modrays(velv, 0, 0, 0.5, 0.5, sx, sz, rx, rz, fom=fom, asgr=asgr, method=0)
+        np.testing.assert_allclose(got[m], want[m], rtol=1e-9, atol=0)
+        assert not np.any(np.abs(got[~m]) < 1e30)      # 1e38 stands for a node not reached
