@@ -572,10 +572,12 @@ __host__ __device__ __forceinline__ double ff_cands0_all(double x0, double x1, d
 __host__ __device__ __forceinline__ bool ff_cands0_min(double x0, double x1, double z0, double z1, const ff_k0 &K,
                                                        double slown, double &c)
 {
-    const double a = x0 < x1 ? x0 : x1, b = z0 < z1 ? z0 : z1;
-    const double ga = (x0 < x1 ? x1 : x0) - a, gb = (z0 < z1 ? z1 : z0) - b;
+    // a neighbour whose time is a NaN is left out, as an absent one; where both of an axis
+    // are, q below is a NaN and every quadrant is evaluated
+    const double a = fp_min(x0, x1), b = fp_min(z0, z1);
+    const double ga = fp_max(x0, x1) - a, gb = fp_max(z0, z1) - b;
     const bool ax = a <= b;
-    const double lo = ax ? a : b, hi = ax ? b : a;
+    const double lo = fp_min(a, b), hi = fp_max(a, b);
     c = FF_BIG;
     if (!(lo < FF_FIN)) return true;
     const double ss = slown * slown, sdz = slown * K.dnz;

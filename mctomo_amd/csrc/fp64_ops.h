@@ -55,6 +55,29 @@ __host__ __device__ __forceinline__ double fp_div_any(double n, double d)
 #endif
 }
 
+// the smaller and the larger of two numbers, the other one where one is a NaN, by one
+// instruction (fmin and fmax put canonicalising ones before it)
+__host__ __device__ __forceinline__ double fp_min(double a, double b)
+{
+#ifdef __HIP_DEVICE_COMPILE__
+    double r;
+    asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+#else
+    return fmin(a, b);
+#endif
+}
+__host__ __device__ __forceinline__ double fp_max(double a, double b)
+{
+#ifdef __HIP_DEVICE_COMPILE__
+    double r;
+    asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+#else
+    return fmax(a, b);
+#endif
+}
+
 // sqrt(x), x >= 0
 __host__ __device__ __forceinline__ double fp_sqrt(double x)
 {

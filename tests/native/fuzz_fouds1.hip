@@ -19,13 +19,17 @@ int mct_fill_i32(int32_t *, long, int32_t, hipStream_t) { return 0; }
 int main(int argc, char **argv)
 {
     const long n = argc > 1 ? atol(argv[1]) : 1000000;
+    // "special": some times NaN or infinite, some slownesses infinite, NaN or 0
+    const bool special = argc > 2 && strcmp(argv[2], "special") == 0;
+    const double odd[] = {__builtin_nan(""), __builtin_huge_val(), FF_BIG, 0.0};
     std::mt19937_64 rng(20261202);
     std::uniform_real_distribution<double> U(0.0, 1.0);
     const double dns[] = {0.5, 0.25, 1.0, 0.125, 0.7, 1.0 / 3.0};
     long bad = 0, far = 0;
     for (long it = 0; it < n; it++) {
         const double dnx = dns[rng() % 6], dnz = dns[rng() % 6];
-        const double slown = 1.0 / (1.5 + 4.0 * U(rng));
+        double slown = 1.0 / (1.5 + 4.0 * U(rng));
+        if (special && rng() % 4 == 0) slown = odd[rng() % 4];
         const double base = 100.0 * U(rng);
         ff_sten S;
         for (int s = 0; s < 2; s++) {
@@ -39,10 +43,14 @@ int main(int argc, char **argv)
             if (!S.ix1[s]) S.tx1[s] = FF_BIG;
             if (!S.iz1[s]) S.tz1[s] = FF_BIG;
             S.tx2[s] = S.tz2[s] = FF_BIG;
+            if (special && rng() % 3 == 0 && S.ix1[s]) S.tx1[s] = odd[rng() % 4];
+            if (special && rng() % 3 == 0 && S.iz1[s]) S.tz1[s] = odd[rng() % 4];
         }
         const double a = ff_cands<0>(S, dnx, dnz, slown);
         const double b = ff_cands0f(S, ff_k0_make(dnx, dnz), slown);
         if (a >= FF_THR0) far++;
+        // a special stencil's result counts where it is a time
+        if (special && !(a < FF_THR0) && !(b < FF_THR0)) continue;
         if (memcmp(&a, &b, sizeof a) != 0) {
             if (bad < 5) printf("mismatch %.17g %.17g\n", a, b);
             bad++;
