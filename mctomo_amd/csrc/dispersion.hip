@@ -134,22 +134,59 @@ __device__ static float d_gtsolh(float a, float b)
 }
 
 // Division, square root and the quotients of one denominator, y = dsp_rcp(d):
-// with NORM the operands are known to be far from the ends of the exponent range
-// (dsp_in_range) and fp64_ops.h's shorter forms give the same bits.
-template <bool NORM> __device__ __forceinline__ double dsp_rcp(double d) { return NORM ? fp_recip(d) : 0.0; }
-template <bool NORM> __device__ __forceinline__ double dsp_quot(double n, double d, double y)
+// with NORM the operands are far from the ends of the exponent range (dsp_in_range,
+// dsp_normal) and fp64_ops.h's shorter forms give the same bits.
+template <bool NORM> __host__ __device__ __forceinline__ double dsp_rcp(double d) { return NORM ? fp_recip(d) : 0.0; }
+template <bool NORM> __host__ __device__ __forceinline__ double dsp_quot(double n, double d, double y)
 {
     return NORM ? fp_quot(n, d, y) : n / d;
 }
-template <bool NORM> __device__ __forceinline__ double dsp_div(double n, double d)
+template <bool NORM> __host__ __device__ __forceinline__ double dsp_div(double n, double d)
 {
     return NORM ? fp_div(n, d) : n / d;
 }
-template <bool NORM> __device__ __forceinline__ double dsp_sqrt(double x) { return NORM ? fp_sqrt(x) : sqrt(x); }
+template <bool NORM> __host__ __device__ __forceinline__ double dsp_sqrt(double x) { return NORM ? fp_sqrt(x) : sqrt(x); }
 
-// SH period equation, dltar1 (surfdisp96.f:1056-1115)
+// the smaller / larger of |a| and |x| (the other one where one is a NaN)
+__host__ __device__ __forceinline__ double dsp_min_abs(double a, double x)
+{
+#ifdef __HIP_DEVICE_COMPILE__
+    double r;
+    asm("v_min_f64 %0, |%1|, |%2|" : "=v"(r) : "v"(a), "v"(x));
+    return r;
+#else
+    return fmin(fabs(a), fabs(x));
+#endif
+}
+__host__ __device__ __forceinline__ double dsp_max_abs(double a, double x)
+{
+#ifdef __HIP_DEVICE_COMPILE__
+    double r;
+    asm("v_max_f64 %0, |%1|, |%2|" : "=v"(r) : "v"(a), "v"(x));
+    return r;
+#else
+    return fmax(fabs(a), fabs(x));
+#endif
+}
+
+// 2^-20 <= x <= 2^20: earth models in km and in m.  With layers, periods and trial
+// velocities in this range wvno lies in 2^+-40, a layer's ra and rb in 2^-67..2^41 or
+// at 0, w and y at most at 2^20, gam and gammk in 2^+-81.  So the quotients and
+// square roots of a layer lie in 2^+-500 and the vector that it hands on below 2^612 (P-SV,
+// the second-lowest layer; 2^448 above it) or 2^142 (SH); how small that vector's
+// components get is looked at as they come (dsp_normal).
+template <class T> __host__ __device__ __forceinline__ bool dsp_in_range(T x) { return x >= (T)0x1p-20 && x <= (T)0x1p20; }
+
+// lo, the smallest component of the vector that a layer hands on, lies where the
+// normalised components (at least lo / 2^612) and the next SH layer's quotient (one
+// of them times 2^-101, over 2^60) stay above 2^-900.  Where not, a component that
+// is 0 among them, the caller evaluates with plain divisions.
+__host__ __device__ __forceinline__ bool dsp_normal(double lo) { return lo >= 0x1p-280; }
+
+// SH period equation, dltar1 (surfdisp96.f:1056-1115); with NORM, ok is cleared where
+// the short forms may not hold
 template <bool NORM, class MD>
-__device__ static double d_dltar1(double wvno, double omega, const MD &M)
+__host__ __device__ static double d_dltar1(double wvno, double omega, const MD &M, bool &ok)
 {
     double beta1 = (double)M.b[M.st * (M.mmax - 1)];
     double rho1 = (double)M.rho[M.st * (M.mmax - 1)];
@@ -188,6 +225,7 @@ __device__ static double d_dltar1(double wvno, double omega, const MD &M)
         double e10 = e1 * cosq + e2 * xmu * z;
         double e20 = dsp_div<NORM>(e1 * y, xmu) + e2 * cosq;
         double xnor = fabs(e10), ynor = fabs(e20);
+        if (NORM) ok &= dsp_normal(dsp_min_abs(e10, e20));
         if (ynor > xnor) xnor = ynor;
         if (xnor < 1.0e-40) xnor = 1.0;
         const double rnor = dsp_rcp<NORM>(xnor);
@@ -197,9 +235,10 @@ __device__ static double d_dltar1(double wvno, double omega, const MD &M)
     return e1;
 }
 
-// P-SV period equation, dltar4 with var and dnka inlined (surfdisp96.f:1119-1414)
+// P-SV period equation, dltar4 with var and dnka inlined (surfdisp96.f:1119-1414); ok
+// as in d_dltar1
 template <bool NORM, class MD>
-__device__ static double d_dltar4(double wvno, double omga, const MD &M)
+__host__ __device__ static double d_dltar4(double wvno, double omga, const MD &M, bool &ok)
 {
     double omega = omga;
     if (omega < 1.0e-4) omega = 1.0e-4;
@@ -324,13 +363,9 @@ __device__ static double d_dltar4(double wvno, double omga, const MD &M)
         ee3 = ee3 + e0 * c14; ee3 = ee3 + e1 * c24; ee3 = ee3 + e2 * c34; ee3 = ee3 + e3 * c44; ee3 = ee3 + e4 * c54;
         ee4 = ee4 + e0 * c15; ee4 = ee4 + e1 * c25; ee4 = ee4 + e2 * c35; ee4 = ee4 + e3 * c45; ee4 = ee4 + e4 * c55;
         // ---- normc
-        double t1 = 0.0;
-        if (fabs(ee0) > t1) t1 = fabs(ee0);
-        if (fabs(ee1) > t1) t1 = fabs(ee1);
-        if (fabs(ee2) > t1) t1 = fabs(ee2);
-        if (fabs(ee3) > t1) t1 = fabs(ee3);
-        if (fabs(ee4) > t1) t1 = fabs(ee4);
-        if (t1 < 1.0e-40) t1 = 1.0;
+        double t1 = dsp_max_abs(dsp_max_abs(dsp_max_abs(ee0, ee1), dsp_max_abs(ee2, ee3)), ee4);
+        if (NORM) ok &= dsp_normal(dsp_min_abs(dsp_min_abs(dsp_min_abs(ee0, ee1), dsp_min_abs(ee2, ee3)), ee4));
+        if (!(t1 >= 1.0e-40)) t1 = 1.0;      // (also where all are NaN)
         const double rt1 = dsp_rcp<NORM>(t1);
         e0 = dsp_quot<NORM>(ee0, t1, rt1);
         e1 = dsp_quot<NORM>(ee1, t1, rt1);
@@ -361,10 +396,16 @@ __device__ static double d_dltar4(double wvno, double omga, const MD &M)
     return e0;
 }
 
-template <bool NORM = false, class MD>
+template <bool NORM, class MD>
+__host__ __device__ __forceinline__ double d_dltar(double wvno, double omega, int ifunc, const MD &M, bool &ok)
+{
+    return ifunc == 1 ? d_dltar1<NORM>(wvno, omega, M, ok) : d_dltar4<NORM>(wvno, omega, M, ok);
+}
+template <class MD>
 __device__ __forceinline__ double d_dltar(double wvno, double omega, int ifunc, const MD &M)
 {
-    return ifunc == 1 ? d_dltar1<NORM>(wvno, omega, M) : d_dltar4<NORM>(wvno, omega, M);
+    bool ok = true;
+    return d_dltar<false>(wvno, omega, ifunc, M, ok);
 }
 
 // nevill (surfdisp96.f:903-1020), run identically by every lane of the wave
@@ -980,10 +1021,6 @@ __global__ void k_dsp_queue_reset(unsigned long long *q)
     if (threadIdx.x == 0) q[0] = 0ull;
 }
 
-// 2^-40 <= x <= 2^40.  Layers, periods and trial velocities in this range keep the
-// period equations' quotients and square roots within 2^-700..2^700 (or at 0).
-template <class T> __device__ __forceinline__ bool dsp_in_range(T x) { return x >= (T)0x1p-40 && x <= (T)0x1p40; }
-
 // Lanes per column, as a power of two: as many as keep the columns' waves within
 // wave_target (0: one lane per column), 16 per CU where 12 are resident at once:
 // with fewer lanes the chain of evaluations bounds the call, with more the
@@ -1073,8 +1110,9 @@ __global__ __launch_bounds__(64, 3) void k_dispersion_sm(mct_dsp_args A, float *
         node = 1;
     };
 
+    bool redo = false;
     for (;;) {
-        bool need = false;
+        bool need = redo;
         while (!need && pc != SM_DONE) {
             switch (pc) {
             case SM_NEXT: {
@@ -1327,8 +1365,17 @@ __global__ __launch_bounds__(64, 3) void k_dispersion_sm(mct_dsp_args A, float *
         if (__builtin_amdgcn_ballot_w64(need) == 0ull) break;     // every lane has run out of columns
         if (need) {
             const double wvno = omega / ceval;
-            if (norm && dsp_in_range(ceval) && dsp_in_range(omega)) res = d_dltar<true>(wvno, omega, IFUNC, M);
-            else res = d_dltar(wvno, omega, IFUNC, M);
+            bool ok = true;
+            if (norm && dsp_in_range(ceval) && dsp_in_range(omega)) {
+                res = d_dltar<true>(wvno, omega, IFUNC, M, ok);
+                ok &= res == res;                  // a NaN takes its sign from the plain forms
+            } else {
+                res = d_dltar(wvno, omega, IFUNC, M);
+            }
+            // the short forms left their range: again, and the column's other points, without
+            redo = !ok;
+            if (GROUPED) redo = (__builtin_amdgcn_ballot_w64(redo) & gmask) != 0;
+            if (redo) norm = false;
         }
     }
 }

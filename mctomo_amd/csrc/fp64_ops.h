@@ -10,10 +10,10 @@
 // correctly rounded results.  Quotients with one denominator share its refined
 // reciprocal, so each further one costs three instructions.
 //
-// Quotients hold for finite arguments with 2^-700 < |n|, |d|, |n/d| < 2^700, or n = 0
-// (whose sign is not kept); fp_div_any's n may also be infinite or a NaN.  Square
-// roots hold for x = 0, 2^-700 < x < 2^700, +inf and NaN.  On the host they are the plain
-// operations.
+// Quotients hold for finite arguments with 2^-900 < |n|, |d|, |n/d| < 2^900, where all
+// residuals are normal numbers, or n = 0 (whose sign is not kept); fp_div_any's n may
+// also be infinite or a NaN.  Square roots hold for x = 0, 2^-900 < x < 2^900, +inf and
+// NaN.  On the host they are the plain operations.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <math.h>

@@ -214,3 +214,21 @@ def test_columns_outside_the_short_forms_range(dz, pmin, iw, igr):
     got = mct.dispersion_columns(vs, dz, per, iw, igr, mode=3)
     for g, w in zip(got[:3], want[:3]):
         np.testing.assert_array_equal(g, w)
+
+
+@pytest.mark.parametrize("ncol,iw,igr", [(130, 1, 0), (130, 1, 1), (130, 2, 0), (132000, 1, 0)])
+def test_columns_that_leave_the_short_forms_on_the_way(ncol, iw, igr):
+    """A slow layer so thick against the shortest period that from its velocity on the
+    phase in it is beyond the sine's range (1e8) and the period equation no number:
+    the queue kernel, which starts such a column with the short forms (64 lanes a
+    column, and one), takes the point again without them.  The lane kernel's results,
+    bit for bit."""
+    rng = np.random.default_rng(5 + iw)
+    vs = np.sort(rng.uniform(1.2, 4.8, (ncol, 4)), axis=1)[:, [2, 0, 1, 3]]
+    vs[1::5] = vs[0]
+    per = np.array([1e-3] if ncol > 1000 else [1e-3, 3.0])
+    say("columns that leave the range", ncol, iw, igr)
+    want = mct.dispersion_columns(vs, 3e5, per, iw, igr, mode=1)
+    got = mct.dispersion_columns(vs, 3e5, per, iw, igr, mode=3)
+    for g, w in zip(got[:3], want[:3]):
+        np.testing.assert_array_equal(g, w)
