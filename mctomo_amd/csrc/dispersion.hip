@@ -538,7 +538,9 @@ __device__ static int d_getsol(double t1, double &c1io, double clow, double dc, 
 
 
 // One wave per column: check_model, convert_to_layer, surfdisp96.
-__global__ __launch_bounds__(64) void k_dispersion(mct_dsp_args A)
+// Two waves per SIMD, as in the two kernels below: left to itself the compiler takes
+// 286 registers, one wave, and 3,000 Rayleigh columns of 24 nodes 26.8 ms instead of 20.3.
+__global__ __launch_bounds__(64, 2) void k_dispersion(mct_dsp_args A)
 {
     __shared__ float sd[DSP_NMAX + 1], sa[DSP_NMAX + 1], sb[DSP_NMAX + 1], sr[DSP_NMAX + 1];
     __shared__ int s_nl;
@@ -684,7 +686,7 @@ __device__ static int d_getsol_seq(double t1, double &c1io, double clow, double 
 // One lane per column: check_model, convert_to_layer and surfdisp96 for 64
 // columns per wave.  The layer model of lane i is stored at lay + i with a
 // stride of 64 floats (planes d, a, b, rho of nlmax x 64 floats per wave).
-__global__ __launch_bounds__(64) void k_dispersion_lane(mct_dsp_args A, float *lay, int nlmax)
+__global__ __launch_bounds__(64, 2) void k_dispersion_lane(mct_dsp_args A, float *lay, int nlmax)
 {
     const int lane = threadIdx.x;
     const long col = (long)blockIdx.x * 64 + lane;
@@ -1474,7 +1476,9 @@ struct mct_layer_args {
     int32_t *ierr;                // (nmod)
 };
 
-__global__ __launch_bounds__(64) void k_dispersion_layers(mct_layer_args A)
+// (two waves per SIMD: 4,000 Rayleigh models of 5 to 24 layers 29.7 ms, with one wave 35.0;
+// group velocities 48.9 and 60.7)
+__global__ __launch_bounds__(64, 2) void k_dispersion_layers(mct_layer_args A)
 {
     __shared__ float sd[DSP_NMAX * 2], sa[DSP_NMAX * 2], sb[DSP_NMAX * 2], sr[DSP_NMAX * 2];
     const int mod = blockIdx.x, lane = threadIdx.x;
