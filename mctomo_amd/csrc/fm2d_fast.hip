@@ -1689,7 +1689,9 @@ __global__ __launch_bounds__(256) void k_fm2d_sweep(mct_fm2d_args A, int32_t *pf
 // the lines do not stay in the L2 between.  48 chains of 201x201 grids (1440
 // problems, order 0): one 8-byte load a step 128 ms, 4 nodes in two 16-byte loads
 // 83 ms, 8 nodes 71 ms, 12 nodes 81 ms and 16 nodes 79 ms (registers).
-#define FF_PF 8
+// The mixed-order update holds twice the stencil: 8 nodes left it one wave per SIMD (279
+// registers), 320 problems of 201x201 99 ms; with 4 nodes, two waves, 97.
+constexpr int ff_pf(int fom) { return fom == 0 ? 8 : 4; }
 typedef double ff_pair __attribute__((ext_vector_type(2), aligned(8)));
 
 // Lane i takes lane i-1's value (wave_shr:1) / lane i+1's (wave_shl:1) by DPP
@@ -1711,8 +1713,9 @@ __device__ __forceinline__ double ff_from_above(double v)
 }
 
 template <int FOM>
-__global__ __launch_bounds__(64) void k_fm2d_strip(mct_fm2d_args A, int32_t *pflag)
+__global__ __launch_bounds__(64, FOM == 0 ? 3 : 2) void k_fm2d_strip(mct_fm2d_args A, int32_t *pflag)
 {
+    constexpr int FF_PF = ff_pf(FOM);
     extern __shared__ double ff_sld[];
     const long slot = ff_xcd_slot(blockIdx.x, gridDim.x);
     if (pflag[slot] != 0) return;

@@ -27,7 +27,7 @@ def kernels():
 @pytest.mark.skipif(not os.path.exists(LIB), reason="library not built")
 @pytest.mark.parametrize("kernel,count,waves,spilled", [
     ("12k_dispersion12mct_dsp_args", 1, 2, 32), ("17k_dispersion_lane", 1, 2, 48), ("19k_dispersion_layers", 1, 2, 24),
-    ("15k_dispersion_sm", 4, 3, 24)])
+    ("15k_dispersion_sm", 4, 3, 24), ("12k_fm2d_stripILi0E", 1, 3, 0), ("12k_fm2d_stripILi1E", 1, 2, 0)])
 def test_waves_per_simd(kernel, count, waves, spilled):
     found = {k: v for k, v in kernels().items() if kernel in k}
     assert len(found) == count
