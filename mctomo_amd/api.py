@@ -76,7 +76,7 @@ def lib():
                      "mct_body_location_likelihood", "mct_body_location_likelihood_batch_dev",
                      "mct_serve_create_mix", "mct_serve_submit_to", "mct_serve_memory", "mct_surf_device_bytes",
                      "mct_surf_set_tuning", "mct_surf_get_tuning", "mct_surf_likelihood_batch_graph",
-                     "mct_fm2d_last_handover", "mct_surf_fm2d_handover", "mct_dispersion_columns",
+                     "mct_fm2d_last_handover", "mct_sfmm_last_handover", "mct_surf_fm2d_handover", "mct_dispersion_columns",
                      "mct_body_stream", "mct_joint_create", "mct_joint_destroy", "mct_joint_parts",
                      "mct_joint_likelihood", "mct_joint_likelihood_batch_dev", "mct_joint_sync",
                      "mct_body_noise_likelihood_from", "mct_surf_noise_likelihood_from",
@@ -330,6 +330,14 @@ def modrays_last_handover():
     parallel path to the sequential solver."""
     n = ctypes.c_longlong()
     _check(lib().mct_fm2d_last_handover(ctypes.byref(n)), "mct_fm2d_last_handover")
+    return n.value
+
+
+def sfmm_last_handover():
+    """Problems of the calling thread's last order-1 3-D solve whose band outgrew
+    its tables in LDS and which the replay in global memory solved."""
+    n = ctypes.c_longlong()
+    _check(lib().mct_sfmm_last_handover(ctypes.byref(n)), "mct_sfmm_last_handover")
     return n.value
 
 

@@ -167,9 +167,9 @@ int sfmm_solve(const mct_eik_problem_set &E, eik_ws &ws, const double *src_pts, 
         else (void)hipGetLastError();
     }
     if ((rc = mct_launch_sfmm(a, s))) return rc;
-    MCT_CHECK(hipMemcpyAsync(ws.h_count, a.err, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+    MCT_CHECK(hipMemcpyAsync(ws.h_count, a.err, 2 * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
     MCT_CHECK(hipStreamSynchronize(s));
-    return mct_sfmm_status(*ws.h_count);
+    return mct_sfmm_status(ws.h_count);
 }
 
 } // namespace

@@ -172,9 +172,9 @@ extern "C" int fastMarching3D(int nx, int ny, int nz, double dx, double dy, doub
             else (void)hipGetLastError();
         }
         if ((rc = mct_launch_sfmm(a, s))) return rc;
-        MCT_CHECK(hipMemcpyAsync(W.h_count, a.err, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+        MCT_CHECK(hipMemcpyAsync(W.h_count, a.err, 2 * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
         MCT_CHECK(hipStreamSynchronize(s));
-        if ((rc = mct_sfmm_status(*W.h_count))) return rc;
+        if ((rc = mct_sfmm_status(W.h_count))) return rc;
     } else if ((rc = eik_rounds(E, W.h_count, dx, dy, dz, s))) {
         return rc;
     }

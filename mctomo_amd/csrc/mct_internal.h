@@ -149,7 +149,9 @@ struct mct_sfmm_args {
 size_t mct_sfmm_lin_bytes(const mct_geom &G, long nprob, long ncw);
 long mct_sfmm_heap_cap(const mct_geom &G);
 int mct_launch_sfmm(const mct_sfmm_args &a, hipStream_t s);
-int mct_sfmm_status(uint32_t err_bits);
+// The status of a replay from err's two words on the host (error bits, problems handed
+// from the replay in LDS to the one in global memory).
+int mct_sfmm_status(const uint32_t *err);
 // Order 1 replays the heap unless the environment sets MCT_EIK_ORDER1=parallel.
 int mct_default_heap_order1();
 

@@ -907,7 +907,10 @@ __global__ __launch_bounds__(64) void k_sfmm_lds(sfl_args S)
         }
     }
     // a band that outgrew the tables is left to k_sfmm
-    if (lane == 0) S.done[prob] = full ? 0u : 1u;
+    if (lane == 0) {
+        S.done[prob] = full ? 0u : 1u;
+        if (full) atomicAdd(A.err + 1, 1u);
+    }
     if (A.pops && lane == 0) A.pops[prob] = (uint32_t)(pops > 0xffffffffL ? 0xffffffffL : pops);
     if (err && lane == 0) atomicOr(A.err, err);
 }
@@ -959,6 +962,10 @@ static sfl_plan sfl_make_plan(const mct_geom &G, long nprob)
     if (nprob > 2L * per_cu * cus) return P;
     P.ns = (int)(room / per_cu) & ~7;
     if (P.ns > 65528) P.ns = 65528;
+    // MCT_SFMM_SLOTS: at most this many, so that wider bands are handed over
+    const char *e = getenv("MCT_SFMM_SLOTS");
+    const int most = e ? atoi(e) & ~7 : 0;
+    if (most > 0 && P.ns > most) P.ns = most < 64 ? 64 : most;
     P.ne = P.ns + P.ns / 8 + 64;
     P.lds = 12 * (size_t)P.ns + 2 * (size_t)P.ne + (size_t)P.ns;
     while (P.lds * per_cu > (size_t)max_lds && P.ns > 64) {
@@ -983,7 +990,7 @@ int mct_launch_sfmm(const mct_sfmm_args &a0, hipStream_t s)
         a.nsrc_eff < 1 || a.nwave < 1)
         return MCT_ERR_ARG;
     if ((long)a.G.ntiles * MCT_TILE_N > 0xffffffffL) return MCT_ERR_ARG;
-    MCT_CHECK(hipMemsetAsync(a.err, 0, sizeof(uint32_t), s));
+    MCT_CHECK(hipMemsetAsync(a.err, 0, 2 * sizeof(uint32_t), s));
     a.done = nullptr;
     const long ncw = (a.nprob + a.nsrc_eff - 1) / a.nsrc_eff;
     const sfl_plan P = a.order == 1 && a.lin ? sfl_make_plan(a.G, a.nprob) : sfl_plan{0, 0, 0};
@@ -1019,8 +1026,20 @@ int mct_launch_sfmm(const mct_sfmm_args &a0, hipStream_t s)
     return MCT_OK;
 }
 
-int mct_sfmm_status(uint32_t err_bits)
+// problems of the calling thread's last replay whose band outgrew the tables in LDS
+static thread_local long long g_sfmm_handover = 0;
+
+extern "C" int mct_sfmm_last_handover(long long *n)
 {
+    if (!n) return MCT_ERR_ARG;
+    *n = g_sfmm_handover;
+    return MCT_OK;
+}
+
+int mct_sfmm_status(const uint32_t *err)
+{
+    const uint32_t err_bits = err[0];
+    g_sfmm_handover = err[1];
     if (!err_bits) return MCT_OK;
     return (err_bits & SF_ERR_HEAP) ? MCT_ERR_NOMEM : MCT_ERR_NOCONV;
 }

@@ -144,12 +144,12 @@ def test_order1_batch_equals_single_calls():
 
 
 @pytest.mark.parametrize("shape,h,where", [((3, 4, 5), (0.2, 0.2, 0.2), "LDS"), ((24, 2, 9), (0.1, 0.3, 0.2), "LDS"),
-                                           ((70, 66, 64), (0.2, 0.2, 0.1), "LDS or handed over"),
+                                           ((70, 66, 64), (0.2, 0.2, 0.1), "LDS"),
                                            ((90, 88, 86), (0.2, 0.2, 0.2), "global")])
 def test_heap_replay_by_size(shape, h, where):
     """The replay keeps its heap and keys in LDS where the band fits (small grids to
-    about 70^3), hands a band that outgrows them to the replay in global memory, and
-    starts there on larger grids: the fields are the oracle's bit for bit."""
+    about 70^3) and runs in global memory on larger grids: the fields are the
+    oracle's bit for bit, and none of these bands is handed over."""
     vel, ext, rng = _voronoi(shape, h, 12, sum(shape))
     rev = rng.uniform(0, 1, (4, 3)) * ext
     for src in (rng.uniform(0, 1, 3) * ext, ext * [0.5, 0.5, 0.0]):
@@ -158,6 +158,7 @@ def test_heap_replay_by_size(shape, h, where):
         to, fo = po.fast_marching_3d(vel, h[0], h[1], h[2], 0, 0, 0, src, rev, 1, field=True)
         assert np.array_equal(fg, fo)
         np.testing.assert_allclose(tg, to, rtol=1e-12)
+        assert mct.sfmm_last_handover() == 0
 
 
 def test_heap_replays_of_different_sizes_in_turn():
@@ -174,3 +175,44 @@ def test_heap_replays_of_different_sizes_in_turn():
         say("heap replays in turn", vel.shape)
         fg = mct.fast_marching_3d(vel, 0.2, 0.2, 0.2, 0, 0, 0, src, rev, 1, field=True)[1]
         np.testing.assert_array_equal(fg, fo)
+
+
+def test_bands_that_outgrow_their_tables_are_handed_over(monkeypatch):
+    """With fewer slots in LDS than a band has cells the replay leaves the problem, at
+    whatever pop that is, to the one in global memory, which starts from the tiles
+    as they were: the oracle's fields bit for bit."""
+    vel, ext, rng = _voronoi((31, 26, 22), (0.2, 0.25, 0.3), 25, 9)
+    rev = rng.uniform(0, 1, (6, 3)) * ext
+    for src in (rng.uniform(0, 1, 3) * ext, ext * [0.5, 0.5, 0.0], ext.copy()):
+        to, fo = po.fast_marching_3d(vel, 0.2, 0.25, 0.3, 0, 0, 0, src, rev, 1, field=True)
+        handed = []
+        for slots in (64, 256, 512, 65528):
+            monkeypatch.setenv("MCT_SFMM_SLOTS", str(slots))
+            tg, fg = mct.fast_marching_3d(vel, 0.2, 0.25, 0.3, 0, 0, 0, src, rev, 1, field=True)
+            handed.append(mct.sfmm_last_handover())
+            say("slots", slots, "src", src, "handed over", handed[-1])
+            np.testing.assert_array_equal(fg, fo)
+            np.testing.assert_allclose(tg, to, rtol=1e-12, atol=0)
+        assert handed[0] == 1 and handed[-1] == 0
+
+
+def test_a_batch_of_which_some_are_handed_over(monkeypatch):
+    """P and S fields of one call, of which the slots suffice for none, some and all:
+    the same times and likelihood bit for bit."""
+    nsrc, nrev = 9, 40
+    w = body_workload(n=27, h=0.3, ncells=40, nsrc=nsrc, nrev=nrev, datatype=1, seed=17)
+    like = mct.BodyLikelihood(w.grid, w.rev, w.ttime, w.raystat, nsrc, datatype=1, order=1, max_cells=64)
+    rc, out0, pt0, _, _ = like.likelihood(w.points, w.params, w.locations, arrays=True)
+    assert rc == 0 and mct.sfmm_last_handover() == 0
+    handed = []
+    for slots in (64, 400, 600, 800, 1000, 1200, 1400, 65528):
+        monkeypatch.setenv("MCT_SFMM_SLOTS", str(slots))
+        rc, out, pt, _, _ = like.likelihood(w.points, w.params, w.locations, arrays=True)
+        handed.append(mct.sfmm_last_handover())
+        say("slots", slots, "handed over", handed[-1])
+        assert rc == 0
+        np.testing.assert_array_equal(pt, pt0)
+        np.testing.assert_array_equal(out, out0)
+    like.close()
+    assert handed[0] == 2 * nsrc and handed[-1] == 0
+    assert any(0 < n < 2 * nsrc for n in handed) and sorted(handed, reverse=True) == handed
