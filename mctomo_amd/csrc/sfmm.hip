@@ -756,6 +756,10 @@ __global__ __launch_bounds__(64) void k_sfmm_lds(sfl_args S)
         }
         wave_sync();
         push(slot, tc[v]);
+        // A source on a node of velocity 0 has a NaN among its corners' times.  The
+        // ballots below compare a path's entries all at once, which puts NaN keys
+        // elsewhere than the loop does: such a problem is left to k_sfmm too.
+        full |= !(tc[v] < sf_inf());
     }
 
     // a lane's place in a block of five levels under the hole, and its ancestors there
@@ -906,7 +910,7 @@ __global__ __launch_bounds__(64) void k_sfmm_lds(sfl_args S)
             push(slot, tn);
         }
     }
-    // a band that outgrew the tables is left to k_sfmm
+    // a band that outgrew the tables, or had a key that is no number, is left to k_sfmm
     if (lane == 0) {
         S.done[prob] = full ? 0u : 1u;
         if (full) atomicAdd(A.err + 1, 1u);
@@ -1026,7 +1030,7 @@ int mct_launch_sfmm(const mct_sfmm_args &a0, hipStream_t s)
     return MCT_OK;
 }
 
-// problems of the calling thread's last replay whose band outgrew the tables in LDS
+// problems that the calling thread's last replay in LDS left to k_sfmm
 static thread_local long long g_sfmm_handover = 0;
 
 extern "C" int mct_sfmm_last_handover(long long *n)

@@ -216,3 +216,26 @@ def test_a_batch_of_which_some_are_handed_over(monkeypatch):
     like.close()
     assert handed[0] == 2 * nsrc and handed[-1] == 0
     assert any(0 < n < 2 * nsrc for n in handed) and sorted(handed, reverse=True) == handed
+
+
+@pytest.mark.parametrize("seed", [73, 112, 424, 676, 700, 848, 1292, 0, 8, 16])
+def test_source_on_a_node_of_velocity_zero(seed):
+    """The source's own corner then has a NaN for a time (0 / 0), corners of the block of
+    velocity 0 around it infinite ones, and the heap is ordered by comparisons with
+    them, which the ballots over a path do not reproduce: the oracle's fields bit for
+    bit, or no convergence where a cell is left without a finite update."""
+    rng = np.random.default_rng(seed)
+    sh = rng.integers(4, 16, 3)
+    v = rng.uniform(2, 6, sh)
+    n = rng.integers(1, sh) if seed % 4 else np.where(rng.random(3) < 0.7, sh - 1, rng.integers(0, sh))
+    lo, hi = np.maximum(n - rng.integers(0, 3, 3), 0), n + 1 + rng.integers(0, 2, 3)
+    v[lo[0]:hi[0], lo[1]:hi[1], lo[2]:hi[2]] = 0
+    say("source on a zero node", seed, sh, n)
+    fo = po.fast_marching_3d(v, 0.25, 0.25, 0.25, 0, 0, 0, n * 0.25, np.zeros((1, 3)), 1, field=True)[1]
+    try:
+        fg = mct.fast_marching_3d(v, 0.25, 0.25, 0.25, 0, 0, 0, n * 0.25, np.zeros((1, 3)), 1, field=True)[1]
+    except mct.MCTError:
+        assert not np.isfinite(fo[v > 0]).all()
+    else:
+        np.testing.assert_array_equal(fg, fo)
+    assert mct.sfmm_last_handover() == 1
