@@ -2156,12 +2156,12 @@ static size_t ff_near_lds(const mct_fm2d_args &a, int &region, int &heap_cap)
 int mct_fm2d_fast_ok(const mct_fm2d_args &a)
 {
     int region, heap_cap;
-    const size_t wn = a.asgr == 1 ? 2 * (size_t)a.sgs + 1 : 1;
-    // The region with room to spare for a second byte per state, 32-bit heap entries
-    // and the window: beyond this line a problem would have a CU to itself, and the
-    // sequential solver takes it.  Heap entries and coordinates are 16-bit.
-    size_t b = ff_near_lds(a, region, heap_cap);
-    b += (size_t)region + 2 * (size_t)(heap_cap + 2) + 10 * wn * wn + 64;
+    // What k_fm2d_near needs, with its static words, has to fit a work-group's LDS
+    // (131 x 131 refined nodes do); a larger window goes to the sequential solver, one
+    // lane per problem: 40 problems of 101x101 grids with 127 x 127 refined nodes
+    // 411 ms, here 6.2, and 1,024 of them 587 and 15.7.  Heap entries and coordinates
+    // are 16-bit.
+    const size_t b = ff_near_lds(a, region, heap_cap) + 64;
     static int lds_max = 0;
     if (!lds_max) {
         int dev = 0, v = 0;

@@ -382,3 +382,23 @@ def test_nodes_of_velocity_zero(fom, asgr, split, monkeypatch):
         got = mct.modrays(velv, 0, 0, 0.5, 0.5, sx, sz, rx, rz, fom=fom, asgr=asgr, method=0)
         np.testing.assert_allclose(got[m], want[m], rtol=1e-9, atol=0)
         assert not np.any(np.abs(got[~m]) < 1e30)      # 1e38 stands for a node not reached
+
+
+@pytest.mark.parametrize("sgs,sgdl,parallel", [(9, 7, True), (8, 8, True), (13, 5, True), (11, 6, False)])
+def test_refined_windows_up_to_what_lds_holds(sgs, sgdl, parallel, monkeypatch):
+    """Refined windows of 127 to 131 nodes a side, the largest that the near-source
+    kernel holds, and 133, which the sequential solver takes: the oracle's times,
+    and on the sequential side bit for bit."""
+    rng = np.random.default_rng(10 * sgs + sgdl)
+    n, h = 41, 0.5
+    velv = rng.uniform(2.4, 3.8, (n + 2, n + 2))
+    L = (n - 1) * h
+    sx, sz = np.r_[rng.uniform(h, L - h, 4), L / 2], np.r_[rng.uniform(h, L - h, 4), L / 2]
+    rx, rz = rng.uniform(0, L, 12), rng.uniform(0, L, 12)
+    monkeypatch.setenv("MCT_FM2D_ORDER1", "check")   # fom 1 takes the near-source kernel too
+    for fom in (0, 1):
+        say("refined window", 2 * sgs * sgdl + 1, "fom", fom)
+        kw = dict(fom=fom, asgr=1, sgs=sgs, sgdl=sgdl)
+        got = mct.modrays(velv, 0, 0, h, h, sx, sz, rx, rz, method=0, **kw)
+        want = po.fm2d(velv, 0, 0, h, h, sx, sz, rx, rz, **kw)
+        agree(got, want, 0 if parallel else 1)
