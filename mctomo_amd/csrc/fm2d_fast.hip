@@ -947,12 +947,12 @@ __device__ __forceinline__ double ff_bilinear(const double nv[2][2], double dsx,
 
 // Heap-loop stop rules.
 struct ff_stop {
-    int mode;                 // 0 none, 1 refined inner-edge exit, 2 block frozen, 3 two generations,
-                              // 4 the exit rule, then the block rule
-    int vnl, vnr, vnt, vnb;   // refined-grid bookkeeping (mode 1)
-    int x0, x1, z0, z1;       // block (mode 2)
+    int mode;                 // 2 block frozen, 3 two generations, 4 a popped node at an inner edge of
+                              // the refined grid, then the block rule
+    int vnl, vnr, vnt, vnb;   // refined-grid bookkeeping (mode 4)
+    int x0, x1, z0, z1;       // block (modes 2 and 4)
     int need, have;
-    int exited;               // mode 1: exit node reached
+    int exited;               // mode 4: exit node reached
     int overflow;             // a node outside the LDS storage would be touched
     uint32_t *gen_bits;       // mode 3: nodes of the two generations (bit per stored node)
     int gen;                  // mode 3: 0 first generation, 1 second
@@ -992,7 +992,7 @@ __device__ __forceinline__ void ff_heap_loop(const fview &V, ff_heap &H, const V
         }
         const int er = __builtin_amdgcn_readfirstlane((int)H.btg[1]);
         const int qx = (int)__umulhi((unsigned)er, mag), ix = qx + V.ox + 1, iz = er - qx * V.ld + V.oz + 1;
-        if (S.mode == 1 || S.mode == 4) {
+        if (S.mode == 4) {
             int swrg = 0;
             if (ix == 1 && S.vnl != 1) swrg = 1;
             if (ix == V.nnx && S.vnr != V.nnx) swrg = 1;
@@ -1451,10 +1451,6 @@ __global__ __launch_bounds__(64) void k_fm2d_near(mct_fm2d_args A, int region_no
                 const int q = BL[k];
                 close_solve(q, close_tlast(q));
             }
-            __syncthreads();
-        } else {
-            for (int q = lane; q < rn; q += 64)
-                if (RN[q] > 0) RN[q] = 1;
             __syncthreads();
         }
         if (A.rays) {
