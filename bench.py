@@ -453,7 +453,8 @@ def run_surface(args):
                    "alg_bytes": int(alg_sweep),
                    "note": "the reference's heap loop for every 2-D problem (the mixed-order times depend on "
                            "its pop order), four problems per wave with their heaps in LDS; algorithmic bytes "
-                           "per solve 4 C + 4 Nr; bound by the pops' dependent latency and VALU issue, not HBM"}
+                           "per solve 4 C + 4 Nr; the pops' stencil loads miss L2 two times in three, so "
+                           "the traffic is far above those bytes (4.5 TB/s)"}
     elif t_sweep > 0:
         a_sweep = alg_sweep / (t_sweep * 1e-3) / 1e9
         r_sweep = {"bound": "hbm", "achieved": round(a_sweep, 3), "peak": HBM_PEAK_GBS, "unit": "GB/s",
@@ -463,8 +464,8 @@ def run_surface(args):
                    "note": "Gauss-Seidel sweeps of the coarse grid, one wave per (chain, period, source); "
                            "algorithmic bytes per solve 4 C + 4 Nr (the survey's 2-D definition without the "
                            "refined nodes, which the near-source kernel handles); the traffic counts every "
-                           "sweep's re-read of the grid (the times and velocities are FP64 here); bound in "
-                           "practice by FP64 VALU issue and latency, not HBM"}
+                           "sweep's re-read of the grid (the times and velocities are FP64 here), which "
+                           "together with FP64 issue bounds it"}
     roof, other = r_disp, r_sweep
     if r_sweep and t_sweep > st_b[1]:
         roof, other = r_sweep, r_disp
@@ -756,7 +757,8 @@ def run_body(args):
     else:
         launches = max(1, tb["round_launches"])
         avg_ms = tb["round_kernels_ms"] / launches
-        kname = "k_eik_round<%d,double,%s>" % (args.order, "double" if f64 else "float")
+        ct = "double" if f64 else "float"
+        kname = "k_eik_round1<double,%s>" % ct if args.order == 1 else "k_eik_round0<1,double,%s>" % ct
     achieved = alg / launches / (avg_ms * 1e-3) / 1e9
     roof = {"bound": "hbm", "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBS, 6), "traffic": None, "kernel": kname,

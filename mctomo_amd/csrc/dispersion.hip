@@ -808,9 +808,11 @@ __global__ __launch_bounds__(64, 2) void k_dispersion_lane(mct_dsp_args A, float
 // 101x101 group-velocity grid: 17.5 -> 1.4 ms.
 //
 // Many columns are bound by the FP64 instructions, which 3 waves per SIMD issue at
-// 79 % of the time and 2 at 70 %: hence the search's state in LDS, one kernel per
+// 76 % of the time and 2 at 70 %: hence the search's state in LDS, one kernel per
 // wave type, and the shorter quotients and sines.  1.4 million different columns of
-// 48 chains, Rayleigh: 91 -> 78 ms; 410,000 columns, Love group: 40 -> 34.7 ms.
+// 48 chains, Rayleigh: 91 -> 76 ms; 410,000 columns, Love group: 40 -> 35.5 ms.  (The
+// Neville tables and up to 24 registers lie in private memory, 27 GB of writes per 1.8
+// million columns.)
 enum {
     SM_NEXT, SM_PERIOD, SM_G0, SM_G1, SM_N0, SM_NLOOP, SM_N1, SM_NBODY, SM_N2, SM_N3,
     SM_NDONE, SM_GDONE, SM_FINISH, SM_DONE

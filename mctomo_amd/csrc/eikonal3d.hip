@@ -319,10 +319,12 @@ __device__ __forceinline__ uint32_t wave_min_u(uint32_t v)
 // passed its key, so the front is swept roughly in arrival order (a tile sees
 // its upwind halo nearly final); tiles not yet due are carried to the next round.
 //
-// What bounds it: FP64 issue.  A visit relaxes its 64 nodes about six times,
-// whatever few of them change, so the update is what counts: ISO (one spacing)
-// needs no sort, no division and two short square roots (60 instructions instead
-// of 150).  A neighbour tile is activated only by a face node whose new time lies
+// What bounds it: many chains move 4.25 TB/s of tiles and halos past L2 (a large copy:
+// 4.9; 42 % L2 hits) with the VALUs 49 % busy, so a visit saved counts on both
+// sides; one chain (34 % busy, 1.4 TB/s, 9.5 waves per CU) waits, in the rounds with
+// many tiles.  A visit relaxes its 64 nodes about six times, whatever few of them
+// change: ISO (one spacing) needs no sort, no division and two short square roots
+// (60 instructions instead of 150).  A neighbour tile is activated only by a face node whose new time lies
 // below the neighbour's node across the face: any other cannot lower it.  The
 // halo may be older than the neighbour's times, never lower, so no activation is
 // missed.  That drops the 42% of the visits that changed nothing, most of them to

@@ -1682,7 +1682,7 @@ __global__ __launch_bounds__(256) void k_fm2d_sweep(mct_fm2d_args A, int32_t *pf
 // A strip without dirty nodes is skipped.
 // With many grids in flight the sweep is bound by memory, not by its arithmetic:
 // 4 doubles of a column at a time fetch each 128-byte line four times over, and
-// the lines do not stay in the L2 between.  48 chains of 201x201 grids (1440
+// the lines do not stay in the L2 between.  48 chains of 201x201 grids (30,720
 // problems, order 0): one 8-byte load a step 128 ms, 4 nodes in two 16-byte loads
 // 83 ms, 8 nodes 71 ms, 12 nodes 81 ms and 16 nodes 79 ms (registers).
 // The mixed-order update holds twice the stencil: 8 nodes left it one wave per SIMD (279
@@ -1723,7 +1723,7 @@ __global__ __launch_bounds__(64, FOM == 0 ? 3 : 2) void k_fm2d_strip(mct_fm2d_ar
     const double dnx = A.dvx / A.gdx, dnz = A.dvz / A.gdz;
     const long cp = g.prob / A.nsrc;
     const double *velnc = A.veln + cp * (long)nnx * nnz;
-    const double *slnc = A.sln ? A.sln + cp * (long)nnx * nnz : nullptr;
+    const double *slnc = A.sln + cp * (long)nnx * nnz;
     double *T = A.ttn + slot * wsz;
     const int32_t *F = A.nsts + slot * wsz;
     const int nn = nnx * nnz;               // the bitmaps fit LDS, so node indices fit 32 bits

@@ -207,8 +207,9 @@ struct mct_fm2d_args {
     int nchain, np, nsrc, nrc;
     const double *velv;         // (nchain*np, (nvx+2)*(nvz+2)) padded control grids, Fortran (nvz+2,nvx+2)
     double *veln;               // (nchain*np, nnx*nnz) coarse velocity, Fortran (nnz,nnx)
-    double *sln;                // the same layout: 1.0 / veln (the sweeps' slowness), or NULL; MCT_FM2D_PAD
-                                // doubles before and after may be read
+    double *sln;                // the same layout: 1.0 / veln, for the sweeps and the wave-wide heap loop
+                                // (mct_launch_fm2d_fast; the lane solver alone does without: NULL);
+                                // MCT_FM2D_PAD doubles before and after may be read
     const double *scx, *scz, *rcx, *rcz;
     const int32_t *srs;         // per period srs_pstride entries; the first nsrc*nrc mark the pairs used (receiver fastest)
     long srs_pstride;

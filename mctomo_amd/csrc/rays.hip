@@ -59,8 +59,8 @@ struct ray_sum {
 __global__ __launch_bounds__(64) void k_fm2d_rays(mct_fm2d_args A)
 {
     // neighbouring blocks (one period's sources, which read the same group
-    // velocities) go to one XCD's L2: bound by gathers (2.9 TB/s, 45 % L2 hits with
-    // blocks in order), 3.9 million rays of 101x101 grids 27.3 -> 23.7 ms
+    // velocities) go to one XCD's L2: bound by gathers (5.8 TB/s past L2), 45 -> 60 %
+    // L2 hits, 3.9 million rays of 101x101 grids 27.3 -> 23.7 ms
     const long nb = gridDim.x, bx = blockIdx.x;
     const long blk = (bx % 8) * (nb / 8) + (bx % 8 < nb % 8 ? bx % 8 : nb % 8) + bx / 8;
     const long t = blk * blockDim.x + threadIdx.x;
