@@ -138,8 +138,9 @@ int mct_noalloc_scratch_bytes(int64_t *bytes);
 int mct_fm2d_last_handover(long long *n);
 
 /* Problems of the calling thread's last order-1 3-D solve (fastMarching3D or a
- * body call) that the replay in LDS left to the one in global memory: their band outgrew
- * its tables, or a corner of the source's cell has no finite time.  No counterpart in the reference: a measurement. */
+ * body call) that the replay in LDS left to the one in global memory: a band outgrew its
+ * tables, or was expected to (then all of the call's), or a corner of the source's cell
+ * has no finite time.  No counterpart in the reference: a measurement. */
 int mct_sfmm_last_handover(long long *n);
 
 /* ---- (c) 3-D eikonal: link-level drop-in ---------------------------------- */

@@ -335,8 +335,8 @@ def modrays_last_handover():
 
 def sfmm_last_handover():
     """Problems of the calling thread's last order-1 3-D solve that the replay in LDS
-    left to the one in global memory (a band that outgrew its tables, a source
-    whose cell has a corner without a finite time)."""
+    left to the one in global memory (a band that outgrew its tables, or was
+    expected to, a source whose cell has a corner without a finite time)."""
     n = ctypes.c_longlong()
     _check(lib().mct_sfmm_last_handover(ctypes.byref(n)), "mct_sfmm_last_handover")
     return n.value

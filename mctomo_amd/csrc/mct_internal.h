@@ -126,8 +126,9 @@ int mct_default_f64();
 // Exact replay of the reference's SFMM heap loop (fmm/fmm.hpp:92-158), one
 // wave per problem, FP64 times and velocities.  T must hold +inf everywhere
 // before the launch (mct_launch_eik_init clears it); the kernel writes the
-// source cells itself.  heap: (nprob, hcap) scratch; err: one word of error
-// bits (read back with mct_sfmm_status); pops: (nprob) pop counts or NULL.
+// source cells itself.  heap: (nprob, hcap) scratch; err: three words, error
+// bits, problems handed over (both read back with mct_sfmm_status) and the widest band
+// expected; pops: (nprob) pop counts or NULL.
 struct mct_sfmm_args {
     mct_geom G;
     int nprob, nsrc_eff, nwave, order;

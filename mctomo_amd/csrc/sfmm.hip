@@ -228,12 +228,11 @@ __device__ __forceinline__ double sf_solve2(const sf_stencil &S, const double le
     return sf_inf();
 }
 
+// the replay of one problem by a wave, its heap in global memory
 template <int HIGH>
-__global__ __launch_bounds__(64) void k_sfmm(mct_sfmm_args A)
+__device__ __forceinline__ void sf_replay(const mct_sfmm_args &A, int prob)
 {
     const int lane = threadIdx.x;
-    const int prob = blockIdx.x;
-    if (A.done && A.done[prob]) return;              // solved with its heap in LDS
     const mct_geom G = A.G;
     const long tsz = (long)G.ntiles * MCT_TILE_N;
     const int si = prob % A.nsrc_eff, cw = prob / A.nsrc_eff, ch = cw / A.nwave;
@@ -482,6 +481,13 @@ __global__ __launch_bounds__(64) void k_sfmm(mct_sfmm_args A)
     if (err && lane == 0) atomicOr(A.err, err);
 }
 
+template <int HIGH>
+__global__ __launch_bounds__(64) void k_sfmm(mct_sfmm_args A)
+{
+    if (A.done && A.done[blockIdx.x]) return;        // solved by k_sfmm_lds
+    sf_replay<HIGH>(A, blockIdx.x);
+}
+
 // ---- the replay with the heap in LDS ----------------------------------------------
 // The same loop for grids whose narrow band fits a compute unit's LDS.  A band cell
 // gets a slot; a heap entry is a slot (16 bits), and a table of the slots' live
@@ -563,7 +569,37 @@ __global__ __launch_bounds__(256) void k_sfl_tiles(mct_geom G, sfl_grid L, const
     if (i >= L.n || !sfl_cell(G, L, i, x, y, z)) return;
     const long q = sf_index(G, x, y, z);
     for (long p = blockIdx.y; p < nprob; p += gridDim.y)
-        if (done[p]) T[p * (long)G.ntiles * MCT_TILE_N + q] = fabs(TL[p * (long)L.n + i]);
+        if (done[p] == 1u) T[p * (long)G.ntiles * MCT_TILE_N + q] = fabs(TL[p * (long)L.n + i]);
+}
+
+// Band cells of a homogeneous medium with the source in cell p when the front has
+// radius r / 24 of the way to the farthest corner: per axis, the grid lines that cross
+// the front where that axis has the largest share of its normal.  h: spacings (their
+// ratios count); the lines are dealt to `lanes` lanes.
+#define SFL_RADII 24
+__host__ __device__ static int sfl_front(const int n[3], const float h[3], const int p[3], int r, int lane, int lanes)
+{
+    float far2 = 0.f;
+    for (int d = 0; d < 3; d++) {
+        const float x = (p[d] > n[d] - 1 - p[d] ? p[d] : n[d] - 1 - p[d]) * h[d];
+        far2 += x * x;
+    }
+    const float t2 = far2 * (float)(r * r) / (float)(SFL_RADII * SFL_RADII);
+    int c = 0;
+#pragma unroll
+    for (int x = 0; x < 3; x++) {
+        const int a = x == 0 ? 1 : 0, b = x == 2 ? 1 : 2;
+        for (int j = 0; j < n[b]; j++) {
+            const float xb = (j - p[b]) * h[b];
+            for (int i = lane; i < n[a]; i += lanes) {
+                const float xa = (i - p[a]) * h[a], w2 = t2 - xa * xa - xb * xb;
+                const float w = sqrtf(w2 > 0.f ? w2 : 0.f), off = w / h[x];
+                const bool on = w2 > 0.f && w * h[x] >= fabsf(xa) * h[a] && w * h[x] >= fabsf(xb) * h[b];
+                c += on ? (p[x] + off <= n[x] - 1) + (p[x] - off >= 0.f) : 0;
+            }
+        }
+    }
+    return c;
 }
 
 struct sfl_args {
@@ -572,8 +608,10 @@ struct sfl_args {
     double *T;                // (nprob, L.n) padded times
     const double *V;          // (chains * waves, L.n) padded velocities
     uint16_t *slot;           // (nprob, L.n) a narrow cell's slot
-    uint32_t *done;           // (nprob) 1 when solved here
+    uint32_t *done;           // (nprob) 1 when solved with the heap in LDS, 2 in global memory
     int ns, ne;               // slots and heap entries in LDS
+    int most;                 // where a wider band is expected (err[2]) all problems are left at once
+    int here;                 // problems left later go on in this kernel (all of its problems run at once)
 };
 
 // lane i of the quad to all four of its lanes
@@ -653,6 +691,31 @@ __device__ __forceinline__ double sfl_solve(int i, double m1, double m2, double 
     return t0 < sf_inf() ? best : tself;
 }
 
+// The widest band that is expected of the problems (sfl_front) to err[2].
+__global__ __launch_bounds__(64) void k_sfl_band(sfl_args S)
+{
+    const mct_sfmm_args &A = S.A;
+    const int lane = threadIdx.x, prob = blockIdx.x;
+    const int si = prob % A.nsrc_eff, ch = prob / A.nsrc_eff / A.nwave;
+    const double *s0 = A.src + (long)ch * A.src_chain_stride + (long)si * A.src_stride;
+    const double p[3] = {s0[0] - A.xmin, s0[1] - A.ymin, s0[2] - A.zmin}, leaf[3] = {A.lx, A.ly, A.lz};
+    const int dims[3] = {A.G.nx, A.G.ny, A.G.nz};
+    const float h[3] = {1.f, (float)(leaf[1] / leaf[0]), (float)(leaf[2] / leaf[0])};
+    int pc[3];
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        const double qd = p[d] / leaf[d];
+        pc[d] = !(qd >= 1.0) ? 0 : (qd >= (double)dims[d] ? dims[d] - 1 : (int)qd);
+    }
+    int widest = 0;
+    for (int r = 1; r <= SFL_RADII; r++) {
+        int c = sfl_front(dims, h, pc, r, lane, 64);
+        for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, 64);
+        widest = c > widest ? c : widest;
+    }
+    if (lane == 0) atomicMax(A.err + 2, (uint32_t)widest);
+}
+
 __global__ __launch_bounds__(64) void k_sfmm_lds(sfl_args S)
 {
     extern __shared__ double sfl_lds[];
@@ -660,6 +723,13 @@ __global__ __launch_bounds__(64) void k_sfmm_lds(sfl_args S)
     const mct_geom &G = A.G;
     const int lane = threadIdx.x;
     const int prob = blockIdx.x;
+    if (S.most > 0 && A.err[2] > (uint32_t)S.most) {
+        if (lane == 0) {
+            S.done[prob] = 0u;
+            atomicAdd(A.err + 1, 1u);
+        }
+        return;
+    }
     const int si = prob % A.nsrc_eff, cw = prob / A.nsrc_eff, ch = cw / A.nwave;
     double *T = S.T + (long)prob * S.L.n;
     const double *V = S.V + (long)cw * S.L.n;
@@ -911,10 +981,15 @@ __global__ __launch_bounds__(64) void k_sfmm_lds(sfl_args S)
             push(slot, tn);
         }
     }
-    // a band that outgrew the tables, or had a key that is no number, is left to k_sfmm
+    // a band that outgrew the tables, or was expected to, or had a key that is no number:
+    // the replay with the heap in global memory, here or by k_sfmm
     if (lane == 0) {
-        S.done[prob] = full ? 0u : 1u;
+        S.done[prob] = !full ? 1u : (S.here ? 2u : 0u);
         if (full) atomicAdd(A.err + 1, 1u);
+    }
+    if (full) {
+        if (S.here) sf_replay<1>(A, prob);
+        return;
     }
     if (A.pops && lane == 0) A.pops[prob] = (uint32_t)(pops > 0xffffffffL ? 0xffffffffL : pops);
     if (err && lane == 0) atomicOr(A.err, err);
@@ -939,11 +1014,11 @@ long mct_sfmm_heap_cap(const mct_geom &G)
 
 // How the replay in LDS would run: slots and heap entries per problem, or 0 slots
 // where it does not pay.
-struct sfl_plan { int ns, ne; size_t lds; };
+struct sfl_plan { int ns, ne, most, here; size_t lds; };
 
 static sfl_plan sfl_make_plan(const mct_geom &G, long nprob)
 {
-    sfl_plan P = {0, 0, 0};
+    sfl_plan P = {0, 0, 0, 0, 0};
     int dev = 0, max_lds = 0, cus = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess ||
@@ -952,9 +1027,10 @@ static sfl_plan sfl_make_plan(const mct_geom &G, long nprob)
     const sfl_grid L = sfl_layout(G);
     // 32-bit byte offsets into a padded grid
     if ((double)(G.nz + 2 * SFL_SLABS) * (G.ny + SFL_PAD + 1) * (G.nx + SFL_PAD + 1) * 8.0 > 2e9) return P;
-    // The band holds 0.4 to 0.8 cells per cell of the grid's three faces (random
-    // Voronoi media, spacings 1:1 to 1:2, sources at the surface and inside), and
-    // about 1.06 entries a cell.  15.3 bytes a slot.
+    // The band holds 0.2 to 0.97 cells per cell of the grid's three faces (1,080 problems:
+    // media of one cell to 1,000 and a gradient, spacings 1:1 to 1:2; sources at a corner
+    // to 0.5, in the middle 0.6 to 0.97), and about 1.06 entries a cell.  15.3 bytes a
+    // slot.
     const double area = (double)G.nx * G.ny + (double)G.ny * G.nz + (double)G.nx * G.nz;
     const double room = (max_lds - 256) / 15.3;
     if (0.55 * area > room) return P;
@@ -965,9 +1041,17 @@ static sfl_plan sfl_make_plan(const mct_geom &G, long nprob)
     // ms for 128 problems, 833 / 1032 for 512, 2488 / 1423 for 1,536; 41^3 (two a
     // unit) 151 / 307 for 128, 313 / 452 for 1,024.
     if (nprob > 2L * per_cu * cus) return P;
+    // In two turns the problems that are left run after the others (33^3, one of 1,300 left
+    // 351 ms, all in global memory 241): only where every band fits.  Run at once, they
+    // go on in place.
+    P.here = nprob <= (long)per_cu * cus;
+    if (!P.here && room / per_cu < area) return P;
+    // no more problems to a unit than it takes to run all at once: wider tables
+    while (per_cu > 1 && nprob <= (long)(per_cu - 1) * cus) per_cu--;
     P.ns = (int)(room / per_cu) & ~7;
     if (P.ns > 65528) P.ns = 65528;
-    // MCT_SFMM_SLOTS: at most this many, so that wider bands are handed over
+    // MCT_SFMM_SLOTS: at most this many, so that wider bands are handed over when they
+    // are that wide
     const char *e = getenv("MCT_SFMM_SLOTS");
     const int most = e ? atoi(e) & ~7 : 0;
     if (most > 0 && P.ns > most) P.ns = most < 64 ? 64 : most;
@@ -978,6 +1062,15 @@ static sfl_plan sfl_make_plan(const mct_geom &G, long nprob)
         P.ne = P.ns + P.ns / 8 + 64;
         P.lds = 12 * (size_t)P.ns + 2 * (size_t)P.ne + (size_t)P.ns;
     }
+    // A band that outgrows the tables has its problem begun twice: a source in the
+    // middle of a 74^3 grid 2.25 s with the tables first, 1.88 at once in global memory,
+    // one at its corner 0.90 in LDS.  Where the tables may be too small, the widest band
+    // of a homogeneous medium tells (the 1,080 problems' was 1.08 times that in the
+    // median, 0.98 to 1.26 for 80 % of them).  Leaving a band that fits costs more than
+    // trying one that does not, so the line lies where about half outgrow the tables.
+    // A launch takes as long as its slowest problem, so one that is left takes the others
+    // along (72^3, 5 of 200 left, some of them late: 2.24 s, all in global memory 1.93).
+    if (!(most > 0) && area > P.ns) P.most = (int)(0.95 * P.ns);
     return P;
 }
 
@@ -995,10 +1088,10 @@ int mct_launch_sfmm(const mct_sfmm_args &a0, hipStream_t s)
         a.nsrc_eff < 1 || a.nwave < 1)
         return MCT_ERR_ARG;
     if ((long)a.G.ntiles * MCT_TILE_N > 0xffffffffL) return MCT_ERR_ARG;
-    MCT_CHECK(hipMemsetAsync(a.err, 0, 2 * sizeof(uint32_t), s));
+    MCT_CHECK(hipMemsetAsync(a.err, 0, 3 * sizeof(uint32_t), s));
     a.done = nullptr;
     const long ncw = (a.nprob + a.nsrc_eff - 1) / a.nsrc_eff;
-    const sfl_plan P = a.order == 1 && a.lin ? sfl_make_plan(a.G, a.nprob) : sfl_plan{0, 0, 0};
+    const sfl_plan P = a.order == 1 && a.lin ? sfl_make_plan(a.G, a.nprob) : sfl_plan{0, 0, 0, 0, 0};
     if (P.ns > 0) {
         sfl_args S;
         S.L = sfl_layout(a.G);
@@ -1008,6 +1101,8 @@ int mct_launch_sfmm(const mct_sfmm_args &a0, hipStream_t s)
         S.slot = (uint16_t *)(S.done + a.nprob);
         S.ns = P.ns;
         S.ne = P.ne;
+        S.most = P.most;
+        S.here = P.here;
         a.done = S.done;
         S.A = a;
         const unsigned gx = (S.L.n + 255) / 256;
@@ -1016,6 +1111,7 @@ int mct_launch_sfmm(const mct_sfmm_args &a0, hipStream_t s)
         hipLaunchKernelGGL(k_sfl_vel, dim3(gx, gc), dim3(256), 0, s, a.G, S.L, a.V, (double *)S.V, ncw);
         if (P.lds > 64 * 1024)
             MCT_CHECK(hipFuncSetAttribute((const void *)k_sfmm_lds, hipFuncAttributeMaxDynamicSharedMemorySize, (int)P.lds));
+        if (P.most > 0) hipLaunchKernelGGL(k_sfl_band, dim3((unsigned)a.nprob), dim3(64), 0, s, S);
         hipLaunchKernelGGL(k_sfmm_lds, dim3((unsigned)a.nprob), dim3(64), P.lds, s, S);
         hipLaunchKernelGGL(k_sfl_tiles, dim3(gx, gy), dim3(256), 0, s, a.G, S.L, S.T, a.T, S.done, (long)a.nprob);
         MCT_CHECK(hipGetLastError());

@@ -239,3 +239,18 @@ def test_source_on_a_node_of_velocity_zero(seed):
     else:
         np.testing.assert_array_equal(fg, fo)
     assert mct.sfmm_last_handover() == 1
+
+
+@pytest.mark.parametrize("n,where,handed", [(33, (0.5, 0.5, 0.5), 0), (70, (0.5, 0.5, 0.5), 1), (70, (0.5, 0.5, 0.0), 0),
+                                            (70, (0.02, 0.02, 0.02), 0)])
+def test_who_solves_a_wide_band(n, where, handed):
+    """A source in the middle of a grid has the widest band: a 33^3 grid's fits when a
+    problem has a unit's LDS to itself, a 70^3 grid's does not (it is left to global
+    memory before the first pop), where those of sources at a face or a corner do.
+    The oracle's fields bit for bit."""
+    vel, ext, rng = _voronoi((n, n, n), (0.2, 0.2, 0.2), 1 if n == 33 else 30, n)
+    src, rev = ext * np.array(where), rng.uniform(0, 1, (3, 3)) * ext
+    say("wide band", n, where)
+    fg = mct.fast_marching_3d(vel, 0.2, 0.2, 0.2, 0, 0, 0, src, rev, 1, field=True)[1]
+    assert mct.sfmm_last_handover() == handed
+    np.testing.assert_array_equal(fg, po.fast_marching_3d(vel, 0.2, 0.2, 0.2, 0, 0, 0, src, rev, 1, field=True)[1])
