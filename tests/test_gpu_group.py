@@ -252,3 +252,32 @@ def test_straight_ray_out_of_area_is_fatal_like_the_oracle():
     assert res[0] < 0
     # the context stays usable for a model within the area
     L.close()
+
+
+@pytest.mark.parametrize("order", [0, 1])
+@pytest.mark.parametrize("sgext,sgdic", [(8, 8), (13, 5)])
+def test_group_rays_through_the_largest_refined_windows(order, sgext, sgdic):
+    """Refined source grids of 129 and 131 nodes a side, the largest that the near-source
+    kernel holds: the rays read its refined grid, and group times and ray lengths are
+    the sequential method's (bit for bit with first-order times) and the oracle's."""
+    w = W.surface_workload(n=41, nz=21, ncells=30, np_=4, nsrc=9, nrev=11, seed=77, order=order)
+    say("group, refined window", 2 * sgext * sgdic + 1, "order", order)
+    got = {}
+    for method in (0, 1):
+        L = ctx_for(w, sgext=sgext, sgdic=sgdic)
+        L.set_method(method)
+        rc, out, pt, sd, _, _ = L.likelihood(w.points, w.params, arrays=True)
+        assert rc == 0
+        got[method] = (out, pt, sd)
+        L.close()
+    orc = po.surf_likelihood(gdict(w.grid), w.points, w.params, w.freqs, w.src, w.rev, w.ttime, w.raystat,
+                             raylov=w.raylov, order=order, phase_group=1, sgext=sgext, sgdic=sgdic,
+                             group_vel=np.zeros((w.grid.nx, w.grid.ny, w.freqs.shape[0])))
+    for k in (1, 2):
+        if order == 0:
+            np.testing.assert_array_equal(got[0][k], got[1][k])
+        else:
+            np.testing.assert_allclose(got[0][k], got[1][k], rtol=1e-9, atol=0)
+    used = w.raystat[:, 0].reshape(orc[2].shape) == 1
+    np.testing.assert_allclose(got[0][1][used], orc[2][used], rtol=1e-4, atol=0)
+    assert abs(got[0][0][0] - orc[1][0]) <= 1e-6 * abs(orc[1][0])
